@@ -1,5 +1,5 @@
-// supernodal.hip -- forward solve on a supernodal (BCSC) lower triangle for
-// gfx950, bit-identical to the reference's blocked solve.
+// supernodal.hip -- solves on a supernodal (BCSC) lower triangle for gfx950,
+// the forward one bit-identical to the reference's blocked solve.
 //
 // Reference: sparse_blas/sptrsv.cpp:176-199 (sptrsv_csc_block) with the dense
 // kernels of sparse_blas/dense_blas/BLAS.cpp: lsolve_BLAS (:3-96) and
@@ -11,27 +11,35 @@
 // nrows_i block rows; its values are a column-major nrows_i x w_i block at
 // Lx[Lp[i]] whose first w_i rows are its own columns and whose row r is row
 // Li[Lp[i] + r] of L.  Per supernode the reference solves the dense top
-// (column blocks of 8, then 4, then 2, then 1; inside a block x_j = (b_j -
-// x_0 m_j0 - ... - x_{j-1} m_j,j-1) / m_jj left to right, then every later
-// top row subtracts the block's products left to right), multiplies the rows
-// below by the solved part (column blocks of 8, then 4, then 1; each block's
-// products summed left to right and added to a zeroed temporary), and
-// subtracts the temporary from x at those rows, supernode after supernode.
+// (every row subtracts its products column by column, left to right, then
+// divides), multiplies the rows below by the solved part (column blocks of 8,
+// then 4, then 1; each block's products summed left to right and added to a
+// zeroed temporary), and subtracts the temporary from x at those rows,
+// supernode after supernode.
 //
-// Executor: one wavefront per task, tasks taken by ticket in order.  A
-// supernode's first task solves its top and multiplies the first SN_CHUNK
-// rows below; each further SN_CHUNK rows below are a task of their own that
-// reads the solved top from memory, so the rows below a wide supernode are
-// multiplied by several waves.  A task only waits for earlier tasks (the
-// producers of its rows' temporaries, or its supernode's top), which running
-// waves already hold.  The subtraction into x is pulled
-// instead of pushed: each supernode writes its temporary to a buffer T and
-// publishes a tag; a supernode starts by waiting for the supernodes that
-// write to its own rows, then forms x at each own row as b minus their
-// temporaries in ascending supernode order -- the order the reference's
-// serial loop subtracts them in -- so x is bit-identical.  The top block is
-// solved in the wave's LDS: lane j of a column block holds row j's entries,
-// x_j is formed on lane j and broadcast; the rows below are one lane each.
+// Executor: one persistent launch of four-wave workgroups that take tickets
+// level by level of the tree.  A ticket is up to four narrow supernodes (at
+// most 64 columns: one wavefront solves the top and multiplies the first
+// SN_NARROW_ROWS rows below), the top of one wide supernode (the workgroup),
+// or 64 rows below a top (the workgroup, its column blocks dealt over the
+// waves).  Every wait is for an earlier ticket, which a running workgroup
+// holds.  The subtraction into x is pulled instead of pushed: each supernode
+// writes its temporaries to T where the rows that subtract them read their
+// lists (ascending supernode order, the order of the reference's serial
+// loop): entry j of the 64 rows of a wave lies side by side, so a load of T
+// is one contiguous run.
+//
+// What bounds it: the chain of tree levels -- for each, the widest top's
+// columns (a division, a broadcast and a multiply-subtract each, about 75 ns)
+// plus the hand-offs -- for one right-hand side and the last levels of a
+// block.  A top's rows lie one per lane, 64 to a wave, and each wave streams
+// its rows' entries with SN_AHEAD column blocks in flight; the wave whose
+// rows are next solves its 64 columns with lane broadcasts and hands x on
+// through LDS, block of 8 by block of 8, while the other waves subtract.
+// Measured on the 13-level nested-dissection-shaped factor (8,191 supernodes
+// up to 512 wide, 36 M values), forward and transposed: one right-hand side
+// 4.35 ms with one wavefront per top -> 1.07 ms, 32 right-hand sides 11.6 ->
+// 3.22 ms.
 #include <algorithm>
 #include <vector>
 
@@ -41,142 +49,27 @@ namespace symamd {
 
 namespace {
 
+constexpr int SN_AHEAD = 4;  // column blocks of 8 whose entries are in flight
+
 struct SnArgs {
   const int *sup, *nrows, *Lp;  // the reference's supernode arrays
   const double *Lx;
   double *x;                    // right-hand side in, solution out
-  double *T;                    // temporaries: supernode i's at T[tb[i] ..]
-  const int *tb;                // nrows_i - w_i values each
-  const int *cptr, *cidx;       // row r subtracts T[cidx[cptr[r] .. cptr[r+1])]
-  const int2 *task;             // task t: (supernode, chunk of its rows below)
-  const int *dptr, *dlist;      // tasks that task t waits for
-  int *flags, *state;           // one tag per (column, task)
-  int ntasks, total_waves;
-  // transposed solve: rows below each supernode (at its temporaries'
-  // offsets tb), and the supernodes owning them that it waits for
-  const int *rowb, *tdptr, *tdlist;
-  const int *torder;            // supernode of each transposed ticket
-  int m;
-  int k;                        // right-hand sides: column c at x + c*ldx
-  int64_t ldx, tstride;         // its temporaries at T + c*tstride
+  double *T;                    // temporaries, placed where the rows' lists are read
+  const int *tb;                // supernode i's rows below start at tb[i]
+  const int *tdst;              // place in T of each row below
+  const int4 *list;             // row r subtracts T[x + j*z], j < y
+  const int2 *unit;             // unit u: (supernode, 0 = top or c = chunk c - 1 below)
+  const int *tick;              // ticket t runs units tick[t] .. tick[t+1]
+  const int *dptr, *dlist;      // units that unit u waits for
+  int *flags, *state;           // one tag per (column tile, unit)
+  int nunits, ntick, total_waves;
+  const int *rowb;              // transposed: rows below (at tb)
+  const int *tbelow;            // transposed: first column-group unit of a supernode, or -1
+  int k, tiles;                 // right-hand sides: column c at x + c*ldx; tiles of KT
+  int64_t ldx, tcount;          // column c's temporaries at T + c*tcount
   uint64_t timeout;
 };
-
-// Column block at `col` of a top of width w: 8 while 8 fit with one to
-// spare (matvec) or without (lsolve), else 4, else 2 (lsolve) or 1.
-__device__ __forceinline__ int lsolve_block(int col, int w) {
-  return col < w - 7 ? 8 : col < w - 3 ? 4 : col < w - 1 ? 2 : 1;
-}
-__device__ __forceinline__ int matvec_block(int col, int w) {
-  return col < w - 7 ? 8 : col < w - 3 ? 4 : 1;
-}
-
-// Rows per lane processed together in the top's updates and the product
-// below (their loads in flight at once).
-constexpr int SN_ROWS = 2;
-static_assert(SN_CHUNK == 64 * SN_ROWS, "a chunk of rows below is one pass of a wave");
-// TOP_ROWS: rows per lane per pass of the top's update after each column
-// block.  Each pass is a memory round trip on the chain from one block to
-// the next; four rows per pass take more registers (two waves per SIMD
-// instead of three), which pays for one right-hand side, where the chain of
-// the widest supernodes sets the time, and not for blocks, where the (task,
-// column) tickets keep every wave busy.
-
-// A supernode's own rows: xs[r] = x[s+r] minus the temporaries listed for
-// row s+r, in list (ascending supernode) order, for rows r0 <= r < w.  Lane l
-// takes rows r0 + l + 64q, q < NQ, and its rows advance together, GB = 16/NQ
-// list entries each per round (32 slots per lane measured slower: most of the
-// extra slots are stand-ins): a round's temporaries are loaded for all of its
-// rows at once (their indices were loaded in the round before), then
-// subtracted row by row in list order.  So a lane pays one memory round
-// trip per GB entries of its longest row, not per eight entries of each row
-// in turn.  No load is behind a branch: list positions past a row's end are
-// clamped into the index array (which holds at least one entry), and their
-// temporaries are replaced by the row's own x (rows past w by row w-1's),
-// loaded and not used; whether a slot is used depends only on the list
-// bounds, so no value is waited for before its use.
-template <int NQ>
-__device__ __forceinline__ void gather_rows(double *xs, const double *x, const double *T,
-                                            const int *cptr, const int *cidx, int s, int w,
-                                            int r0, int lane) {
-  static_assert(NQ >= 1 && NQ <= 8, "at most 512 rows per call");
-  constexpr int GB = 16 / NQ;
-  if (w <= r0) return;
-  double v[NQ];
-  int cp[NQ], ce[NQ], idx[NQ][GB];
-  auto row = [&](int q) { return min(r0 + lane + 64 * q, w - 1); };
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const bool in = r0 + lane + 64 * q < w;
-    v[q] = x[s + row(q)];
-    const int c0 = cptr[s + row(q)], c1 = cptr[s + row(q) + 1];
-    cp[q] = in ? c0 : 0;
-    ce[q] = in ? c1 : 0;
-  }
-  auto load_idx = [&](int q, int c, int (&d)[GB]) {
-#pragma unroll
-    for (int u = 0; u < GB; ++u) d[u] = cidx[max(min(c + u, ce[q] - 1), 0)];
-  };
-  bool more = false;
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    load_idx(q, cp[q], idx[q]);
-    more = more || cp[q] < ce[q];
-  }
-  while (more) {
-    double tv[NQ][GB];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int u = 0; u < GB; ++u)
-        tv[q][u] = ld_dev(cp[q] + u < ce[q] ? &T[idx[q][u]] : &x[s + row(q)]);
-    int nidx[NQ][GB];
-    more = false;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      load_idx(q, cp[q] + GB, nidx[q]);
-      more = more || cp[q] + GB < ce[q];
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-#pragma unroll
-      for (int u = 0; u < GB; ++u)
-        if (cp[q] + u < ce[q]) v[q] -= tv[q][u];
-      cp[q] += GB;
-#pragma unroll
-      for (int u = 0; u < GB; ++u) idx[q][u] = nidx[q][u];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < NQ; ++q)
-    if (r0 + lane + 64 * q < w) xs[r0 + lane + 64 * q] = v[q];
-}
-
-// NB full column blocks of eight from col: each block's products with the
-// solved top summed left to right and added to the row's temporary, for the
-// SN_ROWS rows k0 + 64u (rows past nr read row nr-1; their sums are unused)
-template <int NB>
-__device__ __forceinline__ void product_blocks(double (&t)[SN_ROWS], const double *xs,
-                                               const double *M, int k0, int nr, int col) {
-  double mb[NB][SN_ROWS][8];
-#pragma unroll
-  for (int h = 0; h < NB; ++h)
-#pragma unroll
-    for (int u = 0; u < SN_ROWS; ++u) {
-      const int k = k0 + 64 * u;
-#pragma unroll
-      for (int c = 0; c < 8; ++c) mb[h][u][c] = M[min(k, nr - 1) + (int64_t)(col + 8 * h + c) * nr];
-    }
-#pragma unroll
-  for (int h = 0; h < NB; ++h)
-#pragma unroll
-    for (int u = 0; u < SN_ROWS; ++u) {
-      double sum = xs[col + 8 * h] * mb[h][u][0];
-#pragma unroll
-      for (int c = 1; c < 8; ++c) sum = sum + xs[col + 8 * h + c] * mb[h][u][c];
-      t[u] = t[u] + sum;
-    }
-}
 
 // v on lane j (j uniform), for every lane
 __device__ __forceinline__ double lane_value(double v, int j) {
@@ -186,333 +79,835 @@ __device__ __forceinline__ double lane_value(double v, int j) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-template <int TOP_ROWS>
-__global__ __launch_bounds__(256, TOP_ROWS >= 4 ? 2 : 3) void k_supernodal(SnArgs a) {
-  __shared__ double slab[4][SN_WMAX];
-  double *xs = slab[threadIdx.x >> 6];
+// The right-hand side columns of one tile; columns past k repeat the last
+// one (solved again, not stored).
+template <int KT>
+struct Cols {
+  double *x[KT];
+  bool live[KT];
+  __device__ __forceinline__ Cols(const SnArgs &a, int tile) {
+#pragma unroll
+    for (int c = 0; c < KT; ++c) {
+      const int col = tile * KT + c;
+      live[c] = col < a.k;
+      x[c] = a.x + (int64_t)min(col, a.k - 1) * a.ldx;
+    }
+  }
+};
+
+// The values are computed here: without it the compiler moves a block's
+// subtractions past the wait for the next block, and keeps their operands in
+// registers (and then in scratch memory) until there.
+template <int KT>
+__device__ __forceinline__ void hold(double (&v)[KT]) {
+#pragma unroll
+  for (int c = 0; c < KT; ++c) asm volatile("" : "+v"(v[c]));
+}
+
+// Columns solved so far of the workgroup's top, kept in LDS: the wave that
+// solved a block of eight stores their x, then the count; LDS operations of a
+// wave complete in order, so a wave that reads the count reads those x.
+__device__ __forceinline__ void lds_publish(int *prog, int v, int lane) {
+  asm volatile("" ::: "memory");
+  if (lane == 0) __hip_atomic_store(prog, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// Waits until the count reaches `need`; the waves solve their rows in
+// ascending count order and wait for nothing else, so it always does.
+__device__ __forceinline__ void lds_wait(const int *prog, int need, int &seen) {
+  while (seen < need)
+    seen = __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(prog, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+  asm volatile("" ::: "memory");
+}
+
+// Waits for one tag (every lane reads it); bounded by the watchdog as
+// wait_list is.
+__device__ __forceinline__ void wait_flag(const int *f, int target, int *state,
+                                          uint64_t timeout) {
+  if (ld_dev(f) == target) return;
+  const uint64_t t0 = wall_ticks();
+  for (int rounds = 1; ld_dev(f) != target; ++rounds) {
+    __builtin_amdgcn_s_sleep(1);
+    if ((rounds & 63) == 0 && wall_ticks() - t0 > timeout) {
+      if ((threadIdx.x & 63) == 0) atomicOr(&state[ST_ERROR], 1);
+      break;
+    }
+  }
+  asm volatile("" ::: "memory");
+}
+
+// One lane per row: v minus the row's temporaries, in list order, GB entries
+// per round with the next round's loads in flight.  Entries past the row's
+// list are its last one (or T's first), not used.
+template <int KT>
+__device__ __forceinline__ void gather_list(double (&v)[KT], const double *T, int64_t tcount,
+                                            const int4 &l) {
+  constexpr int GB = 16 / KT;
+  double ta[GB][KT], tb[GB][KT];
+  auto load = [&](double (&t)[GB][KT], int j) {
+#pragma unroll
+    for (int u = 0; u < GB; ++u) {
+      const double *p = T + (l.x + (int64_t)max(min(j + u, l.y - 1), 0) * l.z);
+#pragma unroll
+      for (int q = 0; q < KT; ++q) t[u][q] = ld_dev(p + q * tcount);
+    }
+  };
+  auto subtract = [&](const double (&t)[GB][KT], int j) {
+#pragma unroll
+    for (int u = 0; u < GB; ++u)
+#pragma unroll
+      for (int q = 0; q < KT; ++q) v[q] = j + u < l.y ? v[q] - t[u][q] : v[q];
+  };
+  if (!__any(l.y > 0)) return;
+  load(ta, 0);
+  for (int j = 0;;) {
+    load(tb, j + GB);
+    subtract(ta, j);
+    j += GB;
+    if (!__any(j < l.y)) break;
+    load(ta, j + GB);
+    subtract(tb, j);
+    j += GB;
+    if (!__any(j < l.y)) break;
+  }
+}
+
+// p[i] for a uniform p: a scalar base and a 32-bit lane offset, so a load
+// needs no per-lane 64-bit address.
+__device__ __forceinline__ double at(const double *p, int i) {
+  return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(p) + (unsigned)i * 8u);
+}
+
+// Eight columns from c0 of one row's entries (lane = row), loads clamped to
+// the top's last column.
+__device__ __forceinline__ void load_cols(double (&m)[8], const double *M, int row, int c0,
+                                          int w, int nr) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) m[j] = at(M + (int64_t)min(c0 + j, w - 1) * nr, row);
+}
+
+// A row's diagonal and its correctly rounded reciprocal, for quotients off
+// the IEEE division's long chain: with y = RN(1/d), one Newton step on a * y
+// gives a quotient within one unit in the last place, and a second with its
+// exact remainder the correctly rounded one (Markstein, IBM J. Res. Dev. 34,
+// 1990), as long as no step leaves the normal range.  `usable` says so for
+// the diagonal, in_range() for a dividend; otherwise the division is done.
+struct Diag {
+  double d, y;
+  bool usable;
+  __device__ __forceinline__ explicit Diag(double v) : d(v), y(1.0 / v), usable(in_range(v, 100)) {}
+  // 2^-e <= |v| < 2^e
+  static __device__ __forceinline__ bool in_range(double v, int e) {
+    const unsigned hi = (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) & 0x7fffffffu;
+    return hi - ((unsigned)(1023 - e) << 20) < ((unsigned)(2 * e) << 20);
+  }
+  __device__ __forceinline__ double divide(double a) const {
+    const double q0 = a * y;
+    const double q1 = __builtin_fma(__builtin_fma(-d, q0, a), y, q0);
+    return __builtin_fma(__builtin_fma(-d, q1, a), y, q1);
+  }
+};
+
+// Eight columns of a wave's own diagonal, lanes lb .. lb + B - 1 their rows
+// (B < 8 in the last block only): at step j lane lb + j divides, the quotient
+// is broadcast, and every later row subtracts its product; TRANS takes the
+// columns from the last one.  res keeps a lane's quotient.  Lanes already
+// solved, and lanes past the last column, go on computing values that nothing
+// reads.  entry(j) loads m[j] again, for the block whose quotients need the
+// division.
+template <int KT, bool TRANS, typename Entry>
+__device__ __forceinline__ void solve_block(double (&acc)[KT], double (&res)[KT],
+                                            const double (&m)[8], const Diag &dg, int lb, int B,
+                                            int lane, Entry entry) {
+  double start[KT], num[KT];
+#pragma unroll
+  for (int c = 0; c < KT; ++c) {
+    start[c] = acc[c];
+    num[c] = 1.0;
+  }
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    const int j = TRANS ? 7 - t : t;
+    if (TRANS && j >= B) continue;
+    double q[KT];
+#pragma unroll
+    for (int c = 0; c < KT; ++c) {
+      num[c] = lane == lb + j ? acc[c] : num[c];
+      q[c] = dg.divide(acc[c]);
+      res[c] = lane == lb + j ? q[c] : res[c];
+    }
+#pragma unroll
+    for (int c = 0; c < KT; ++c) acc[c] = acc[c] - lane_value(q[c], lb + j) * m[j];
+  }
+  bool ok = dg.usable;
+#pragma unroll
+  for (int c = 0; c < KT; ++c) ok = ok && Diag::in_range(num[c], 900);
+  if (__any(lane >= lb && lane < lb + min(B, 8) && !ok)) {
+#pragma unroll
+    for (int c = 0; c < KT; ++c) acc[c] = start[c];
+#pragma unroll 1
+    for (int t = 0; t < min(B, 8); ++t) {
+      const int j = TRANS ? min(B, 8) - 1 - t : t;
+      const double mj = entry(j);
+#pragma unroll
+      for (int c = 0; c < KT; ++c) {
+        const double q = acc[c] / dg.d;
+        res[c] = lane == lb + j ? q : res[c];
+        acc[c] = acc[c] - lane_value(q, lb + j) * mj;
+      }
+    }
+  }
+}
+
+// A wave's own n <= 64 columns from column c0, the first SN_AHEAD blocks in
+// buf; done(lb, B) after each block.  Rounds of SN_AHEAD full blocks take no
+// branch, so the waits for their loads stay exact.
+template <int KT, typename Done>
+__device__ __forceinline__ void own_columns(double (&acc)[KT], double (&res)[KT],
+                                            double (&buf)[SN_AHEAD][8], const Diag &dg, int c0,
+                                            int n, const double *M, int row, int w, int nr,
+                                            int lane, Done done) {
+  auto block = [&](int b, const double (&m)[8]) {
+    const int B = min(8, n - 8 * b);
+    solve_block<KT, false>(acc, res, m, dg, 8 * b, B, lane, [&](int j) {
+      return at(M + (int64_t)(c0 + 8 * b + j) * nr, row);
+    });
+    done(8 * b, B);
+  };
+  int b = 0;
+  for (; 8 * (b + SN_AHEAD) <= n; b += SN_AHEAD) {
+#pragma unroll
+    for (int q = 0; q < SN_AHEAD; ++q) {
+      block(b + q, buf[q]);
+      load_cols(buf[q], M, row, c0 + 8 * (b + q + SN_AHEAD), w, nr);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < SN_AHEAD; ++q)
+    if (8 * (b + q) < n) block(b + q, buf[q]);
+}
+
+// Rows 64g .. 64g+63 of a wide top, by one wave.  `buf` holds the first
+// SN_AHEAD column blocks of the wave's rows.
+template <int KT>
+__device__ __forceinline__ void top_group(const SnArgs &a, const Cols<KT> &col, const double *T,
+                                          double (&buf)[SN_AHEAD][8], const Diag &dg, int g,
+                                          int s, int w, int nr, const double *M, double *xs,
+                                          int *prog, int &seen, int lane) {
+  const int row = min(64 * g + lane, w - 1);
+  double acc[KT], res[KT];
+#pragma unroll
+  for (int c = 0; c < KT; ++c) {
+    acc[c] = col.x[c][s + row];
+    res[c] = 0.0;
+  }
+  gather_list<KT>(acc, T, a.tcount, a.list[s + row]);
+  // columns of earlier groups: x from LDS as it is solved
+  for (int b0 = 0; b0 < 8 * g; b0 += SN_AHEAD) {
+#pragma unroll
+    for (int q = 0; q < SN_AHEAD; ++q) {
+      const int c0 = 8 * (b0 + q);
+      lds_wait(prog, c0 + 8, seen);
+      double xv[8][KT];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int c = 0; c < KT; ++c) xv[j][c] = xs[(c0 + j) * KT + c];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+#pragma unroll
+        for (int c = 0; c < KT; ++c) acc[c] = acc[c] - xv[j][c] * buf[q][j];
+      }
+      hold<KT>(acc);
+      load_cols(buf[q], M, row, c0 + 8 * SN_AHEAD, w, nr);
+    }
+  }
+  // the group's own columns
+  own_columns<KT>(acc, res, buf, dg, 64 * g, min(64, w - 64 * g), M, row, w, nr, lane,
+                  [&](int lb, int B) {
+                    if (lane >= lb && lane < lb + B) {
+#pragma unroll
+                      for (int c = 0; c < KT; ++c) xs[(64 * g + lane) * KT + c] = res[c];
+                    }
+                    lds_publish(prog, 64 * g + lb + B, lane);
+                  });
+#pragma unroll
+  for (int c = 0; c < KT; ++c)
+    if (64 * g + lane < w && col.live[c]) st_dev(&col.x[c][s + row], res[c]);
+}
+
+// A narrow supernode (w <= SN_NARROW) by one wave: the top, then the first
+// SN_NARROW_ROWS rows below, two per lane; xs is the wave's LDS.
+template <int KT>
+__device__ __forceinline__ void narrow_unit(const SnArgs &a, const Cols<KT> &col, double *T,
+                                            int u, int tile, int i, int target, double *xs,
+                                            int lane) {
+  const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i];
+  const double *M = a.Lx + a.Lp[i];
+  const int row = min(lane, w - 1);
+  double buf[SN_AHEAD][8];
+#pragma unroll
+  for (int q = 0; q < SN_AHEAD; ++q) load_cols(buf[q], M, row, 8 * q, w, nr);
+  const Diag dg(M[row + (int64_t)row * nr]);
+  double acc[KT], res[KT];
+#pragma unroll
+  for (int c = 0; c < KT; ++c) {
+    acc[c] = col.x[c][s + row];
+    res[c] = 0.0;
+  }
+  const int4 list = a.list[s + row];
+  int *const flags = a.flags + (int64_t)tile * a.nunits;
+  wait_units(a.dptr, a.dlist, u, flags, target, a.state, a.timeout);
+  gather_list<KT>(acc, T, a.tcount, list);
+  own_columns<KT>(acc, res, buf, dg, 0, w, M, row, w, nr, lane, [](int, int) {});
+  if (lane < w) {
+#pragma unroll
+    for (int c = 0; c < KT; ++c) {
+      xs[lane * KT + c] = res[c];
+      if (col.live[c]) st_dev(&col.x[c][s + lane], res[c]);
+    }
+  }
+  wave_lds_sync();
+  const int below = min(nr - w, SN_NARROW_ROWS);
+  for (int r0 = 0; r0 < below; r0 += 64) {
+    const int k = w + min(r0 + lane, below - 1);
+    double t[KT];
+#pragma unroll
+    for (int c = 0; c < KT; ++c) t[c] = 0.0;
+    int cb = 0;
+    // two blocks' entries in flight, one where their x fill the registers
+    constexpr int NB = KT < 4 ? 2 : 1;
+    for (; w - cb >= 8 * NB; cb += 8 * NB) {
+      double m[NB][8];
+#pragma unroll
+      for (int h = 0; h < NB; ++h) load_cols(m[h], M, k, cb + 8 * h, w, nr);
+#pragma unroll
+      for (int h = 0; h < NB; ++h)
+#pragma unroll
+        for (int c = 0; c < KT; ++c) {
+          double sum = xs[(cb + 8 * h) * KT + c] * m[h][0];
+#pragma unroll
+          for (int j = 1; j < 8; ++j) sum = sum + xs[(cb + 8 * h + j) * KT + c] * m[h][j];
+          t[c] = t[c] + sum;
+        }
+    }
+    for (int B; cb < w; cb += B) {
+      B = w - cb >= 8 ? 8 : w - cb >= 4 ? 4 : 1;
+      double m[8];
+      load_cols(m, M, k, cb, w, nr);
+#pragma unroll
+      for (int c = 0; c < KT; ++c) {
+        double sum = xs[cb * KT + c] * m[0];
+#pragma unroll
+        for (int j = 1; j < 8; ++j)
+          if (j < B) sum = sum + xs[(cb + j) * KT + c] * m[j];
+        t[c] = t[c] + sum;
+      }
+    }
+    if (r0 + lane < below) {
+      const int64_t p = a.tdst[a.tb[i] + r0 + lane];
+#pragma unroll
+      for (int c = 0; c < KT; ++c) st_dev(&T[p + c * a.tcount], t[c]);
+    }
+  }
+  publish_fence();
+  if (lane == 0) st_dev(&flags[u], target);
+  wave_lds_sync();
+}
+
+// 64 rows below a top by the workgroup: the column blocks of eight are dealt
+// over the waves, NBW consecutive blocks each per pass; the block sums go to
+// LDS and wave c adds column c's in block order.  The entries are loaded
+// before the wait for the top.
+template <int KT>
+__device__ __forceinline__ void below_unit(const SnArgs &a, const Cols<KT> &col, double *T,
+                                           int u, int tile, int i, int first, int target,
+                                           double *xs, double *sums) {
+  constexpr int NBW = 8 / KT;
   const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i];
+  const double *M = a.Lx + a.Lp[i];
+  const int k = min(w + first + lane, nr - 1);
+  int *const flags = a.flags + (int64_t)tile * a.nunits;
+  const int nb = w / 8;  // full blocks; then one of 4 where 4 are left, then single columns
+  double m[NBW][8], tail[8];
+#pragma unroll
+  for (int h = 0; h < NBW; ++h) load_cols(m[h], M, k, 8 * (wave * NBW + h), w, nr);
+  load_cols(tail, M, k, 8 * nb, w, nr);
+  const int64_t place = a.tdst[a.tb[i] + k - w];
+  if (wave == 0) wait_units(a.dptr, a.dlist, u, flags, target, a.state, a.timeout);
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < KT; ++c)
+    for (int r = threadIdx.x; r < w; r += 256) xs[r * KT + c] = ld_dev(&col.x[c][s + r]);
+  __syncthreads();
+  double t = 0.0;  // waves 0 .. KT-1: this row's temporary of column `wave`
+  int half = 0;
+  for (int p = 0; p < nb; p += 4 * NBW) {
+    double *const out = sums + half * (4 * NBW * KT * 64);
+#pragma unroll
+    for (int h = 0; h < NBW; ++h) {
+      const int b = p + wave * NBW + h;
+      if (b < nb) {
+#pragma unroll
+        for (int c = 0; c < KT; ++c) {
+          double sum = xs[8 * b * KT + c] * m[h][0];
+#pragma unroll
+          for (int j = 1; j < 8; ++j) sum = sum + xs[(8 * b + j) * KT + c] * m[h][j];
+          out[((wave * NBW + h) * KT + c) * 64 + lane] = sum;
+        }
+      }
+    }
+    if (p + 4 * NBW < nb) {
+#pragma unroll
+      for (int h = 0; h < NBW; ++h)
+        load_cols(m[h], M, k, 8 * (p + (4 + wave) * NBW + h), w, nr);
+    }
+    __syncthreads();
+    if (wave < KT) {
+      const int cnt = min(4 * NBW, nb - p);
+      for (int b = 0; b < cnt; ++b) t = t + out[(b * KT + wave) * 64 + lane];
+    }
+    half ^= 1;
+  }
+  if (wave < KT) {
+    int cb = 8 * nb, q = 0;
+    if (w - cb >= 4) {
+      double sum = xs[cb * KT + wave] * tail[0];
+#pragma unroll
+      for (int j = 1; j < 4; ++j) sum = sum + xs[(cb + j) * KT + wave] * tail[j];
+      t = t + sum;
+      q = 4;
+    }
+#pragma unroll
+    for (int j = 0; j < 7; ++j)
+      if (j >= q && cb + j < w) t = t + xs[(cb + j) * KT + wave] * tail[j];
+    if (w + first + lane < nr) st_dev(&T[place + wave * a.tcount], t);
+    publish_fence();
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) st_dev(&flags[u], target);
+}
+
+// Workgroup's next (ticket, column tile), ticket-major; -1 past the last.
+__device__ __forceinline__ int next_ticket(const SnArgs &a, int *slot) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    slot[0] = atomicAdd(&a.state[ST_TICKET], 1);
+    slot[1] = 0;
+  }
+  __syncthreads();
+  const int tt = __builtin_amdgcn_readfirstlane(slot[0]);
+  return tt < a.ntick * a.tiles ? tt : -1;
+}
+
+template <int KT>
+__global__ __launch_bounds__(256, 2) void k_supernodal(SnArgs a) {
+  __shared__ double xs[SN_WMAX * KT];
+  __shared__ double sums[2 * 4 * 8 * 64];
+  __shared__ int slot[2];  // the ticket; columns solved of the current top
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int target = ld_dev(&a.state[ST_EPOCH]) + 1;
   for (;;) {
-    // ticket -> (task, column), task-major: the k columns of one task run
-    // side by side (sharing its block in the caches) and every wait is for
-    // an earlier ticket
-    int tt = 0;
-    if (lane == 0) tt = atomicAdd(&a.state[ST_TICKET], 1);
-    tt = __shfl(tt, 0);
-    if (tt >= a.ntasks * a.k) break;
-    const int tk = tt / a.k, colk = tt - tk * a.k;
-    double *const x = a.x + colk * a.ldx;
-    double *const T = a.T + colk * a.tstride;
-    int *const flags = a.flags + (int64_t)colk * a.ntasks;
-    const int2 td = a.task[tk];
-    const int i = __builtin_amdgcn_readfirstlane(td.x);
-    const int chunk = __builtin_amdgcn_readfirstlane(td.y);
-    const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i];
-    const double *M = a.Lx + a.Lp[i];
-    // 1. the tasks that write to this task's inputs (for a later chunk of the
-    // rows below: the supernode's own top)
-    wait_units(a.dptr, a.dlist, tk, flags, target, a.state, a.timeout);
+    const int tt = next_ticket(a, slot);
+    if (tt < 0) break;
+    const int tk = tt / a.tiles, tile = tt - tk * a.tiles;
+    const Cols<KT> col(a, tile);
+    double *const T = a.T + (int64_t)tile * a.tcount * KT;
+    const int u0 = a.tick[tk], u1 = a.tick[tk + 1];
+    const int2 un = a.unit[u0];
+    const int i = __builtin_amdgcn_readfirstlane(un.x);
+    const int chunk = __builtin_amdgcn_readfirstlane(un.y);
+    const int w = a.sup[i + 1] - a.sup[i];
     if (chunk > 0) {
-      // a later chunk of the rows below: the solved top from memory
-      for (int r = lane; r < w; r += 64) xs[r] = ld_dev(&x[s + r]);
-      wave_lds_sync();
+      const int first = (w <= SN_NARROW ? SN_NARROW_ROWS : 0) + (chunk - 1) * 64;
+      below_unit<KT>(a, col, T, u0, tile, i, first, target, xs, sums);
+    } else if (w <= SN_NARROW) {
+      if (u0 + wave < u1) {
+        const int node = __builtin_amdgcn_readfirstlane(a.unit[u0 + wave].x);
+        narrow_unit<KT>(a, col, T, u0 + wave, tile, node, target, xs + wave * 64 * KT, lane);
+      }
     } else {
-      // 2. own rows: b minus the temporaries, in ascending supernode order
-      if (w <= 64)
-        gather_rows<1>(xs, x, T, a.cptr, a.cidx, s, w, 0, lane);
-      else if (w <= 128)
-        gather_rows<2>(xs, x, T, a.cptr, a.cidx, s, w, 0, lane);
-      else if (w <= 256)
-        gather_rows<4>(xs, x, T, a.cptr, a.cidx, s, w, 0, lane);
-      else
-        for (int r0 = 0; r0 < w; r0 += 512)
-          gather_rows<8>(xs, x, T, a.cptr, a.cidx, s, w, r0, lane);
-      wave_lds_sync();
-      // 3. the dense top, column block by column block.  Block (col, B):
-      // lane j < B holds row col+j of the block's columns (and its diagonal)
-      // in mr, and mk the first TOP_ROWS rows per lane of the update after
-      // the block (B = 0: past the last block, nothing loaded).  The entries
-      // do not depend on the solve: with PF the next block's are loaded
-      // while this block is solved.
-      constexpr bool PF = TOP_ROWS >= 4;
-      // Addresses outside the block are clamped into the top, so the loads
-      // need no branches; the values so loaded are never used (a lane's
-      // triangle reads its own row up to its diagonal, the update skips
-      // columns past B and rows past w).  B = 0 loads the top's last entry.
-      auto load_block = [&](int col, int B, double (&mr)[8], double (&mk)[TOP_ROWS][8]) {
-        const int rl = min(lane, B - 1);
+      const int s = a.sup[i], nr = a.nrows[i];
+      const double *M = a.Lx + a.Lp[i];
+      int *const flags = a.flags + (int64_t)tile * a.nunits;
+      int seen = 0;
+      for (int g = wave; g < 4 || 64 * g < w; g += 4) {
+        const int row = min(64 * g + lane, w - 1);
+        double buf[SN_AHEAD][8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) mr[c] = M[(col + rl) + (int64_t)(col + min(c, rl)) * nr];
-        const int k0 = col + B + lane;
-#pragma unroll
-        for (int u = 0; u < TOP_ROWS; ++u) {
-          const int k = k0 + 64 * u;
-#pragma unroll
-          for (int c = 0; c < 8; ++c)
-            mk[u][c] = M[min(k, w - 1) + (int64_t)(col + min(c, B - 1)) * nr];
+        for (int q = 0; q < SN_AHEAD; ++q) load_cols(buf[q], M, row, 8 * q, w, nr);
+        const Diag dg(M[row + (int64_t)row * nr]);
+        if (g < 4) {  // each wave's first group: the entries are on their way
+          if (wave == 0) wait_units(a.dptr, a.dlist, u0, flags, target, a.state, a.timeout);
+          __syncthreads();
         }
-      };
-      double mrow[8], mk[TOP_ROWS][8];
-      int B = w > 0 ? lsolve_block(0, w) : 0;
-      if constexpr (PF) load_block(0, B, mrow, mk);
-      for (int col = 0; col < w;) {
-        const int cn = col + B;
-        const int Bn = cn < w ? lsolve_block(cn, w) : 0;
-        double nrow[8], nk[TOP_ROWS][8];
-        if constexpr (PF)
-          load_block(cn, Bn, nrow, nk);
-        else
-          load_block(col, B, mrow, mk);
-        const int k0 = col + B + lane;
-        // the block's triangle: lane l < B keeps its row's running value;
-        // at step j lane j divides, the quotient is broadcast, and every
-        // lane subtracts its product (each row loses its products in column
-        // order, as the reference computes them)
-        double acc = lane < B ? xs[col + lane] : 0.0, mine = 0.0;
-        double xv[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          if (j < B) {
-            const double q = acc / mrow[j];
-            mine = lane == j ? q : mine;
-            xv[j] = lane_value(q, j);
-            acc = acc - xv[j] * mrow[j];
-          } else {
-            xv[j] = 0.0;
-          }
-        }
-        wave_lds_sync();
-        if (lane < B) xs[col + lane] = mine;
-        // TOP_ROWS rows per lane at a time: all their entries in flight at once
-        for (int kc = k0; kc < w; kc += 64 * TOP_ROWS) {
-          if (kc != k0) {
-#pragma unroll
-            for (int u = 0; u < TOP_ROWS; ++u) {
-              const int k = kc + 64 * u;
-#pragma unroll
-              for (int c = 0; c < 8; ++c)
-                mk[u][c] = M[min(k, w - 1) + (int64_t)(col + min(c, B - 1)) * nr];
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < TOP_ROWS; ++u) {
-            const int k = kc + 64 * u;
-            if (k < w) {
-              double t = xs[k];
-#pragma unroll
-              for (int c = 0; c < 8; ++c)
-                if (c < B) t = t - xv[c] * mk[u][c];
-              xs[k] = t;
-            }
-          }
-        }
-        wave_lds_sync();
-        if constexpr (PF) {
-#pragma unroll
-          for (int c = 0; c < 8; ++c) mrow[c] = nrow[c];
-#pragma unroll
-          for (int u = 0; u < TOP_ROWS; ++u)
-#pragma unroll
-            for (int c = 0; c < 8; ++c) mk[u][c] = nk[u][c];
-        }
-        col = cn;
-        B = Bn;
+        if (64 * g < w) top_group<KT>(a, col, T, buf, dg, g, s, w, nr, M, xs, &slot[1], seen, lane);
       }
-      for (int r = lane; r < w; r += 64) st_dev(&x[s + r], xs[r]);
+      publish_fence();
+      __syncthreads();
+      if (threadIdx.x == 0) st_dev(&flags[u0], target);
     }
-    // 4. this task's chunk of the rows below: products with the solved top
-    // into T; SN_ROWS rows per lane, each column block's entries of those
-    // rows loaded together, each row's sum kept in the reference's order.
-    // Lanes past the last row load row nr-1 (no branch per load) and store
-    // nothing; the tail skips the columns past its block.
-    const int tb = a.tb[i];
-    {
-      const int k0 = w + chunk * SN_CHUNK + lane;
-      double t[SN_ROWS];
-#pragma unroll
-      for (int u = 0; u < SN_ROWS; ++u) t[u] = 0.0;
-      // full blocks of eight, WIDE (one right-hand side: 4, where the
-      // registers allow; else 2) and then 2 at a time: all their entries in
-      // flight together, each block's sum formed and added as the reference
-      // orders it
-      constexpr int WIDE = TOP_ROWS >= 4 ? 4 : 2;
-      int col = 0;
-      for (; w - col >= 8 * WIDE; col += 8 * WIDE) product_blocks<WIDE>(t, xs, M, k0, nr, col);
-      for (; w - col >= 16; col += 16) product_blocks<2>(t, xs, M, k0, nr, col);
-      // the last columns in blocks of 8, 4 and 1
-      while (col < w) {
-        const int B = matvec_block(col, w);
-        double mk[SN_ROWS][8];
-#pragma unroll
-        for (int u = 0; u < SN_ROWS; ++u) {
-          const int k = k0 + 64 * u;
-#pragma unroll
-          for (int c = 0; c < 8; ++c)
-            mk[u][c] = M[min(k, nr - 1) + (int64_t)(col + min(c, B - 1)) * nr];
-        }
-#pragma unroll
-        for (int u = 0; u < SN_ROWS; ++u) {
-          double sum = xs[col] * mk[u][0];
-#pragma unroll
-          for (int c = 1; c < 8; ++c)
-            if (c < B) sum = sum + xs[col + c] * mk[u][c];
-          t[u] = t[u] + sum;
-        }
-        col += B;
-      }
-#pragma unroll
-      for (int u = 0; u < SN_ROWS; ++u)
-        if (k0 + 64 * u < nr) st_dev(&T[tb + k0 + 64 * u - w], t[u]);
-    }
-    // 5. publish
-    publish_fence();
-    if (lane == 0) st_dev(&flags[tk], target);
-    wave_lds_sync();
   }
   persistent_finish(a.state, a.total_waves);
 }
-
 
 // ---------------------------------------------------- transposed solve
 // L^T x = b on the same storage (the semantics of parsy's blockedLTsolve,
-// sparse_blas/parsy/triangularSolve/Triangular_BCSC.cpp:125-186), supernodes
-// level by level from the root (torder); one wave per (supernode, column)
-// ticket, supernode-major, so every wait is for an earlier ticket.  Per supernode:
-// wait for the supernodes owning its rows below (solved earlier); per top
-// column c (lanes), t = sum over the rows below, ascending, of M[r, c] times
-// x at that row (the rows' x staged in LDS chunk by chunk), x[s+c] -= t;
-// then the top's transposed solve in LDS from the last column: x_c /= M[c, c]
-// and every x_r, r < c, loses M[c, r] * x_c.  The order is the oracle's
-// (orc_sptrsv_csc_block_t).
+// sparse_blas/parsy/triangularSolve/Triangular_BCSC.cpp:125-186), tickets
+// level by level from the root.  Per supernode: for each top column c, t =
+// sum over the rows below, ascending, of M[r, c] times x at that row, and
+// x[s+c] -= t; then the top's transposed solve from its last column: x_c /=
+// M[c, c] and every x_r, r < c, loses M[c, r] * x_c.  The order is the
+// oracle's (orc_sptrsv_csc_block_t).
 //
-// NT column tiles of 64 per lane (NT * 64 >= w).  The matrix entries do
-// not depend on the solve, so their loads are batched: RB rows below per
-// round (RB * NT loads in flight per lane), and the top's columns in groups
-// of D whose entries load while the group before is finished.  Addresses
-// are clamped into the block (no branch per load); the values so loaded are
-// not used.
-constexpr int SN_TCHUNK = 256;  // rows below staged per pass
+// A narrow supernode with at most SN_NARROW_ROWS rows below is one wave's
+// work, four to a ticket.  Otherwise 64 of its columns' sums over the rows
+// below are a ticket (the workgroup: tiles of 64 x 64 entries are loaded
+// along the rows, coalesced, and turned in LDS so that a lane then owns a
+// column), and its top another (waves take groups of 64 columns from the
+// last one, hand x on through LDS as in the forward solve, and wait for
+// their own group's sums only).
 
-template <int NT>
-__device__ __forceinline__ void sn_solve_t_top(double *xs, double *xb, const double *x,
-                                               const double *M, const int *rows, int s,
-                                               int w, int nr, int lane) {
-  constexpr int RB = 32 / NT;           // rows below per round
-  constexpr int D = NT >= 8 ? 32 / NT : 8;  // top columns per group
-  int cl[NT];
+// Rows r0 .. r0+7 of one column's entries (lane = column; the pointer is at
+// its row 0); rows past `last` repeat it.
+__device__ __forceinline__ void load_rows(double (&m)[8], const double *C, int r0, int last) {
+  if (r0 + 7 <= last) {
 #pragma unroll
-  for (int j = 0; j < NT; ++j) cl[j] = min(lane + 64 * j, w - 1);
-  // 1. the rows below: one running sum per top column, rows ascending
-  double t[NT];
+    for (int j = 0; j < 8; ++j) m[j] = C[r0 + j];
+  } else {
 #pragma unroll
-  for (int j = 0; j < NT; ++j) t[j] = 0.0;
-  for (int r0 = w; r0 < nr; r0 += SN_TCHUNK) {
-    const int cnt = min(SN_TCHUNK, nr - r0);
-    for (int r = lane; r < cnt; r += 64) xb[r] = ld_dev(&x[rows[r0 - w + r]]);
-    wave_lds_sync();
-    for (int rb = 0; rb < cnt; rb += RB) {
-      double mv[RB][NT];
-#pragma unroll
-      for (int u = 0; u < RB; ++u) {
-        const int row = r0 + min(rb + u, cnt - 1);
-#pragma unroll
-        for (int j = 0; j < NT; ++j) mv[u][j] = M[row + (int64_t)cl[j] * nr];
-      }
-#pragma unroll
-      for (int u = 0; u < RB; ++u) {
-        if (rb + u < cnt) {
-          const double v = xb[rb + u];
-          const bool first = r0 + rb + u == w;
-#pragma unroll
-          for (int j = 0; j < NT; ++j) {
-            const double p = mv[u][j] * v;
-            t[j] = first ? p : t[j] + p;
-          }
-        }
-      }
-    }
-    wave_lds_sync();
+    for (int j = 0; j < 8; ++j) m[j] = C[max(min(r0 + j, last), 0)];
   }
+}
+
+// Columns 64g .. 64g+63 of a top, by one wave: x from LDS for the columns of
+// later groups (xs and the count are not used by a narrow supernode, whose
+// only group is the last).
+template <int KT>
+__device__ __forceinline__ void top_group_t(double (&acc)[KT], double (&res)[KT],
+                                            double (&buf)[SN_AHEAD][8], const Diag &dg, int g,
+                                            int w, int nr, const double *M, double *xs,
+                                            int *prog, int &seen, int lane) {
+  const double *C = M + (int64_t)min(64 * g + lane, w - 1) * nr;
+  const int top = (w - 1) / 8;  // last block of eight rows
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int c = lane + 64 * j;
-    if (c < w) xs[c] = nr > w ? x[s + c] - t[j] : x[s + c];
-  }
-  wave_lds_sync();
-  // 2. the top, transposed, from the last column, D columns per group
-  auto load_group = [&](int cb, double (&m)[D][NT], double (&dg)[D]) {
+  for (int c = 0; c < KT; ++c) res[c] = 0.0;
+  int b = top;
+  auto later = [&](double (&m)[8]) {
+    const int c0 = 8 * b, B = min(8, w - c0);
+    lds_wait(prog, w - c0, seen);
+    double xv[8][KT];
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
-      const int c = max(cb - k, 0);
+    for (int j = 0; j < 8; ++j)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) m[k][j] = M[c + (int64_t)cl[j] * nr];
-      dg[k] = M[c + (int64_t)c * nr];
+      for (int c = 0; c < KT; ++c) xv[j][c] = xs[min(c0 + j, w - 1) * KT + c];
+#pragma unroll
+    for (int j = 7; j >= 0; --j)
+      if (j < B) {
+#pragma unroll
+        for (int c = 0; c < KT; ++c) acc[c] = acc[c] - m[j] * xv[j][c];
+      }
+    hold<KT>(acc);
+  };
+  auto own = [&](double (&m)[8]) {
+    const int c0 = 8 * b, lb = c0 - 64 * g;
+    solve_block<KT, true>(acc, res, m, dg, lb, w - c0, lane,
+                          [&](int j) { return C[c0 + j]; });
+    if (xs) {
+      if (lane >= lb && lane < lb + 8 && 64 * g + lane < w) {
+#pragma unroll
+        for (int c = 0; c < KT; ++c) xs[(64 * g + lane) * KT + c] = res[c];
+      }
+      lds_publish(prog, w - c0, lane);
     }
   };
-  double mc[D][NT], dc[D];
-  load_group(w - 1, mc, dc);
-  for (int cb = w - 1; cb >= 0; cb -= D) {
-    double mn[D][NT], dn[D];
-    load_group(cb - D, mn, dn);
+  // SN_AHEAD blocks per round, slot q of round n holding block top - 4n - q
+  for (int b0 = top; b0 >= 8 * g; b0 -= SN_AHEAD) {
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
-      const int c = cb - k;
-      if (c >= 0) {
-        const double y = xs[c] / dc[k];
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          const int r = lane + 64 * j;
-          if (r < c) xs[r] = xs[r] - mc[k][j] * y;
-        }
-        if (lane == (c & 63)) xs[c] = y;
-        wave_lds_sync();
+    for (int q = 0; q < SN_AHEAD; ++q) {
+      b = b0 - q;
+      if (b >= 8 * g) {
+        if (b >= 8 * g + 8)
+          later(buf[q]);
+        else
+          own(buf[q]);
       }
-    }
-#pragma unroll
-    for (int k = 0; k < D; ++k) {
-      dc[k] = dn[k];
-#pragma unroll
-      for (int j = 0; j < NT; ++j) mc[k][j] = mn[k][j];
+      load_rows(buf[q], C, max(8 * (b - SN_AHEAD), 0), nr - 1);
     }
   }
 }
 
-__global__ __launch_bounds__(256) void k_supernodal_t(SnArgs a) {
-  __shared__ double slab[4][SN_WMAX];
-  __shared__ double below[4][SN_TCHUNK];
-  double *xs = slab[threadIdx.x >> 6];
-  double *xb = below[threadIdx.x >> 6];
+__device__ __forceinline__ void preload_t(double (&buf)[SN_AHEAD][8], const double *M, int g,
+                                          int w, int nr, int lane) {
+  const double *C = M + (int64_t)min(64 * g + lane, w - 1) * nr;
+  const int top = (w - 1) / 8;
+#pragma unroll
+  for (int q = 0; q < SN_AHEAD; ++q) load_rows(buf[q], C, max(8 * (top - q), 0), nr - 1);
+}
+
+template <int KT>
+__device__ __forceinline__ void narrow_unit_t(const SnArgs &a, const Cols<KT> &col, int u,
+                                              int tile, int i, int target, int lane) {
+  const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i], below = nr - w;
+  const double *M = a.Lx + a.Lp[i];
+  const int *rows = a.rowb + a.tb[i];
+  const int c = min(lane, w - 1);
+  double buf[SN_AHEAD][8];
+  preload_t(buf, M, 0, w, nr, lane);
+  const Diag dg(M[c + (int64_t)c * nr]);
+  double acc[KT], res[KT], t[KT];
+#pragma unroll
+  for (int q = 0; q < KT; ++q) {
+    acc[q] = col.x[q][s + c];
+    t[q] = 0.0;
+  }
+  const double *C = M + (int64_t)c * nr + w;
+  int *const flags = a.flags + (int64_t)tile * a.nunits;
+  double ma[8], mb[8];
+  if (below > 0) {
+    load_rows(ma, C, 0, below - 1);
+    wait_units(a.dptr, a.dlist, u, flags, target, a.state, a.timeout);
+    for (int r0 = 0; r0 < below; r0 += 64) {
+      double xr[KT];
+      const int row = rows[min(r0 + lane, below - 1)];
+#pragma unroll
+      for (int q = 0; q < KT; ++q) xr[q] = ld_dev(&col.x[q][row]);
+      auto add = [&](const double (&m)[8], int r) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (r + j < below) {
+#pragma unroll
+            for (int q = 0; q < KT; ++q) {
+              const double p = m[j] * lane_value(xr[q], (r + j) & 63);
+              t[q] = r + j == 0 ? p : t[q] + p;
+            }
+          }
+      };
+      const int end = min(r0 + 64, below);
+      for (int r = r0; r < end; r += 16) {
+        load_rows(mb, C, min(r + 8, below - 1), below - 1);
+        add(ma, r);
+        load_rows(ma, C, min(r + 16, below - 1), below - 1);
+        if (r + 8 < end) add(mb, r + 8);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < KT; ++q) acc[q] = acc[q] - t[q];
+  }
+  int seen = 0;
+  top_group_t<KT>(acc, res, buf, dg, 0, w, nr, M, nullptr, nullptr, seen, lane);
+#pragma unroll
+  for (int q = 0; q < KT; ++q)
+    if (lane < w && col.live[q]) st_dev(&col.x[q][s + lane], res[q]);
+  publish_fence();
+  if (lane == 0) st_dev(&flags[u], target);
+}
+
+constexpr int SN_PITCH = 65;  // doubles per column of a turned tile (no bank conflicts)
+
+// The sums over the rows below of columns 64g .. 64g+63, by the workgroup.
+// Tiles of 64 rows; wave v loads 16 columns of a tile along its rows, the
+// next tile's entries and x in flight while this one is summed; wave c then
+// adds right-hand side c's products, a lane per column.
+template <int KT>
+__device__ __forceinline__ void below_unit_t(const SnArgs &a, int u, int tile, int i, int g,
+                                             int target, double *turn, double *xrow) {
   const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i], below = nr - w;
+  const double *M = a.Lx + a.Lp[i] + w;
+  const int *rows = a.rowb + a.tb[i];
+  int *const flags = a.flags + (int64_t)tile * a.nunits;
+  double m[16];
+  auto load = [&](int r0) {
+    const int r = min(r0 + lane, below - 1);
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      m[j] = at(M + (int64_t)min(64 * g + 16 * wave + j, w - 1) * nr, r);
+  };
+  load(0);
+  int row = rows[min(lane, below - 1)];
+  if (wave == 0) wait_units(a.dptr, a.dlist, u, flags, target, a.state, a.timeout);
+  __syncthreads();
+  // wave c of the first KT holds x of right-hand side c at the tile's rows
+  const int cw = tile * KT + wave;
+  double *const xc = a.x + (int64_t)min(cw, a.k - 1) * a.ldx;
+  const bool mine = cw < a.k;
+  double xr = wave < KT ? ld_dev(&xc[row]) : 0.0;
+  double t = 0.0;
+  int half = 0;
+  for (int r0 = 0; r0 < below; r0 += 64) {
+    double *const tl = turn + half * 64 * SN_PITCH;
+    double *const xl = xrow + (half * KT + min(wave, KT - 1)) * 64;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) tl[(16 * wave + j) * SN_PITCH + lane] = m[j];
+    if (wave < KT) xl[lane] = xr;
+    if (r0 + 64 < below) {
+      load(r0 + 64);
+      row = rows[min(r0 + 64 + lane, below - 1)];
+      if (wave < KT) xr = ld_dev(&xc[row]);
+    }
+    __syncthreads();
+    if (wave < KT) {
+      const int cnt = min(64, below - r0);
+      int r = 0;
+      if (r0 == 0) {
+        t = tl[lane * SN_PITCH] * xl[0];
+        r = 1;
+      }
+      for (; r + 8 <= cnt; r += 8) {
+        double p[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = tl[lane * SN_PITCH + r + j] * xl[r + j];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t = t + p[j];
+      }
+      for (; r < cnt; ++r) t = t + tl[lane * SN_PITCH + r] * xl[r];
+    }
+    half ^= 1;
+  }
+  if (wave < KT) {
+    const int c = 64 * g + lane;
+    if (c < w && mine) st_dev(&xc[s + c], xc[s + c] - t);
+    publish_fence();
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) st_dev(&flags[u], target);
+}
+
+template <int KT>
+__global__ __launch_bounds__(256, 2) void k_supernodal_t(SnArgs a) {
+  // a top's x, or two turned tiles and the x at their rows
+  constexpr int TILES = 2 * 64 * SN_PITCH + 2 * KT * 64;
+  __shared__ double mem[SN_WMAX * KT > TILES ? SN_WMAX * KT : TILES];
+  __shared__ int slot[2];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int target = ld_dev(&a.state[ST_EPOCH]) + 1;
   for (;;) {
-    int tt = 0;
-    if (lane == 0) tt = atomicAdd(&a.state[ST_TICKET], 1);
-    tt = __shfl(tt, 0);
-    if (tt >= a.m * a.k) break;
-    const int ti = tt / a.k, colk = tt - ti * a.k;
-    const int i = a.torder[ti];
-    double *const x = a.x + colk * a.ldx;
-    int *const flags = a.flags + (int64_t)colk * a.ntasks;
-    wait_units(a.tdptr, a.tdlist, i, flags, target, a.state, a.timeout);
+    const int tt = next_ticket(a, slot);
+    if (tt < 0) break;
+    const int tk = tt / a.tiles, tile = tt - tk * a.tiles;
+    const Cols<KT> col(a, tile);
+    const int u0 = a.tick[tk], u1 = a.tick[tk + 1];
+    const int2 un = a.unit[u0];
+    const int i = __builtin_amdgcn_readfirstlane(un.x);
+    const int chunk = __builtin_amdgcn_readfirstlane(un.y);
     const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i];
-    const double *M = a.Lx + a.Lp[i];
-    const int *rows = a.rowb + a.tb[i];
-    if (w <= 64)
-      sn_solve_t_top<1>(xs, xb, x, M, rows, s, w, nr, lane);
-    else if (w <= 128)
-      sn_solve_t_top<2>(xs, xb, x, M, rows, s, w, nr, lane);
-    else if (w <= 256)
-      sn_solve_t_top<4>(xs, xb, x, M, rows, s, w, nr, lane);
-    else if (w <= 512)
-      sn_solve_t_top<8>(xs, xb, x, M, rows, s, w, nr, lane);
-    else
-      sn_solve_t_top<16>(xs, xb, x, M, rows, s, w, nr, lane);
-    for (int r = lane; r < w; r += 64) st_dev(&x[s + r], xs[r]);
-    publish_fence();
-    if (lane == 0) st_dev(&flags[i], target);
-    wave_lds_sync();
+    int *const flags = a.flags + (int64_t)tile * a.nunits;
+    if (chunk > 0) {
+      below_unit_t<KT>(a, u0, tile, i, chunk - 1, target, mem, mem + 2 * 64 * SN_PITCH);
+    } else if (w <= SN_NARROW && nr - w <= SN_NARROW_ROWS) {
+      if (u0 + wave < u1) {
+        const int node = __builtin_amdgcn_readfirstlane(a.unit[u0 + wave].x);
+        narrow_unit_t<KT>(a, col, u0 + wave, tile, node, target, lane);
+      }
+    } else {
+      const double *M = a.Lx + a.Lp[i];
+      const int G = (w + 63) / 64, ub = a.tbelow[i];
+      int seen = 0;
+      for (int g = G - 1 - wave; g >= 0; g -= 4) {
+        double buf[SN_AHEAD][8];
+        preload_t(buf, M, g, w, nr, lane);
+        const int c = min(64 * g + lane, w - 1);
+        const Diag dg(M[c + (int64_t)c * nr]);
+        if (ub >= 0)
+          wait_flag(&flags[ub + g], target, a.state, a.timeout);
+        double acc[KT], res[KT];
+#pragma unroll
+        for (int q = 0; q < KT; ++q) acc[q] = ld_dev(&col.x[q][s + c]);
+        top_group_t<KT>(acc, res, buf, dg, g, w, nr, M, mem, &slot[1], seen, lane);
+#pragma unroll
+        for (int q = 0; q < KT; ++q)
+          if (64 * g + lane < w && col.live[q]) st_dev(&col.x[q][s + c], res[q]);
+      }
+      publish_fence();
+      __syncthreads();
+      if (threadIdx.x == 0) st_dev(&flags[u0], target);
+    }
   }
   persistent_finish(a.state, a.total_waves);
+}
+
+}  // namespace
+
+namespace {
+
+// Units and tickets of one direction, level by level.  Per level: the column
+// groups of the wide supernodes (transposed only; they come before the top
+// that uses them), the wide tops, the narrow supernodes four to a ticket, and
+// the further rows below (forward only, 64 per unit).
+struct SnSchedule {
+  std::vector<int2> unit;  // (supernode, 0 or 1 + chunk)
+  std::vector<int> tick;   // unit bounds per ticket
+  std::vector<int> top;    // per supernode: the unit that solves its top
+  std::vector<int> first;  // per supernode: its first chunk unit, or -1
+};
+
+void sn_schedule(int m, const int *h_sup, const std::vector<int> &lev,
+                 const std::vector<int> &tb, bool transposed, SnSchedule &s) {
+  std::vector<int> order(m);
+  for (int i = 0; i < m; ++i) order[i] = transposed ? m - 1 - i : i;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return lev[x] < lev[y]; });
+  s.tick.assign(1, 0);
+  s.top.assign(m, -1);
+  s.first.assign(m > 0 ? m : 1, -1);
+  auto width = [&](int i) { return h_sup[i + 1] - h_sup[i]; };
+  auto below = [&](int i) { return tb[i + 1] - tb[i]; };
+  auto narrow = [&](int i) {
+    return width(i) <= SN_NARROW && (!transposed || below(i) <= SN_NARROW_ROWS);
+  };
+  auto close = [&] { s.tick.push_back((int)s.unit.size()); };
+  auto chunks = [&](int i, int count) {
+    for (int c = 0; c < count; ++c) {
+      if (c == 0) s.first[i] = (int)s.unit.size();
+      s.unit.push_back(make_int2(i, c + 1));
+      close();
+    }
+  };
+  for (int a = 0, b = 0; a < m; a = b) {
+    while (b < m && lev[order[b]] == lev[order[a]]) ++b;
+    if (transposed)
+      for (int j = a; j < b; ++j)
+        if (!narrow(order[j]) && below(order[j]) > 0) chunks(order[j], (width(order[j]) + 63) / 64);
+    for (int j = a; j < b; ++j)
+      if (!narrow(order[j])) {
+        s.top[order[j]] = (int)s.unit.size();
+        s.unit.push_back(make_int2(order[j], 0));
+        close();
+      }
+    int open = 0;
+    for (int j = a; j < b; ++j)
+      if (narrow(order[j])) {
+        s.top[order[j]] = (int)s.unit.size();
+        s.unit.push_back(make_int2(order[j], 0));
+        if (++open == 4) {
+          close();
+          open = 0;
+        }
+      }
+    if (open) close();
+    if (!transposed)
+      for (int j = a; j < b; ++j) {
+        const int i = order[j], rest = below(i) - (narrow(i) ? SN_NARROW_ROWS : 0);
+        if (rest > 0) chunks(i, (rest + 63) / 64);
+      }
+  }
+}
+
+void flatten_deps(std::vector<std::vector<int>> &deps, std::vector<int> &ptr,
+                  std::vector<int> &list) {
+  ptr.assign(1, 0);
+  list.clear();
+  for (std::vector<int> &d : deps) {
+    std::sort(d.begin(), d.end());
+    d.erase(std::unique(d.begin(), d.end()), d.end());
+    list.insert(list.end(), d.begin(), d.end());
+    ptr.push_back((int)list.size());
+  }
 }
 
 }  // namespace
@@ -546,91 +941,92 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
     tb[i + 1] = tb[i] + (nr - w);
   }
   for (int r = 0; r < n; ++r) cnt[r + 1] += cnt[r];
-  // contributions per row in ascending supernode order; dependency lists
-  std::vector<int> cidx(cnt[n] > 0 ? cnt[n] : 1), fill(cnt.begin(), cnt.end() - 1);
+  // the rows' lists, in ascending supernode order, and the place in T of each
+  // row below: entry j of the rows one wave gathers (64 consecutive ones of a
+  // supernode) lies side by side, lists padded to the longest; rows of very
+  // uneven lists (padding past three entries in four) keep theirs contiguous
+  std::vector<int> tdst(tb[m] > 0 ? tb[m] : 1), rowb(tb[m] > 0 ? tb[m] : 1);
+  std::vector<int4> list(n > 0 ? n : 1, make_int4(0, 0, 0, 0));
+  int64_t tcount = 0;
+  for (int i = 0; i < m; ++i)
+    for (int r0 = h_sup[i]; r0 < h_sup[i + 1]; r0 += 64) {
+      const int r1 = std::min(r0 + 64, h_sup[i + 1]);
+      const int64_t total = cnt[r1] - cnt[r0];
+      int64_t longest = 0;
+      for (int r = r0; r < r1; ++r) longest = std::max<int64_t>(longest, cnt[r + 1] - cnt[r]);
+      const bool side = longest * (r1 - r0) <= 4 * total;
+      for (int r = r0; r < r1; ++r)
+        if (cnt[r + 1] > cnt[r])
+          list[r] = make_int4((int)(tcount + (side ? r - r0 : cnt[r] - cnt[r0])), 0,
+                              side ? r1 - r0 : 1, 0);
+      tcount += side ? longest * (r1 - r0) : total;
+      if (tcount > INT_MAX)
+        return fail(SYMAMD_ERR_NOT_SUPPORTED, "supernodal analyze: over 2^31 temporaries");
+    }
   std::vector<int> owner(n);
   for (int i = 0; i < m; ++i)
     for (int c = h_sup[i]; c < h_sup[i + 1]; ++c) owner[c] = i;
-  // tasks: supernode i's top (with the first SN_CHUNK rows below), then one
-  // task per further SN_CHUNK rows below.  Tickets are dealt level by level
-  // (a supernode's level is one above the highest of the supernodes writing
-  // to its rows), so every leaf is taken before any supernode that waits,
-  // and the chain of the last subtree does not start behind the others;
-  // every task still waits only for tasks dealt before it.
-  std::vector<int> lev(m, 0);
+  // levels (a supernode is one above the highest of the supernodes writing
+  // to its rows; transposed: one below the deepest of the supernodes owning
+  // its rows below): tickets are dealt level by level, so every leaf is taken
+  // before any supernode that waits, and every unit waits only for units
+  // dealt before it
+  std::vector<int> lev(m, 0), tlev(m, 0);
+  int old_tasks = 0;
   for (int i = 0; i < m; ++i) {
     const int w = h_sup[i + 1] - h_sup[i];
-    for (int r = w; r < h_nrows[i]; ++r) {
-      const int o = owner[h_Li[h_Lp[i] + r]];
-      lev[o] = std::max(lev[o], lev[i] + 1);
-    }
-  }
-  std::vector<int> order(m);
-  for (int i = 0; i < m; ++i) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return lev[x] < lev[y]; });
-  std::vector<int> first(m + 1, 0), ntask(m);  // first[i]: ticket of i's top
-  int ntasks = 0;
-  for (int i : order) {
-    const int below = h_nrows[i] - (h_sup[i + 1] - h_sup[i]);
-    ntask[i] = std::max(1, (below + SN_CHUNK - 1) / SN_CHUNK);
-    first[i] = ntasks;
-    ntasks += ntask[i];
-  }
-  std::vector<int2> task(ntasks > 0 ? ntasks : 1);
-  for (int i = 0; i < m; ++i)
-    for (int c = 0; c < ntask[i]; ++c) task[first[i] + c] = make_int2(i, c);
-  // a top task waits for the tasks writing its rows' temporaries, a later
-  // chunk for its supernode's top
-  std::vector<std::vector<int>> deps(ntasks);
-  for (int i = 0; i < m; ++i) {
-    const int w = h_sup[i + 1] - h_sup[i];
-    for (int k = 0; k < h_nrows[i] - w; ++k) {
-      const int row = h_Li[h_Lp[i] + w + k];
-      cidx[fill[row]++] = tb[i] + k;
-      std::vector<int> &d = deps[first[owner[row]]];
-      const int producer = first[i] + k / SN_CHUNK;
-      if (d.empty() || d.back() != producer) d.push_back(producer);
-    }
-    for (int t = first[i] + 1; t < first[i] + ntask[i]; ++t) deps[t].push_back(first[i]);
-  }
-  // transposed solve: the rows below of each supernode (in temporaries
-  // order) and the supernodes owning them, which it waits for
-  std::vector<int> rowb(tb[m] > 0 ? tb[m] : 1), tdptr(m + 1, 0), tdlist;
-  for (int i = 0; i < m; ++i) {
-    const int w = h_sup[i + 1] - h_sup[i];
-    std::vector<int> own;
     for (int k = 0; k < h_nrows[i] - w; ++k) {
       const int row = h_Li[h_Lp[i] + w + k];
       rowb[tb[i] + k] = row;
-      own.push_back(owner[row]);
+      tdst[tb[i] + k] = list[row].x + list[row].y++ * list[row].z;
+      lev[owner[row]] = std::max(lev[owner[row]], lev[i] + 1);
     }
-    std::sort(own.begin(), own.end());
-    own.erase(std::unique(own.begin(), own.end()), own.end());
-    tdlist.insert(tdlist.end(), own.begin(), own.end());
-    tdptr[i + 1] = (int)tdlist.size();
+    old_tasks += std::max(1, (h_nrows[i] - w + 127) / 128);
   }
-  // transposed tickets level by level from the root: a supernode's level is
-  // one below the deepest of the supernodes owning its rows below (all of
-  // higher index), so each waits only for tickets dealt before it, and no
-  // subtree's waiting supernodes hold the waves another chain needs
-  std::vector<int> tlev(m, 0), torder(m > 0 ? m : 1);
   for (int i = m - 1; i >= 0; --i)
-    for (int e = tdptr[i]; e < tdptr[i + 1]; ++e) tlev[i] = std::max(tlev[i], tlev[tdlist[e]] + 1);
-  for (int i = 0; i < m; ++i) torder[i] = m - 1 - i;
-  std::stable_sort(torder.begin(), torder.begin() + m,
-                   [&](int x, int y) { return tlev[x] < tlev[y]; });
-  std::vector<int> dptr(ntasks + 1, 0), dlist;
-  for (int j = 0; j < ntasks; ++j) {
-    std::sort(deps[j].begin(), deps[j].end());
-    deps[j].erase(std::unique(deps[j].begin(), deps[j].end()), deps[j].end());
-    dlist.insert(dlist.end(), deps[j].begin(), deps[j].end());
-    dptr[j + 1] = (int)dlist.size();
+    for (int k = tb[i]; k < tb[i + 1]; ++k) tlev[i] = std::max(tlev[i], tlev[owner[rowb[k]]] + 1);
+  SnSchedule fwd, bwd;
+  sn_schedule(m, h_sup, lev, tb, false, fwd);
+  sn_schedule(m, h_sup, tlev, tb, true, bwd);
+  // forward: a top waits for the units that write its rows' temporaries, a
+  // chunk of the rows below for its top
+  std::vector<std::vector<int>> deps(fwd.unit.size());
+  for (int i = 0; i < m; ++i) {
+    const int head = h_sup[i + 1] - h_sup[i] <= SN_NARROW ? SN_NARROW_ROWS : 0;
+    for (int k = 0; k < tb[i + 1] - tb[i]; ++k) {
+      const int producer = k < head ? fwd.top[i] : fwd.first[i] + (k - head) / 64;
+      std::vector<int> &d = deps[fwd.top[owner[rowb[tb[i] + k]]]];
+      if (d.empty() || d.back() != producer) d.push_back(producer);
+    }
   }
+  for (size_t u = 0; u < fwd.unit.size(); ++u)
+    if (fwd.unit[u].y > 0) deps[u].push_back(fwd.top[fwd.unit[u].x]);
+  std::vector<int> dptr, dlist, tdptr, tdlist;
+  flatten_deps(deps, dptr, dlist);
+  // transposed: the units that read x at the rows below (a narrow supernode,
+  // the column groups of a wide one) wait for the tops of their owners; a
+  // wide top waits for its own groups by tag
+  deps.assign(bwd.unit.size(), {});
+  for (size_t u = 0; u < bwd.unit.size(); ++u) {
+    const int i = bwd.unit[u].x;
+    if (bwd.unit[u].y == 0 && bwd.first[i] >= 0) continue;
+    std::vector<int> &d = deps[u];
+    for (int k = tb[i]; k < tb[i + 1]; ++k) {
+      const int o = bwd.top[owner[rowb[k]]];
+      if (d.empty() || d.back() != o) d.push_back(o);
+    }
+  }
+  flatten_deps(deps, tdptr, tdlist);
   auto *q = new symamd_snplan_s();
   q->n = n;
   q->m = m;
-  q->tcount = tb[m];
-  q->ntasks = ntasks;
+  q->tcount = tcount;
+  q->ntasks = old_tasks;
+  q->units = (int)fwd.unit.size();
+  q->tickets = (int)fwd.tick.size() - 1;
+  q->tunits = (int)bwd.unit.size();
+  q->ttickets = (int)bwd.tick.size() - 1;
+  const int64_t flags = std::max(1, std::max(q->units, q->tunits));
   int rc = SYMAMD_OK;
   auto up = [&](int **dst, const int *src, size_t count) {
     if (rc != SYMAMD_OK) return;
@@ -642,27 +1038,29 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
   up(&q->d_nrows, h_nrows, m);
   up(&q->d_Lp, h_Lp, m + 1);
   up(&q->d_tb, tb.data(), m + 1);
-  up(&q->d_cptr, cnt.data(), n + 1);
-  up(&q->d_cidx, cidx.data(), cnt[n]);
-  up(&q->d_dptr, dptr.data(), ntasks + 1);
-  up(&q->d_dlist, dlist.data(), dlist.size());
-  up(&q->d_task, reinterpret_cast<const int *>(task.data()), 2 * (size_t)ntasks);
+  up(&q->d_list, reinterpret_cast<const int *>(list.data()), 4 * (size_t)n);
+  up(&q->d_tdst, tdst.data(), tb[m]);
   up(&q->d_rowb, rowb.data(), tb[m]);
-  up(&q->d_tdptr, tdptr.data(), m + 1);
+  up(&q->d_unit, reinterpret_cast<const int *>(fwd.unit.data()), 2 * fwd.unit.size());
+  up(&q->d_tick, fwd.tick.data(), fwd.tick.size());
+  up(&q->d_dptr, dptr.data(), dptr.size());
+  up(&q->d_dlist, dlist.data(), dlist.size());
+  up(&q->d_tunit, reinterpret_cast<const int *>(bwd.unit.data()), 2 * bwd.unit.size());
+  up(&q->d_ttick, bwd.tick.data(), bwd.tick.size());
+  up(&q->d_tdptr, tdptr.data(), tdptr.size());
   up(&q->d_tdlist, tdlist.data(), tdlist.size());
-  up(&q->d_torder, torder.data(), m);
+  up(&q->d_tbelow, bwd.first.data(), m);
   if (rc == SYMAMD_OK &&
       (hipMalloc(&q->d_T, sizeof(double) * (q->tcount > 0 ? q->tcount : 1)) != hipSuccess ||
-       hipMalloc(&q->d_flags, sizeof(int) * (ntasks > 0 ? ntasks : 1)) != hipSuccess ||
+       hipMalloc(&q->d_flags, sizeof(int) * flags) != hipSuccess ||
        hipMalloc(&q->d_state, sizeof(int) * ST_WORDS) != hipSuccess ||
-       hipMemset(q->d_flags, 0, sizeof(int) * (ntasks > 0 ? ntasks : 1)) != hipSuccess ||
+       hipMemset(q->d_flags, 0, sizeof(int) * flags) != hipSuccess ||
        hipMemset(q->d_state, 0, sizeof(int) * ST_WORDS) != hipSuccess))
     rc = fail(SYMAMD_ERR_ALLOC, "supernodal plan allocation failed");
   if (rc != SYMAMD_OK) {
     sn_destroy(q);
     return rc;
   }
-  q->deps = (int64_t)dlist.size();
   (void)h;
   *out = q;
   return SYMAMD_OK;
@@ -676,25 +1074,33 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
     return fail(SYMAMD_ERR_NOT_SUPPORTED,
                 "supernodal solve: %d tasks x %d columns exceed the 32-bit ticket range; "
                 "solve the columns in smaller batches", q->ntasks, k);
-  // temporaries and tags for k columns
-  if (k > q->kcap) {
+  // columns per tile: a row's entries are loaded once for the columns of a
+  // tile, but each step of a top's chain then divides for all of them.  On
+  // the 13-level factor, forward + transposed with tiles of 1 / 2 / 4: k = 2
+  // 1.19 / 1.29 / - ms, k = 4 1.46 / 1.38 / 1.73 ms, k = 32 5.86 / 3.57 /
+  // 3.21 ms.
+  const int kt = k < 4 ? 1 : k < 16 ? 2 : 4;
+  const int tiles = (k + kt - 1) / kt;
+  // temporaries and tags for the tiles' columns
+  if (tiles * kt > q->kcap) {
     double *T = nullptr;
     int *flags = nullptr;
+    const int64_t cols = (int64_t)tiles * kt;
     const int64_t tc = q->tcount > 0 ? q->tcount : 1;
-    const int64_t nt = q->ntasks > 0 ? q->ntasks : 1;
-    if (hipMalloc(&T, sizeof(double) * tc * k) != hipSuccess ||
-        hipMalloc(&flags, sizeof(int) * nt * k) != hipSuccess) {
+    const int64_t nt = std::max(1, std::max(q->units, q->tunits));
+    if (hipMalloc(&T, sizeof(double) * tc * cols) != hipSuccess ||
+        hipMalloc(&flags, sizeof(int) * nt * cols) != hipSuccess) {
       if (T) (void)hipFree(T);
       return fail(SYMAMD_ERR_ALLOC, "supernodal temporaries for %d columns", k);
     }
     // cleared tags read as "not ready" in every epoch
-    SYMAMD_HIP(hipMemsetAsync(flags, 0, sizeof(int) * nt * k, h->stream));
+    SYMAMD_HIP(hipMemsetAsync(flags, 0, sizeof(int) * nt * cols, h->stream));
     SYMAMD_HIP(hipStreamSynchronize(h->stream));
     if (q->d_T) (void)hipFree(q->d_T);
     if (q->d_flags) (void)hipFree(q->d_flags);
     q->d_T = T;
     q->d_flags = flags;
-    q->kcap = k;
+    q->kcap = (int)cols;
   }
   SnArgs a;
   a.sup = q->d_sup;
@@ -704,42 +1110,35 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
   a.x = d_x;
   a.T = q->d_T;
   a.tb = q->d_tb;
-  a.cptr = q->d_cptr;
-  a.cidx = q->d_cidx;
-  a.dptr = q->d_dptr;
-  a.dlist = q->d_dlist;
-  a.task = reinterpret_cast<const int2 *>(q->d_task);
+  a.tdst = q->d_tdst;
+  a.list = reinterpret_cast<const int4 *>(q->d_list);
+  a.unit = reinterpret_cast<const int2 *>(transposed ? q->d_tunit : q->d_unit);
+  a.tick = transposed ? q->d_ttick : q->d_tick;
+  a.dptr = transposed ? q->d_tdptr : q->d_dptr;
+  a.dlist = transposed ? q->d_tdlist : q->d_dlist;
+  a.nunits = transposed ? q->tunits : q->units;
+  a.ntick = transposed ? q->ttickets : q->tickets;
   a.rowb = q->d_rowb;
-  a.tdptr = q->d_tdptr;
-  a.tdlist = q->d_tdlist;
-  a.torder = q->d_torder;
-  a.m = q->m;
+  a.tbelow = q->d_tbelow;
   a.flags = q->d_flags;
   a.state = q->d_state;
-  a.ntasks = q->ntasks;
   a.k = k;
+  a.tiles = tiles;
   a.ldx = ldx;
-  a.tstride = q->tcount > 0 ? q->tcount : 1;
+  a.tcount = q->tcount > 0 ? q->tcount : 1;
   a.timeout = h->timeout_ticks();
-  const void *kfn = transposed ? (const void *)&k_supernodal_t
-                    : k == 1   ? (const void *)&k_supernodal<4>
-                               : (const void *)&k_supernodal<2>;
+  void (*const kfn)(SnArgs) =
+      transposed ? (kt == 1 ? k_supernodal_t<1> : kt == 2 ? k_supernodal_t<2> : k_supernodal_t<4>)
+                 : (kt == 1 ? k_supernodal<1> : kt == 2 ? k_supernodal<2> : k_supernodal<4>);
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, 256, 0) != hipSuccess ||
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)kfn, 256, 0) !=
+          hipSuccess ||
       per_cu < 1)
     per_cu = 1;
-  int64_t grid = (int64_t)per_cu * h->num_cus;
-  const int64_t want = ((int64_t)(transposed ? q->m : q->ntasks) * k + 3) / 4;
-  if (want < grid) grid = want;
-  if (grid < 1) grid = 1;
+  // tickets are dealt in order, so any grid size is safe
+  const int64_t grid = std::min((int64_t)per_cu * h->num_cus, (int64_t)a.ntick * tiles);
   a.total_waves = (int)grid * 4;
-  // tickets are dealt in task order, so any grid size is safe
-  if (transposed)
-    k_supernodal_t<<<(unsigned)grid, 256, 0, h->stream>>>(a);
-  else if (k == 1)
-    k_supernodal<4><<<(unsigned)grid, 256, 0, h->stream>>>(a);
-  else
-    k_supernodal<2><<<(unsigned)grid, 256, 0, h->stream>>>(a);
+  kfn<<<(unsigned)grid, 256, 0, h->stream>>>(a);
   SYMAMD_HIP(hipGetLastError());
   return SYMAMD_OK;
 }
@@ -754,10 +1153,10 @@ int sn_check(symamd_handle h, symamd_snplan_s *q) {
 
 void sn_destroy(symamd_snplan_s *q) {
   if (!q) return;
-  void *ptrs[] = {q->d_sup,   q->d_nrows, q->d_Lp,    q->d_tb,     q->d_cptr,
-                  q->d_cidx,  q->d_dptr,  q->d_dlist, q->d_T,      q->d_flags,
-                  q->d_state, q->d_task,  q->d_rowb,  q->d_tdptr, q->d_tdlist,
-                  q->d_torder};
+  void *ptrs[] = {q->d_sup,  q->d_nrows, q->d_Lp,    q->d_tb,     q->d_list,  q->d_tdst,
+                  q->d_rowb, q->d_unit,  q->d_tick,  q->d_dptr,   q->d_dlist, q->d_tunit,
+                  q->d_ttick, q->d_tdptr, q->d_tdlist, q->d_tbelow, q->d_T,   q->d_flags,
+                  q->d_state};
   for (void *x : ptrs)
     if (x) (void)hipFree(x);
   delete q;
