@@ -384,22 +384,21 @@ struct symamd_ilu0_s {
   int *d_pa = nullptr, *d_pb = nullptr, *d_dpos = nullptr;
 };
 
-// Supernodal (BCSC) solve plan (supernodal.hip): the reference's supernode
-// arrays on the device, the rows' lists of temporaries, and per direction the
-// units, tickets and dependency lists; tags and state.
+// Supernodal (BCSC) solve plan (supernodal.hip): the rows' lists of
+// temporaries, and per direction the units, four slots to a ticket, and the
+// slots they wait for; tags and state.
 constexpr int SN_WMAX = 1024;         // widest supernode (its x in LDS)
 constexpr int SN_NARROW = 64;         // widest supernode one wavefront solves
 constexpr int SN_NARROW_ROWS = 128;   // rows below a narrow top its wavefront takes
+// a list longer than this is gathered by a workgroup ahead of its wide top
+constexpr int SN_GATHER_LONG = 48;
 struct symamd_snplan_s {
   int n = 0, m = 0, kcap = 1;  // kcap: columns d_T and d_flags hold
   int ntasks = 0;              // tops and 128-row chunks below (bounds the columns accepted)
-  int units = 0, tickets = 0, tunits = 0, ttickets = 0;
+  int tickets = 0, ttickets = 0;
   int64_t tcount = 0;
-  int *d_sup = nullptr, *d_nrows = nullptr, *d_Lp = nullptr, *d_tb = nullptr;
-  int *d_list = nullptr, *d_tdst = nullptr, *d_rowb = nullptr;
-  int *d_unit = nullptr, *d_tick = nullptr, *d_dptr = nullptr, *d_dlist = nullptr;
-  int *d_tunit = nullptr, *d_ttick = nullptr, *d_tdptr = nullptr, *d_tdlist = nullptr;
-  int *d_tbelow = nullptr;     // transposed: first column-group unit per supernode
+  int *d_tdst = nullptr, *d_rowb = nullptr, *d_list = nullptr;
+  int *d_unit = nullptr, *d_dlist = nullptr, *d_tunit = nullptr, *d_tdlist = nullptr;
   double *d_T = nullptr;
   int *d_flags = nullptr, *d_state = nullptr;
 };

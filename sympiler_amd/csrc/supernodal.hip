@@ -30,16 +30,20 @@
 // is one contiguous run.
 //
 // What bounds it: the chain of tree levels -- for each, the widest top's
-// columns (a division, a broadcast and a multiply-subtract each, about 75 ns)
-// plus the hand-offs -- for one right-hand side and the last levels of a
-// block.  A top's rows lie one per lane, 64 to a wave, and each wave streams
-// its rows' entries with SN_AHEAD column blocks in flight; the wave whose
-// rows are next solves its 64 columns with lane broadcasts and hands x on
-// through LDS, block of 8 by block of 8, while the other waves subtract.
+// columns (about 70 clocks each: two Newton steps for the quotient, a
+// broadcast, a multiply and a subtract) and the hand-offs -- for one
+// right-hand side and the last levels of a block.  A top's rows lie one per
+// lane, 64 to a wave, and each wave streams its rows' entries with SN_AHEAD
+// column blocks in flight; the wave whose rows are next solves its 64 columns
+// with lane broadcasts and hands x on through LDS, block of 8 by block of 8,
+// while the other waves subtract.  Long lists of temporaries are gathered by
+// workgroups of their own ahead of the top.
 // Measured on the 13-level nested-dissection-shaped factor (8,191 supernodes
-// up to 512 wide, 36 M values), forward and transposed: one right-hand side
-// 4.35 ms with one wavefront per top -> 1.07 ms, 32 right-hand sides 11.6 ->
-// 3.22 ms.
+// up to 512 wide, 36 M values), forward + transposed, in ms: one right-hand
+// side 1.36 + 3.06 with one wavefront per top, 0.45 + 0.65 with a workgroup,
+// 0.32 + 0.44 with the quotients from reciprocals, the whole diagonal block
+// in flight, gathered lists and turned tiles; 32 right-hand sides 4.6 + 6.9,
+// 1.71 + 1.50, 1.34 + 1.30.
 #include <algorithm>
 #include <vector>
 
@@ -49,23 +53,32 @@ namespace symamd {
 
 namespace {
 
-constexpr int SN_AHEAD = 4;  // column blocks of 8 whose entries are in flight
+// Column blocks of 8 whose entries are in flight: a wave's own 64 columns,
+// whose chain (about 20 ns a column) runs ahead of any load issued during it.
+constexpr int SN_AHEAD = 8;
+
+// One unit, read in one scalar load: the supernode's first column, width and
+// block rows, its values at Lx[p], its rows below at tdst / rowb[tb], and the
+// slots it waits for, dlist[d0 .. d0 + dn).  kind: SN_NARROW_UNIT, SN_TOP, or
+// first row below / column group of a chunk, or SN_GATHER_UNIT - row group.  A
+// top whose row groups are gathered, and a transposed top, waits for the slots
+// d0 + 4g of its groups (dn < 0).  w = 0: no unit.
+struct SnUnit {
+  int s, w, nr, kind, p, tb, d0, dn;
+};
+constexpr int SN_GATHER_UNIT = -3, SN_NARROW_UNIT = -2, SN_TOP = -1;
 
 struct SnArgs {
-  const int *sup, *nrows, *Lp;  // the reference's supernode arrays
+  const SnUnit *unit;           // slots 4t .. 4t+3: the units of ticket t
   const double *Lx;
   double *x;                    // right-hand side in, solution out
   double *T;                    // temporaries, placed where the rows' lists are read
-  const int *tb;                // supernode i's rows below start at tb[i]
   const int *tdst;              // place in T of each row below
   const int4 *list;             // row r subtracts T[x + j*z], j < y
-  const int2 *unit;             // unit u: (supernode, 0 = top or c = chunk c - 1 below)
-  const int *tick;              // ticket t runs units tick[t] .. tick[t+1]
-  const int *dptr, *dlist;      // units that unit u waits for
-  int *flags, *state;           // one tag per (column tile, unit)
-  int nunits, ntick, total_waves;
-  const int *rowb;              // transposed: rows below (at tb)
-  const int *tbelow;            // transposed: first column-group unit of a supernode, or -1
+  const int *dlist;             // slots that a unit waits for
+  int *flags, *state;           // one tag per (column tile, slot)
+  int ntick, total_waves;
+  const int *rowb;              // transposed: rows below
   int k, tiles;                 // right-hand sides: column c at x + c*ldx; tiles of KT
   int64_t ldx, tcount;          // column c's temporaries at T + c*tcount
   uint64_t timeout;
@@ -95,9 +108,11 @@ struct Cols {
   }
 };
 
-// The values are computed here: without it the compiler moves a block's
-// subtractions past the wait for the next block, and keeps their operands in
-// registers (and then in scratch memory) until there.
+// The values are computed (and loads they come from waited for) here.  After
+// a block's subtractions: the compiler would move them past the wait for the
+// next block and keep their operands in registers until there.  Before a loop
+// that loads ahead: a load that may still be pending on its entry makes every
+// round wait for all of its loads.
 template <int KT>
 __device__ __forceinline__ void hold(double (&v)[KT]) {
 #pragma unroll
@@ -139,10 +154,9 @@ __device__ __forceinline__ void wait_flag(const int *f, int target, int *state,
 // One lane per row: v minus the row's temporaries, in list order, GB entries
 // per round with the next round's loads in flight.  Entries past the row's
 // list are its last one (or T's first), not used.
-template <int KT>
+template <int KT, int GB>
 __device__ __forceinline__ void gather_list(double (&v)[KT], const double *T, int64_t tcount,
                                             const int4 &l) {
-  constexpr int GB = 16 / KT;
   double ta[GB][KT], tb[GB][KT];
   auto load = [&](double (&t)[GB][KT], int j) {
 #pragma unroll
@@ -187,25 +201,28 @@ __device__ __forceinline__ void load_cols(double (&m)[8], const double *M, int r
 }
 
 // A row's diagonal and its correctly rounded reciprocal, for quotients off
-// the IEEE division's long chain: with y = RN(1/d), one Newton step on a * y
+// the IEEE division's longer chain: with y = RN(1/d), one Newton step on a * y
 // gives a quotient within one unit in the last place, and a second with its
 // exact remainder the correctly rounded one (Markstein, IBM J. Res. Dev. 34,
-// 1990), as long as no step leaves the normal range.  `usable` says so for
-// the diagonal, in_range() for a dividend; otherwise the division is done.
+// 1990), as long as no step leaves the normal range.  usable says so for the
+// diagonal, in_range() of the quotient for the rest (a zero, infinite, tiny or
+// huge dividend leaves a quotient out of its range); otherwise the division
+// is done.
 struct Diag {
   double d, y;
   bool usable;
-  __device__ __forceinline__ explicit Diag(double v) : d(v), y(1.0 / v), usable(in_range(v, 100)) {}
+  __device__ __forceinline__ explicit Diag(double v) : d(v), y(1.0 / v), usable(in_range(v, 100)) {
+    asm volatile("" : "+v"(d), "+v"(y));
+  }
   // 2^-e <= |v| < 2^e
   static __device__ __forceinline__ bool in_range(double v, int e) {
     const unsigned hi = (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) & 0x7fffffffu;
     return hi - ((unsigned)(1023 - e) << 20) < ((unsigned)(2 * e) << 20);
   }
-  __device__ __forceinline__ double divide(double a) const {
-    const double q0 = a * y;
-    const double q1 = __builtin_fma(__builtin_fma(-d, q0, a), y, q0);
-    return __builtin_fma(__builtin_fma(-d, q1, a), y, q1);
+  __device__ __forceinline__ double step(double a, double q) const {
+    return __builtin_fma(__builtin_fma(-d, q, a), y, q);
   }
+  __device__ __forceinline__ double divide(double a) const { return step(a, step(a, a * y)); }
 };
 
 // Eight columns of a wave's own diagonal, lanes lb .. lb + B - 1 their rows
@@ -219,12 +236,9 @@ template <int KT, bool TRANS, typename Entry>
 __device__ __forceinline__ void solve_block(double (&acc)[KT], double (&res)[KT],
                                             const double (&m)[8], const Diag &dg, int lb, int B,
                                             int lane, Entry entry) {
-  double start[KT], num[KT];
+  double start[KT];
 #pragma unroll
-  for (int c = 0; c < KT; ++c) {
-    start[c] = acc[c];
-    num[c] = 1.0;
-  }
+  for (int c = 0; c < KT; ++c) start[c] = acc[c];
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
     const int j = TRANS ? 7 - t : t;
@@ -232,7 +246,6 @@ __device__ __forceinline__ void solve_block(double (&acc)[KT], double (&res)[KT]
     double q[KT];
 #pragma unroll
     for (int c = 0; c < KT; ++c) {
-      num[c] = lane == lb + j ? acc[c] : num[c];
       q[c] = dg.divide(acc[c]);
       res[c] = lane == lb + j ? q[c] : res[c];
     }
@@ -241,7 +254,7 @@ __device__ __forceinline__ void solve_block(double (&acc)[KT], double (&res)[KT]
   }
   bool ok = dg.usable;
 #pragma unroll
-  for (int c = 0; c < KT; ++c) ok = ok && Diag::in_range(num[c], 900);
+  for (int c = 0; c < KT; ++c) ok = ok && Diag::in_range(res[c], 790);
   if (__any(lane >= lb && lane < lb + min(B, 8) && !ok)) {
 #pragma unroll
     for (int c = 0; c < KT; ++c) acc[c] = start[c];
@@ -259,49 +272,63 @@ __device__ __forceinline__ void solve_block(double (&acc)[KT], double (&res)[KT]
   }
 }
 
-// A wave's own n <= 64 columns from column c0, the first SN_AHEAD blocks in
-// buf; done(lb, B) after each block.  Rounds of SN_AHEAD full blocks take no
-// branch, so the waits for their loads stay exact.
-template <int KT, typename Done>
-__device__ __forceinline__ void own_columns(double (&acc)[KT], double (&res)[KT],
-                                            double (&buf)[SN_AHEAD][8], const Diag &dg, int c0,
-                                            int n, const double *M, int row, int w, int nr,
-                                            int lane, Done done) {
-  auto block = [&](int b, const double (&m)[8]) {
-    const int B = min(8, n - 8 * b);
-    solve_block<KT, false>(acc, res, m, dg, 8 * b, B, lane, [&](int j) {
-      return at(M + (int64_t)(c0 + 8 * b + j) * nr, row);
-    });
-    done(8 * b, B);
-  };
-  int b = 0;
-  for (; 8 * (b + SN_AHEAD) <= n; b += SN_AHEAD) {
+// The last B < 8 columns of a row below: a block of four where four are left,
+// then single columns.
+template <int KT>
+__device__ __forceinline__ void last_columns(double &t, const double *x, const double (&m)[8],
+                                             int B) {
+  if (B >= 4) {
+    double sum = x[0] * m[0];
 #pragma unroll
-    for (int q = 0; q < SN_AHEAD; ++q) {
-      block(b + q, buf[q]);
-      load_cols(buf[q], M, row, c0 + 8 * (b + q + SN_AHEAD), w, nr);
-    }
+    for (int j = 1; j < 4; ++j) sum = sum + x[j * KT] * m[j];
+    t = t + sum;
   }
 #pragma unroll
-  for (int q = 0; q < SN_AHEAD; ++q)
-    if (8 * (b + q) < n) block(b + q, buf[q]);
+  for (int j = 0; j < 7; ++j)
+    if (j >= (B & 4) && j < B) t = t + x[j * KT] * m[j];
+}
+
+// A wave's own n <= 64 columns from column c0, in buf; done(lb, B) after each
+// block.
+template <int KT, typename Done>
+__device__ __forceinline__ void own_columns(double (&acc)[KT], double (&res)[KT],
+                                            const double (&buf)[SN_AHEAD][8], const Diag &dg,
+                                            int c0, int n, const double *M, int row, int nr,
+                                            int lane, Done done) {
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const int B = min(8, n - 8 * b);
+    if (B > 0) {
+      solve_block<KT, false>(acc, res, buf[b], dg, 8 * b, B, lane, [&](int j) {
+        return at(M + (int64_t)(c0 + 8 * b + j) * nr, row);
+      });
+      done(8 * b, B);
+    }
+  }
 }
 
 // Rows 64g .. 64g+63 of a wide top, by one wave.  `buf` holds the first
 // SN_AHEAD column blocks of the wave's rows.
 template <int KT>
 __device__ __forceinline__ void top_group(const SnArgs &a, const Cols<KT> &col, const double *T,
-                                          double (&buf)[SN_AHEAD][8], const Diag &dg, int g,
-                                          int s, int w, int nr, const double *M, double *xs,
+                                          double (&buf)[SN_AHEAD][8], const Diag &dg,
+                                          const int4 &list, const int *gathered, int target,
+                                          int g, int s, int w, int nr, const double *M, double *xs,
                                           int *prog, int &seen, int lane) {
   const int row = min(64 * g + lane, w - 1);
   double acc[KT], res[KT];
 #pragma unroll
-  for (int c = 0; c < KT; ++c) {
-    acc[c] = col.x[c][s + row];
-    res[c] = 0.0;
+  for (int c = 0; c < KT; ++c) res[c] = 0.0;
+  if (gathered) {
+    wait_flag(gathered, target, a.state, a.timeout);
+#pragma unroll
+    for (int c = 0; c < KT; ++c) acc[c] = ld_dev(&col.x[c][s + row]);
+  } else {
+#pragma unroll
+    for (int c = 0; c < KT; ++c) acc[c] = col.x[c][s + row];
+    gather_list<KT, 16 / KT>(acc, T, a.tcount, list);
   }
-  gather_list<KT>(acc, T, a.tcount, a.list[s + row]);
+  hold<KT>(acc);
   // columns of earlier groups: x from LDS as it is solved
   for (int b0 = 0; b0 < 8 * g; b0 += SN_AHEAD) {
 #pragma unroll
@@ -323,12 +350,12 @@ __device__ __forceinline__ void top_group(const SnArgs &a, const Cols<KT> &col, 
     }
   }
   // the group's own columns
-  own_columns<KT>(acc, res, buf, dg, 64 * g, min(64, w - 64 * g), M, row, w, nr, lane,
+  own_columns<KT>(acc, res, buf, dg, 64 * g, min(64, w - 64 * g), M, row, nr, lane,
                   [&](int lb, int B) {
-                    if (lane >= lb && lane < lb + B) {
+                    // every lane stores: solved rows their x again, the
+                    // others what no wave reads before their own block's count
 #pragma unroll
-                      for (int c = 0; c < KT; ++c) xs[(64 * g + lane) * KT + c] = res[c];
-                    }
+                    for (int c = 0; c < KT; ++c) xs[(64 * g + lane) * KT + c] = res[c];
                     lds_publish(prog, 64 * g + lb + B, lane);
                   });
 #pragma unroll
@@ -337,29 +364,45 @@ __device__ __forceinline__ void top_group(const SnArgs &a, const Cols<KT> &col, 
 }
 
 // A narrow supernode (w <= SN_NARROW) by one wave: the top, then the first
-// SN_NARROW_ROWS rows below, two per lane; xs is the wave's LDS.
+// SN_NARROW_ROWS rows below, a lane per row; xs is the wave's LDS.  The first
+// blocks of the rows below are loaded before the wait too.
 template <int KT>
 __device__ __forceinline__ void narrow_unit(const SnArgs &a, const Cols<KT> &col, double *T,
-                                            int u, int tile, int i, int target, double *xs,
-                                            int lane) {
-  const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i];
-  const double *M = a.Lx + a.Lp[i];
+                                            const SnUnit &n, int *flags, int slot, int target,
+                                            double *xs, int lane) {
+  constexpr int LA = 2;  // blocks of the rows below in flight
+  const int s = n.s, w = n.w, nr = n.nr;
+  const double *M = a.Lx + n.p;
   const int row = min(lane, w - 1);
   double buf[SN_AHEAD][8];
 #pragma unroll
   for (int q = 0; q < SN_AHEAD; ++q) load_cols(buf[q], M, row, 8 * q, w, nr);
-  const Diag dg(M[row + (int64_t)row * nr]);
+  const int4 list = a.list[s + row];
+  // the rows below: item it is block it % nb of the lane's row of half it / nb
+  const int below = min(nr - w, SN_NARROW_ROWS), nb = (w + 7) >> 3;
+  const int items = ((below + 63) >> 6) * nb;
+  double low[LA][8];
+  auto load_item = [&](double (&m)[8], int it) {
+    const int h = it >= nb ? 1 : 0;
+    load_cols(m, M, w + max(min(64 * h + lane, below - 1), -1), 8 * (it - h * nb), w, nr);
+  };
+#pragma unroll
+  for (int q = 0; q < LA; ++q) load_item(low[q], q);
+  int place[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    place[h] = below > 0 ? a.tdst[n.tb + min(64 * h + lane, below - 1)] : 0;
   double acc[KT], res[KT];
 #pragma unroll
   for (int c = 0; c < KT; ++c) {
     acc[c] = col.x[c][s + row];
     res[c] = 0.0;
   }
-  const int4 list = a.list[s + row];
-  int *const flags = a.flags + (int64_t)tile * a.nunits;
-  wait_units(a.dptr, a.dlist, u, flags, target, a.state, a.timeout);
-  gather_list<KT>(acc, T, a.tcount, list);
-  own_columns<KT>(acc, res, buf, dg, 0, w, M, row, w, nr, lane, [](int, int) {});
+  const Diag dg(at(M + (int64_t)row * nr, row));
+  wait_list(a.dlist + n.d0, n.dn, flags, target, a.state, a.timeout);
+  gather_list<KT, 8 / KT>(acc, T, a.tcount, list);
+  hold<KT>(acc);
+  own_columns<KT>(acc, res, buf, dg, 0, w, M, row, nr, lane, [](int, int) {});
   if (lane < w) {
 #pragma unroll
     for (int c = 0; c < KT; ++c) {
@@ -368,50 +411,40 @@ __device__ __forceinline__ void narrow_unit(const SnArgs &a, const Cols<KT> &col
     }
   }
   wave_lds_sync();
-  const int below = min(nr - w, SN_NARROW_ROWS);
-  for (int r0 = 0; r0 < below; r0 += 64) {
-    const int k = w + min(r0 + lane, below - 1);
-    double t[KT];
+  double t[KT];
 #pragma unroll
-    for (int c = 0; c < KT; ++c) t[c] = 0.0;
-    int cb = 0;
-    // two blocks' entries in flight, one where their x fill the registers
-    constexpr int NB = KT < 4 ? 2 : 1;
-    for (; w - cb >= 8 * NB; cb += 8 * NB) {
-      double m[NB][8];
+  for (int c = 0; c < KT; ++c) t[c] = 0.0;
+  for (int i0 = 0; i0 < items; i0 += LA) {
 #pragma unroll
-      for (int h = 0; h < NB; ++h) load_cols(m[h], M, k, cb + 8 * h, w, nr);
+    for (int q = 0; q < LA; ++q) {
+      const int it = i0 + q;
+      if (it < items) {
+        const int h = it >= nb ? 1 : 0, cb = 8 * (it - h * nb);
+        if (w - cb >= 8) {
 #pragma unroll
-      for (int h = 0; h < NB; ++h)
+          for (int c = 0; c < KT; ++c) {
+            double sum = xs[cb * KT + c] * low[q][0];
 #pragma unroll
-        for (int c = 0; c < KT; ++c) {
-          double sum = xs[(cb + 8 * h) * KT + c] * m[h][0];
+            for (int j = 1; j < 8; ++j) sum = sum + xs[(cb + j) * KT + c] * low[q][j];
+            t[c] = t[c] + sum;
+          }
+        } else {
 #pragma unroll
-          for (int j = 1; j < 8; ++j) sum = sum + xs[(cb + 8 * h + j) * KT + c] * m[h][j];
-          t[c] = t[c] + sum;
+          for (int c = 0; c < KT; ++c) last_columns<KT>(t[c], xs + cb * KT + c, low[q], w - cb);
         }
-    }
-    for (int B; cb < w; cb += B) {
-      B = w - cb >= 8 ? 8 : w - cb >= 4 ? 4 : 1;
-      double m[8];
-      load_cols(m, M, k, cb, w, nr);
+        if (cb + 8 >= w) {
 #pragma unroll
-      for (int c = 0; c < KT; ++c) {
-        double sum = xs[cb * KT + c] * m[0];
-#pragma unroll
-        for (int j = 1; j < 8; ++j)
-          if (j < B) sum = sum + xs[(cb + j) * KT + c] * m[j];
-        t[c] = t[c] + sum;
+          for (int c = 0; c < KT; ++c) {
+            if (64 * h + lane < below) st_dev(&T[place[h] + c * a.tcount], t[c]);
+            t[c] = 0.0;
+          }
+        }
       }
-    }
-    if (r0 + lane < below) {
-      const int64_t p = a.tdst[a.tb[i] + r0 + lane];
-#pragma unroll
-      for (int c = 0; c < KT; ++c) st_dev(&T[p + c * a.tcount], t[c]);
+      load_item(low[q], min(it + LA, 2 * nb - 1));
     }
   }
   publish_fence();
-  if (lane == 0) st_dev(&flags[u], target);
+  if (lane == 0) st_dev(&flags[slot], target);
   wave_lds_sync();
 }
 
@@ -421,22 +454,21 @@ __device__ __forceinline__ void narrow_unit(const SnArgs &a, const Cols<KT> &col
 // before the wait for the top.
 template <int KT>
 __device__ __forceinline__ void below_unit(const SnArgs &a, const Cols<KT> &col, double *T,
-                                           int u, int tile, int i, int first, int target,
+                                           const SnUnit &n, int *flags, int slot, int target,
                                            double *xs, double *sums) {
   constexpr int NBW = 8 / KT;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i];
-  const double *M = a.Lx + a.Lp[i];
+  const int s = n.s, w = n.w, nr = n.nr, first = n.kind;
+  const double *M = a.Lx + n.p;
   const int k = min(w + first + lane, nr - 1);
-  int *const flags = a.flags + (int64_t)tile * a.nunits;
   const int nb = w / 8;  // full blocks; then one of 4 where 4 are left, then single columns
   double m[NBW][8], tail[8];
 #pragma unroll
   for (int h = 0; h < NBW; ++h) load_cols(m[h], M, k, 8 * (wave * NBW + h), w, nr);
   load_cols(tail, M, k, 8 * nb, w, nr);
-  const int64_t place = a.tdst[a.tb[i] + k - w];
-  if (wave == 0) wait_units(a.dptr, a.dlist, u, flags, target, a.state, a.timeout);
+  const int64_t place = a.tdst[n.tb + k - w];
+  if (wave == 0) wait_list(a.dlist + n.d0, n.dn, flags, target, a.state, a.timeout);
   __syncthreads();
 #pragma unroll
   for (int c = 0; c < KT; ++c)
@@ -472,22 +504,79 @@ __device__ __forceinline__ void below_unit(const SnArgs &a, const Cols<KT> &col,
     half ^= 1;
   }
   if (wave < KT) {
-    int cb = 8 * nb, q = 0;
-    if (w - cb >= 4) {
-      double sum = xs[cb * KT + wave] * tail[0];
-#pragma unroll
-      for (int j = 1; j < 4; ++j) sum = sum + xs[(cb + j) * KT + wave] * tail[j];
-      t = t + sum;
-      q = 4;
-    }
-#pragma unroll
-    for (int j = 0; j < 7; ++j)
-      if (j >= q && cb + j < w) t = t + xs[(cb + j) * KT + wave] * tail[j];
+    const int cb = 8 * nb;
+    last_columns<KT>(t, xs + cb * KT + wave, tail, w - cb);
     if (w + first + lane < nr) st_dev(&T[place + wave * a.tcount], t);
     publish_fence();
   }
   __syncthreads();
-  if (threadIdx.x == 0) st_dev(&flags[u], target);
+  if (threadIdx.x == 0) st_dev(&flags[slot], target);
+}
+
+// x of rows 64g .. 64g+63 of a wide top minus their temporaries, by the
+// workgroup: rounds of 64 / KT list entries, a quarter of them loaded by each
+// wave with the next round's in flight, turned over in LDS to wave c, which
+// subtracts right-hand side c's in list order.  For tops of long lists: one
+// wave per 64 rows took 19 us for the 512 rows of about 200 entries at the
+// root of the 13-level factor, twice, before and during the solve.
+template <int KT>
+__device__ __forceinline__ void gather_unit(const SnArgs &a, const double *T, const SnUnit &n,
+                                            int tile, int *flags, int slot, int target,
+                                            double *stage) {
+  constexpr int EW = 16 / KT, E = 4 * EW;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = 64 * (SN_GATHER_UNIT - n.kind) + lane;
+  const int row = n.s + min(r, n.w - 1);
+  const int4 l = a.list[row];
+  const int cw = tile * KT + wave;
+  double *const xc = a.x + (int64_t)min(cw, a.k - 1) * a.ldx;
+  double v = xc[row];
+  int longest = l.y;
+  for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
+  longest = __builtin_amdgcn_readfirstlane(longest);
+  if (wave == 0) wait_list(a.dlist + n.d0, n.dn, flags, target, a.state, a.timeout);
+  __syncthreads();
+  double ta[EW][KT], tb[EW][KT];
+  auto load = [&](double (&t)[EW][KT], int j0) {
+#pragma unroll
+    for (int u = 0; u < EW; ++u) {
+      const double *p = T + (l.x + (int64_t)max(min(j0 + wave * EW + u, l.y - 1), 0) * l.z);
+#pragma unroll
+      for (int q = 0; q < KT; ++q) t[u][q] = ld_dev(p + q * a.tcount);
+    }
+  };
+  auto round = [&](double (&t)[EW][KT], int j0) {
+    __syncthreads();  // the round before is read
+#pragma unroll
+    for (int u = 0; u < EW; ++u)
+#pragma unroll
+      for (int q = 0; q < KT; ++q) stage[((wave * EW + u) * KT + q) * 64 + lane] = t[u][q];
+    load(t, j0 + 2 * E);
+    __syncthreads();
+    if (wave < KT) {
+      const int cnt = min(E, longest - j0);
+      for (int e = 0; e < cnt; e += 8) {
+        double p[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) p[u] = stage[(min(e + u, E - 1) * KT + wave) * 64 + lane];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v = j0 + e + u < min(l.y, j0 + E) ? v - p[u] : v;
+      }
+    }
+  };
+  load(ta, 0);
+  load(tb, E);
+  for (int j0 = 0; j0 < longest; j0 += 2 * E) {
+    round(ta, j0);
+    if (j0 + E < longest) round(tb, j0 + E);
+  }
+  if (wave < KT) {
+    if (r < n.w && cw < a.k) st_dev(&xc[row], v);
+    publish_fence();
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) st_dev(&flags[slot], target);
 }
 
 // Workgroup's next (ticket, column tile), ticket-major; -1 past the last.
@@ -516,39 +605,39 @@ __global__ __launch_bounds__(256, 2) void k_supernodal(SnArgs a) {
     const int tk = tt / a.tiles, tile = tt - tk * a.tiles;
     const Cols<KT> col(a, tile);
     double *const T = a.T + (int64_t)tile * a.tcount * KT;
-    const int u0 = a.tick[tk], u1 = a.tick[tk + 1];
-    const int2 un = a.unit[u0];
-    const int i = __builtin_amdgcn_readfirstlane(un.x);
-    const int chunk = __builtin_amdgcn_readfirstlane(un.y);
-    const int w = a.sup[i + 1] - a.sup[i];
-    if (chunk > 0) {
-      const int first = (w <= SN_NARROW ? SN_NARROW_ROWS : 0) + (chunk - 1) * 64;
-      below_unit<KT>(a, col, T, u0, tile, i, first, target, xs, sums);
-    } else if (w <= SN_NARROW) {
-      if (u0 + wave < u1) {
-        const int node = __builtin_amdgcn_readfirstlane(a.unit[u0 + wave].x);
-        narrow_unit<KT>(a, col, T, u0 + wave, tile, node, target, xs + wave * 64 * KT, lane);
-      }
+    int *const flags = a.flags + (int64_t)tile * a.ntick * 4;
+    const SnUnit n = a.unit[4 * tk];
+    if (n.kind >= 0) {
+      below_unit<KT>(a, col, T, n, flags, 4 * tk, target, xs, sums);
+    } else if (n.kind <= SN_GATHER_UNIT) {
+      gather_unit<KT>(a, T, n, tile, flags, 4 * tk, target, sums);
+    } else if (n.kind == SN_NARROW_UNIT) {
+      const SnUnit m = a.unit[4 * tk + wave];
+      if (m.w > 0)
+        narrow_unit<KT>(a, col, T, m, flags, 4 * tk + wave, target, xs + wave * 64 * KT, lane);
     } else {
-      const int s = a.sup[i], nr = a.nrows[i];
-      const double *M = a.Lx + a.Lp[i];
-      int *const flags = a.flags + (int64_t)tile * a.nunits;
+      const int w = n.w, nr = n.nr;
+      const double *M = a.Lx + n.p;
       int seen = 0;
       for (int g = wave; g < 4 || 64 * g < w; g += 4) {
         const int row = min(64 * g + lane, w - 1);
         double buf[SN_AHEAD][8];
 #pragma unroll
         for (int q = 0; q < SN_AHEAD; ++q) load_cols(buf[q], M, row, 8 * q, w, nr);
-        const Diag dg(M[row + (int64_t)row * nr]);
+        const int4 list = a.list[n.s + row];
+        const Diag dg(at(M + (int64_t)row * nr, row));
         if (g < 4) {  // each wave's first group: the entries are on their way
-          if (wave == 0) wait_units(a.dptr, a.dlist, u0, flags, target, a.state, a.timeout);
+          if (wave == 0 && n.dn > 0)
+            wait_list(a.dlist + n.d0, n.dn, flags, target, a.state, a.timeout);
           __syncthreads();
         }
-        if (64 * g < w) top_group<KT>(a, col, T, buf, dg, g, s, w, nr, M, xs, &slot[1], seen, lane);
+        if (64 * g < w)
+          top_group<KT>(a, col, T, buf, dg, list, n.dn < 0 ? &flags[n.d0 + 4 * g] : nullptr,
+                        target, g, n.s, w, nr, M, xs, &slot[1], seen, lane);
       }
       publish_fence();
       __syncthreads();
-      if (threadIdx.x == 0) st_dev(&flags[u0], target);
+      if (threadIdx.x == 0) st_dev(&flags[4 * tk], target);
     }
   }
   persistent_finish(a.state, a.total_waves);
@@ -565,268 +654,312 @@ __global__ __launch_bounds__(256, 2) void k_supernodal(SnArgs a) {
 //
 // A narrow supernode with at most SN_NARROW_ROWS rows below is one wave's
 // work, four to a ticket.  Otherwise 64 of its columns' sums over the rows
-// below are a ticket (the workgroup: tiles of 64 x 64 entries are loaded
-// along the rows, coalesced, and turned in LDS so that a lane then owns a
-// column), and its top another (waves take groups of 64 columns from the
-// last one, hand x on through LDS as in the forward solve, and wait for
-// their own group's sums only).
+// below are a ticket (the workgroup), and its top another: waves take groups
+// of 64 columns from the last one, hand x on through LDS as in the forward
+// solve, and wait for their own group's sums only.
+//
+// A lane owns a column, and a column's entries are contiguous: reading them
+// lane by lane touches 64 cache lines per load.  So entries are loaded along
+// the rows and turned in LDS.
 
-// Rows r0 .. r0+7 of one column's entries (lane = column; the pointer is at
-// its row 0); rows past `last` repeat it.
-__device__ __forceinline__ void load_rows(double (&m)[8], const double *C, int r0, int last) {
-  if (r0 + 7 <= last) {
+constexpr int SN_ROWS_T = 16;            // rows of a turned block
+constexpr int SN_PITCH_T = SN_ROWS_T + 1;
+
+// Rows r0 .. r0+15 of columns c0 .. c0+63: four columns per load, lane l row
+// l & 15 of column 4j + l / 16.  Clamped to the block's last row and the
+// top's last column.
+__device__ __forceinline__ void load_turn(double (&m)[16], const double *M, int r0, int c0,
+                                          int w, int nr, int lane) {
+  const double *R = M + min(r0 + (lane & 15), nr - 1);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) m[j] = C[r0 + j];
-  } else {
+  for (int j = 0; j < 16; ++j) m[j] = R[(int64_t)min(c0 + 4 * j + (lane >> 4), w - 1) * nr];
+}
+
+// The block turned: v[r] = row r of the lane's column.  tile: the wave's LDS.
+__device__ __forceinline__ void turn(double (&v)[16], const double (&m)[16], double *tile,
+                                     int lane) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) m[j] = C[max(min(r0 + j, last), 0)];
+  for (int j = 0; j < 16; ++j) tile[(4 * j + (lane >> 4)) * SN_PITCH_T + (lane & 15)] = m[j];
+  wave_lds_sync();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) v[r] = tile[lane * SN_PITCH_T + r];
+  wave_lds_sync();
+}
+
+// Eight rows c0 .. c0+7 of a wave's own columns (lanes lb .. lb+7).
+template <int KT, typename Done>
+__device__ __forceinline__ void own_rows(double (&acc)[KT], double (&res)[KT],
+                                         const double (&m)[8], const Diag &dg, int c0, int lb,
+                                         int w, const double *C, int lane, Done done) {
+  if (c0 < w) {
+    solve_block<KT, true>(acc, res, m, dg, lb, w - c0, lane, [&](int j) { return C[c0 + j]; });
+    done();
   }
 }
 
-// Columns 64g .. 64g+63 of a top, by one wave: x from LDS for the columns of
-// later groups (xs and the count are not used by a narrow supernode, whose
-// only group is the last).
+// Columns 64g .. 64g+63 of a top, by one wave, from its last row: x from LDS
+// for the columns of later groups (a narrow supernode, with one group, passes
+// no xs).  m: the first two blocks of 16 rows, from the last.
 template <int KT>
 __device__ __forceinline__ void top_group_t(double (&acc)[KT], double (&res)[KT],
-                                            double (&buf)[SN_AHEAD][8], const Diag &dg, int g,
-                                            int w, int nr, const double *M, double *xs,
+                                            double (&m)[2][16], const Diag &dg, int g, int w,
+                                            int nr, const double *M, double *tile, double *xs,
                                             int *prog, int &seen, int lane) {
   const double *C = M + (int64_t)min(64 * g + lane, w - 1) * nr;
-  const int top = (w - 1) / 8;  // last block of eight rows
 #pragma unroll
   for (int c = 0; c < KT; ++c) res[c] = 0.0;
-  int b = top;
-  auto later = [&](double (&m)[8]) {
-    const int c0 = 8 * b, B = min(8, w - c0);
-    lds_wait(prog, w - c0, seen);
-    double xv[8][KT];
+  hold<KT>(acc);
+  const int last = (w - 1) >> 4;
+  for (int b0 = last; b0 >= 4 * g; b0 -= 2) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int q = 0; q < 2; ++q) {
+      const int b = b0 - q;
+      if (b >= 4 * g) {
+        double v[16];
+        turn(v, m[q], tile, lane);
+        load_turn(m[q], M, max(16 * (b - 2), 0), 64 * g, w, nr, lane);
 #pragma unroll
-      for (int c = 0; c < KT; ++c) xv[j][c] = xs[min(c0 + j, w - 1) * KT + c];
+        for (int h = 1; h >= 0; --h) {
+          const int c0 = 16 * b + 8 * h;
+          double v8[8];
 #pragma unroll
-    for (int j = 7; j >= 0; --j)
-      if (j < B) {
+          for (int j = 0; j < 8; ++j) v8[j] = v[8 * h + j];
+          if (b >= 4 * g + 4) {
+            if (c0 < w) {
+              lds_wait(prog, w - c0, seen);
+              double xv[8][KT];
 #pragma unroll
-        for (int c = 0; c < KT; ++c) acc[c] = acc[c] - m[j] * xv[j][c];
+              for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int c = 0; c < KT; ++c) xv[j][c] = xs[min(c0 + j, w - 1) * KT + c];
+#pragma unroll
+              for (int j = 7; j >= 0; --j)
+                if (c0 + j < w) {
+#pragma unroll
+                  for (int c = 0; c < KT; ++c) acc[c] = acc[c] - v8[j] * xv[j][c];
+                }
+              hold<KT>(acc);
+            }
+          } else {
+            const int lb = c0 - 64 * g;
+            own_rows<KT>(acc, res, v8, dg, c0, lb, w, C, lane, [&] {
+              if (xs) {
+#pragma unroll
+                for (int c = 0; c < KT; ++c) xs[(64 * g + lane) * KT + c] = res[c];
+                lds_publish(prog, w - c0, lane);
+              }
+            });
+          }
+        }
       }
-    hold<KT>(acc);
-  };
-  auto own = [&](double (&m)[8]) {
-    const int c0 = 8 * b, lb = c0 - 64 * g;
-    solve_block<KT, true>(acc, res, m, dg, lb, w - c0, lane,
-                          [&](int j) { return C[c0 + j]; });
-    if (xs) {
-      if (lane >= lb && lane < lb + 8 && 64 * g + lane < w) {
-#pragma unroll
-        for (int c = 0; c < KT; ++c) xs[(64 * g + lane) * KT + c] = res[c];
-      }
-      lds_publish(prog, w - c0, lane);
-    }
-  };
-  // SN_AHEAD blocks per round, slot q of round n holding block top - 4n - q
-  for (int b0 = top; b0 >= 8 * g; b0 -= SN_AHEAD) {
-#pragma unroll
-    for (int q = 0; q < SN_AHEAD; ++q) {
-      b = b0 - q;
-      if (b >= 8 * g) {
-        if (b >= 8 * g + 8)
-          later(buf[q]);
-        else
-          own(buf[q]);
-      }
-      load_rows(buf[q], C, max(8 * (b - SN_AHEAD), 0), nr - 1);
     }
   }
-}
-
-__device__ __forceinline__ void preload_t(double (&buf)[SN_AHEAD][8], const double *M, int g,
-                                          int w, int nr, int lane) {
-  const double *C = M + (int64_t)min(64 * g + lane, w - 1) * nr;
-  const int top = (w - 1) / 8;
-#pragma unroll
-  for (int q = 0; q < SN_AHEAD; ++q) load_rows(buf[q], C, max(8 * (top - q), 0), nr - 1);
 }
 
 template <int KT>
-__device__ __forceinline__ void narrow_unit_t(const SnArgs &a, const Cols<KT> &col, int u,
-                                              int tile, int i, int target, int lane) {
-  const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i], below = nr - w;
-  const double *M = a.Lx + a.Lp[i];
-  const int *rows = a.rowb + a.tb[i];
+__device__ __forceinline__ void narrow_unit_t(const SnArgs &a, const Cols<KT> &col,
+                                              const SnUnit &n, int *flags, int slot, int target,
+                                              double *tile, int lane) {
+  const int s = n.s, w = n.w, nr = n.nr, below = nr - w;
+  const double *M = a.Lx + n.p;
+  const int *rows = a.rowb + n.tb;
   const int c = min(lane, w - 1);
-  double buf[SN_AHEAD][8];
-  preload_t(buf, M, 0, w, nr, lane);
+  // blocks of 16 rows below, ascending, then the top's from its last
+  const int nb = (below + 15) >> 4, last = (w - 1) >> 4;
+  auto first_row = [&](int it) { return it < nb ? w + 16 * it : max(16 * (last - (it - nb)), 0); };
+  double m[2][16];
+  load_turn(m[0], M, first_row(0), 0, w, nr, lane);
+  load_turn(m[1], M, first_row(1), 0, w, nr, lane);
+  double acc[KT], res[KT];
+#pragma unroll
+  for (int q = 0; q < KT; ++q) acc[q] = col.x[q][s + c];
   const Diag dg(M[c + (int64_t)c * nr]);
-  double acc[KT], res[KT], t[KT];
-#pragma unroll
-  for (int q = 0; q < KT; ++q) {
-    acc[q] = col.x[q][s + c];
-    t[q] = 0.0;
-  }
-  const double *C = M + (int64_t)c * nr + w;
-  int *const flags = a.flags + (int64_t)tile * a.nunits;
-  double ma[8], mb[8];
   if (below > 0) {
-    load_rows(ma, C, 0, below - 1);
-    wait_units(a.dptr, a.dlist, u, flags, target, a.state, a.timeout);
-    for (int r0 = 0; r0 < below; r0 += 64) {
-      double xr[KT];
-      const int row = rows[min(r0 + lane, below - 1)];
+    const int r0 = rows[min(lane, below - 1)], r1 = rows[min(64 + lane, below - 1)];
+    wait_list(a.dlist + n.d0, n.dn, flags, target, a.state, a.timeout);
+    double x0[KT], x1[KT], t[KT];
 #pragma unroll
-      for (int q = 0; q < KT; ++q) xr[q] = ld_dev(&col.x[q][row]);
-      auto add = [&](const double (&m)[8], int r) {
+    for (int q = 0; q < KT; ++q) {
+      x0[q] = ld_dev(&col.x[q][r0]);
+      x1[q] = ld_dev(&col.x[q][r1]);
+      t[q] = 0.0;
+    }
+    hold<KT>(x0);
+    hold<KT>(x1);
+    for (int i0 = 0; i0 < nb; i0 += 2) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (r + j < below) {
+      for (int u = 0; u < 2; ++u) {
+        const int it = i0 + u;
+        if (it < nb) {
+          double v[16];
+          turn(v, m[u], tile, lane);
+          load_turn(m[u], M, first_row(it + 2), 0, w, nr, lane);
+          if (it == 4) {
 #pragma unroll
-            for (int q = 0; q < KT; ++q) {
-              const double p = m[j] * lane_value(xr[q], (r + j) & 63);
-              t[q] = r + j == 0 ? p : t[q] + p;
-            }
+            for (int q = 0; q < KT; ++q) x0[q] = x1[q];
           }
-      };
-      const int end = min(r0 + 64, below);
-      for (int r = r0; r < end; r += 16) {
-        load_rows(mb, C, min(r + 8, below - 1), below - 1);
-        add(ma, r);
-        load_rows(ma, C, min(r + 16, below - 1), below - 1);
-        if (r + 8 < end) add(mb, r + 8);
+          const int cnt = below - 16 * it;
+#pragma unroll
+          for (int j = 0; j < 16; ++j)
+            if (j < cnt) {
+#pragma unroll
+              for (int q = 0; q < KT; ++q) {
+                const double p = v[j] * lane_value(x0[q], (16 * it + j) & 63);
+                t[q] = 16 * it + j == 0 ? p : t[q] + p;
+              }
+            }
+        }
       }
     }
 #pragma unroll
     for (int q = 0; q < KT; ++q) acc[q] = acc[q] - t[q];
+    if (nb & 1) {  // the top's first block is in m[1]
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const double d = m[0][j];
+        m[0][j] = m[1][j];
+        m[1][j] = d;
+      }
+    }
   }
   int seen = 0;
-  top_group_t<KT>(acc, res, buf, dg, 0, w, nr, M, nullptr, nullptr, seen, lane);
+  top_group_t<KT>(acc, res, m, dg, 0, w, nr, M, tile, nullptr, nullptr, seen, lane);
 #pragma unroll
   for (int q = 0; q < KT; ++q)
     if (lane < w && col.live[q]) st_dev(&col.x[q][s + lane], res[q]);
   publish_fence();
-  if (lane == 0) st_dev(&flags[u], target);
+  if (lane == 0) st_dev(&flags[slot], target);
 }
 
-constexpr int SN_PITCH = 65;  // doubles per column of a turned tile (no bank conflicts)
+constexpr int SN_PITCH = 65;   // doubles per column of a turned 64 x 64 tile
+constexpr int SN_TILES = 4;    // tiles of 64 rows below in flight
 
 // The sums over the rows below of columns 64g .. 64g+63, by the workgroup.
-// Tiles of 64 rows; wave v loads 16 columns of a tile along its rows, the
-// next tile's entries and x in flight while this one is summed; wave c then
-// adds right-hand side c's products, a lane per column.
+// Tiles of 64 rows; wave v loads 16 columns of a tile along its rows, four
+// tiles in flight, x at the rows of 256 at a time in LDS; wave c then adds
+// right-hand side c's products, a lane per column.
 template <int KT>
-__device__ __forceinline__ void below_unit_t(const SnArgs &a, int u, int tile, int i, int g,
-                                             int target, double *turn, double *xrow) {
+__device__ __forceinline__ void below_unit_t(const SnArgs &a, const Cols<KT> &col,
+                                             const SnUnit &n, int tile, int *flags, int slot,
+                                             int target, double *turned, double *xrow) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i], below = nr - w;
-  const double *M = a.Lx + a.Lp[i] + w;
-  const int *rows = a.rowb + a.tb[i];
-  int *const flags = a.flags + (int64_t)tile * a.nunits;
-  double m[16];
-  auto load = [&](int r0) {
+  const int s = n.s, w = n.w, nr = n.nr, below = nr - w, g = n.kind;
+  const double *M = a.Lx + n.p + w;
+  const int *rows = a.rowb + n.tb;
+  double m[SN_TILES][16];
+  auto load = [&](double (&d)[16], int r0) {
     const int r = min(r0 + lane, below - 1);
 #pragma unroll
     for (int j = 0; j < 16; ++j)
-      m[j] = at(M + (int64_t)min(64 * g + 16 * wave + j, w - 1) * nr, r);
+      d[j] = at(M + (int64_t)min(64 * g + 16 * wave + j, w - 1) * nr, r);
   };
-  load(0);
-  int row = rows[min(lane, below - 1)];
-  if (wave == 0) wait_units(a.dptr, a.dlist, u, flags, target, a.state, a.timeout);
+#pragma unroll
+  for (int q = 0; q < SN_TILES; ++q) load(m[q], 64 * q);
+  int row = rows[min((int)threadIdx.x, below - 1)];
+  if (wave == 0) wait_list(a.dlist + n.d0, n.dn, flags, target, a.state, a.timeout);
   __syncthreads();
-  // wave c of the first KT holds x of right-hand side c at the tile's rows
-  const int cw = tile * KT + wave;
-  double *const xc = a.x + (int64_t)min(cw, a.k - 1) * a.ldx;
-  const bool mine = cw < a.k;
-  double xr = wave < KT ? ld_dev(&xc[row]) : 0.0;
+  double xn[KT];
+#pragma unroll
+  for (int c = 0; c < KT; ++c) xn[c] = ld_dev(&col.x[c][row]);
+  row = rows[min(256 + (int)threadIdx.x, below - 1)];
   double t = 0.0;
   int half = 0;
-  for (int r0 = 0; r0 < below; r0 += 64) {
-    double *const tl = turn + half * 64 * SN_PITCH;
-    double *const xl = xrow + (half * KT + min(wave, KT - 1)) * 64;
+  for (int r0 = 0; r0 < below; r0 += 64 * SN_TILES) {
+    __syncthreads();  // the x of the rows before are read
 #pragma unroll
-    for (int j = 0; j < 16; ++j) tl[(16 * wave + j) * SN_PITCH + lane] = m[j];
-    if (wave < KT) xl[lane] = xr;
-    if (r0 + 64 < below) {
-      load(r0 + 64);
-      row = rows[min(r0 + 64 + lane, below - 1)];
-      if (wave < KT) xr = ld_dev(&xc[row]);
+    for (int c = 0; c < KT; ++c) xrow[c * 256 + threadIdx.x] = xn[c];
+    if (r0 + 256 < below) {
+#pragma unroll
+      for (int c = 0; c < KT; ++c) xn[c] = ld_dev(&col.x[c][row]);
+      row = rows[min(r0 + 512 + (int)threadIdx.x, below - 1)];
     }
-    __syncthreads();
-    if (wave < KT) {
-      const int cnt = min(64, below - r0);
-      int r = 0;
-      if (r0 == 0) {
-        t = tl[lane * SN_PITCH] * xl[0];
-        r = 1;
-      }
-      for (; r + 8 <= cnt; r += 8) {
-        double p[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) p[j] = tl[lane * SN_PITCH + r + j] * xl[r + j];
+    for (int q = 0; q < SN_TILES; ++q) {
+      const int r = r0 + 64 * q;
+      if (r < below) {
+        double *const tl = turned + half * 64 * SN_PITCH;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) t = t + p[j];
+        for (int j = 0; j < 16; ++j) tl[(16 * wave + j) * SN_PITCH + lane] = m[q][j];
+        load(m[q], r + 64 * SN_TILES);
+        __syncthreads();
+        if (wave < KT) {
+          const double *const xl = xrow + wave * 256 + 64 * q, *const ml = tl + lane * SN_PITCH;
+          const int cnt = min(64, below - r);
+          int i = 0;
+          if (r == 0) {
+            t = ml[0] * xl[0];
+            i = 1;
+          }
+          for (; i + 8 <= cnt; i += 8) {
+            double p[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) p[j] = ml[i + j] * xl[i + j];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) t = t + p[j];
+          }
+          for (; i < cnt; ++i) t = t + ml[i] * xl[i];
+        }
+        half ^= 1;
       }
-      for (; r < cnt; ++r) t = t + tl[lane * SN_PITCH + r] * xl[r];
     }
-    half ^= 1;
   }
   if (wave < KT) {
-    const int c = 64 * g + lane;
-    if (c < w && mine) st_dev(&xc[s + c], xc[s + c] - t);
+    const int c = 64 * g + lane, cw = tile * KT + wave;
+    double *const xc = a.x + (int64_t)min(cw, a.k - 1) * a.ldx;
+    if (c < w && cw < a.k) st_dev(&xc[s + c], xc[s + c] - t);
     publish_fence();
   }
   __syncthreads();
-  if (threadIdx.x == 0) st_dev(&flags[u], target);
+  if (threadIdx.x == 0) st_dev(&flags[slot], target);
 }
 
 template <int KT>
 __global__ __launch_bounds__(256, 2) void k_supernodal_t(SnArgs a) {
-  // a top's x, or two turned tiles and the x at their rows
-  constexpr int TILES = 2 * 64 * SN_PITCH + 2 * KT * 64;
-  __shared__ double mem[SN_WMAX * KT > TILES ? SN_WMAX * KT : TILES];
+  // a top's x and the waves' turned blocks, or two turned tiles and the x at
+  // their rows
+  constexpr int TOP = SN_WMAX * KT + 4 * 64 * SN_PITCH_T;
+  constexpr int TILES = 2 * 64 * SN_PITCH + 256 * KT;
+  __shared__ double mem[TOP > TILES ? TOP : TILES];
   __shared__ int slot[2];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int target = ld_dev(&a.state[ST_EPOCH]) + 1;
+  double *const mine = mem + SN_WMAX * KT + wave * 64 * SN_PITCH_T;
   for (;;) {
     const int tt = next_ticket(a, slot);
     if (tt < 0) break;
     const int tk = tt / a.tiles, tile = tt - tk * a.tiles;
     const Cols<KT> col(a, tile);
-    const int u0 = a.tick[tk], u1 = a.tick[tk + 1];
-    const int2 un = a.unit[u0];
-    const int i = __builtin_amdgcn_readfirstlane(un.x);
-    const int chunk = __builtin_amdgcn_readfirstlane(un.y);
-    const int s = a.sup[i], w = a.sup[i + 1] - s, nr = a.nrows[i];
-    int *const flags = a.flags + (int64_t)tile * a.nunits;
-    if (chunk > 0) {
-      below_unit_t<KT>(a, u0, tile, i, chunk - 1, target, mem, mem + 2 * 64 * SN_PITCH);
-    } else if (w <= SN_NARROW && nr - w <= SN_NARROW_ROWS) {
-      if (u0 + wave < u1) {
-        const int node = __builtin_amdgcn_readfirstlane(a.unit[u0 + wave].x);
-        narrow_unit_t<KT>(a, col, u0 + wave, tile, node, target, lane);
-      }
+    int *const flags = a.flags + (int64_t)tile * a.ntick * 4;
+    const SnUnit n = a.unit[4 * tk];
+    if (n.kind >= 0) {
+      below_unit_t<KT>(a, col, n, tile, flags, 4 * tk, target, mem, mem + 2 * 64 * SN_PITCH);
+    } else if (n.kind == SN_NARROW_UNIT) {
+      const SnUnit u = a.unit[4 * tk + wave];
+      if (u.w > 0) narrow_unit_t<KT>(a, col, u, flags, 4 * tk + wave, target, mine, lane);
     } else {
-      const double *M = a.Lx + a.Lp[i];
-      const int G = (w + 63) / 64, ub = a.tbelow[i];
+      const int w = n.w, nr = n.nr;
+      const double *M = a.Lx + n.p;
       int seen = 0;
-      for (int g = G - 1 - wave; g >= 0; g -= 4) {
-        double buf[SN_AHEAD][8];
-        preload_t(buf, M, g, w, nr, lane);
-        const int c = min(64 * g + lane, w - 1);
+      for (int g = (w + 63) / 64 - 1 - wave; g >= 0; g -= 4) {
+        const int last = (w - 1) >> 4, c = min(64 * g + lane, w - 1);
+        double m[2][16];
+        load_turn(m[0], M, 16 * last, 64 * g, w, nr, lane);
+        load_turn(m[1], M, max(16 * (last - 1), 0), 64 * g, w, nr, lane);
         const Diag dg(M[c + (int64_t)c * nr]);
-        if (ub >= 0)
-          wait_flag(&flags[ub + g], target, a.state, a.timeout);
+        if (n.dn < 0) wait_flag(&flags[n.d0 + 4 * g], target, a.state, a.timeout);
         double acc[KT], res[KT];
 #pragma unroll
-        for (int q = 0; q < KT; ++q) acc[q] = ld_dev(&col.x[q][s + c]);
-        top_group_t<KT>(acc, res, buf, dg, g, w, nr, M, mem, &slot[1], seen, lane);
+        for (int q = 0; q < KT; ++q) acc[q] = ld_dev(&col.x[q][n.s + c]);
+        top_group_t<KT>(acc, res, m, dg, g, w, nr, M, mine, mem, &slot[1], seen, lane);
 #pragma unroll
         for (int q = 0; q < KT; ++q)
-          if (64 * g + lane < w && col.live[q]) st_dev(&col.x[q][s + c], res[q]);
+          if (64 * g + lane < w && col.live[q]) st_dev(&col.x[q][n.s + c], res[q]);
       }
       publish_fence();
       __syncthreads();
-      if (threadIdx.x == 0) st_dev(&flags[u0], target);
+      if (threadIdx.x == 0) st_dev(&flags[4 * tk], target);
     }
   }
   persistent_finish(a.state, a.total_waves);
@@ -836,77 +969,82 @@ __global__ __launch_bounds__(256, 2) void k_supernodal_t(SnArgs a) {
 
 namespace {
 
-// Units and tickets of one direction, level by level.  Per level: the column
-// groups of the wide supernodes (transposed only; they come before the top
-// that uses them), the wide tops, the narrow supernodes four to a ticket, and
-// the further rows below (forward only, 64 per unit).
+// Tickets of one direction, level by level, in slots of four units.  Per
+// level: the groups of 64 rows or columns that are gathered or summed ahead of
+// a wide top (forward: where a row's list is longer than SN_GATHER_LONG;
+// transposed: where there are rows below), the wide tops, the narrow
+// supernodes four to a ticket, and the further rows below (forward only, 64
+// per unit).
 struct SnSchedule {
-  std::vector<int2> unit;  // (supernode, 0 or 1 + chunk)
-  std::vector<int> tick;   // unit bounds per ticket
-  std::vector<int> top;    // per supernode: the unit that solves its top
-  std::vector<int> first;  // per supernode: its first chunk unit, or -1
+  std::vector<SnUnit> unit;           // four slots per ticket
+  std::vector<std::vector<int>> deps; // per slot
+  std::vector<int> top;               // per supernode: the slot that solves its top
+  std::vector<int> group;             // per supernode: the slot of its first group, or -1
+  std::vector<int> first;             // per supernode: the slot of its first chunk, or -1
+  std::vector<int> dlist;
 };
 
-void sn_schedule(int m, const int *h_sup, const std::vector<int> &lev,
-                 const std::vector<int> &tb, bool transposed, SnSchedule &s) {
+void sn_schedule(int m, const int *h_sup, const int *h_nrows, const int *h_Lp,
+                 const std::vector<int> &lev, const std::vector<int> &tb,
+                 const std::vector<int> &longest, bool transposed, SnSchedule &s) {
   std::vector<int> order(m);
   for (int i = 0; i < m; ++i) order[i] = transposed ? m - 1 - i : i;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return lev[x] < lev[y]; });
-  s.tick.assign(1, 0);
   s.top.assign(m, -1);
-  s.first.assign(m > 0 ? m : 1, -1);
+  s.group.assign(m, -1);
+  s.first.assign(m, -1);
   auto width = [&](int i) { return h_sup[i + 1] - h_sup[i]; };
   auto below = [&](int i) { return tb[i + 1] - tb[i]; };
   auto narrow = [&](int i) {
     return width(i) <= SN_NARROW && (!transposed || below(i) <= SN_NARROW_ROWS);
   };
-  auto close = [&] { s.tick.push_back((int)s.unit.size()); };
-  auto chunks = [&](int i, int count) {
-    for (int c = 0; c < count; ++c) {
-      if (c == 0) s.first[i] = (int)s.unit.size();
-      s.unit.push_back(make_int2(i, c + 1));
-      close();
-    }
+  auto put = [&](int i, int kind) {
+    s.unit.push_back({h_sup[i], width(i), h_nrows[i], kind, h_Lp[i], tb[i], 0, 0});
+    return (int)s.unit.size() - 1;
+  };
+  auto close = [&] {
+    while (s.unit.size() % 4) s.unit.push_back({0, 0, 0, SN_NARROW_UNIT, 0, 0, 0, 0});
   };
   for (int a = 0, b = 0; a < m; a = b) {
     while (b < m && lev[order[b]] == lev[order[a]]) ++b;
-    if (transposed)
-      for (int j = a; j < b; ++j)
-        if (!narrow(order[j]) && below(order[j]) > 0) chunks(order[j], (width(order[j]) + 63) / 64);
+    for (int j = a; j < b; ++j)
+      if (!narrow(order[j]) &&
+          (transposed ? below(order[j]) > 0 : longest[order[j]] > SN_GATHER_LONG))
+        for (int g = 0; 64 * g < width(order[j]); ++g) {
+          const int u = put(order[j], transposed ? g : SN_GATHER_UNIT - g);
+          if (g == 0) s.group[order[j]] = u;
+          close();
+        }
     for (int j = a; j < b; ++j)
       if (!narrow(order[j])) {
-        s.top[order[j]] = (int)s.unit.size();
-        s.unit.push_back(make_int2(order[j], 0));
+        s.top[order[j]] = put(order[j], SN_TOP);
         close();
       }
-    int open = 0;
     for (int j = a; j < b; ++j)
-      if (narrow(order[j])) {
-        s.top[order[j]] = (int)s.unit.size();
-        s.unit.push_back(make_int2(order[j], 0));
-        if (++open == 4) {
-          close();
-          open = 0;
-        }
-      }
-    if (open) close();
+      if (narrow(order[j])) s.top[order[j]] = put(order[j], SN_NARROW_UNIT);
+    close();
     if (!transposed)
       for (int j = a; j < b; ++j) {
-        const int i = order[j], rest = below(i) - (narrow(i) ? SN_NARROW_ROWS : 0);
-        if (rest > 0) chunks(i, (rest + 63) / 64);
+        const int i = order[j];
+        for (int r = narrow(i) ? SN_NARROW_ROWS : 0; r < below(i); r += 64) {
+          const int u = put(i, r);
+          if (s.first[i] < 0) s.first[i] = u;
+          close();
+        }
       }
   }
+  s.deps.assign(s.unit.size(), {});
 }
 
-void flatten_deps(std::vector<std::vector<int>> &deps, std::vector<int> &ptr,
-                  std::vector<int> &list) {
-  ptr.assign(1, 0);
-  list.clear();
-  for (std::vector<int> &d : deps) {
+void flatten_deps(SnSchedule &s) {
+  for (size_t u = 0; u < s.unit.size(); ++u) {
+    std::vector<int> &d = s.deps[u];
+    if (d.empty()) continue;
     std::sort(d.begin(), d.end());
     d.erase(std::unique(d.begin(), d.end()), d.end());
-    list.insert(list.end(), d.begin(), d.end());
-    ptr.push_back((int)list.size());
+    s.unit[u].d0 = (int)s.dlist.size();
+    s.unit[u].dn = (int)d.size();
+    s.dlist.insert(s.dlist.end(), d.begin(), d.end());
   }
 }
 
@@ -985,48 +1123,51 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
   }
   for (int i = m - 1; i >= 0; --i)
     for (int k = tb[i]; k < tb[i + 1]; ++k) tlev[i] = std::max(tlev[i], tlev[owner[rowb[k]]] + 1);
+  std::vector<int> longest(m, 0);  // longest list of a supernode's rows
+  for (int i = 0; i < m; ++i)
+    for (int r = h_sup[i]; r < h_sup[i + 1]; ++r) longest[i] = std::max(longest[i], cnt[r + 1] - cnt[r]);
   SnSchedule fwd, bwd;
-  sn_schedule(m, h_sup, lev, tb, false, fwd);
-  sn_schedule(m, h_sup, tlev, tb, true, bwd);
-  // forward: a top waits for the units that write its rows' temporaries, a
-  // chunk of the rows below for its top
-  std::vector<std::vector<int>> deps(fwd.unit.size());
+  sn_schedule(m, h_sup, h_nrows, h_Lp, lev, tb, longest, false, fwd);
+  sn_schedule(m, h_sup, h_nrows, h_Lp, tlev, tb, longest, true, bwd);
+  // forward: a top, or the row groups of one that has them, waits for the
+  // units that write its rows' temporaries, a chunk of the rows below for its
+  // top.  transposed: the units that read x at the rows below (a narrow
+  // supernode, the column groups of a wide one) wait for the tops of their
+  // owners.  A top with groups waits for those
   for (int i = 0; i < m; ++i) {
-    const int head = h_sup[i + 1] - h_sup[i] <= SN_NARROW ? SN_NARROW_ROWS : 0;
+    const int w = h_sup[i + 1] - h_sup[i];
+    const int head = w <= SN_NARROW ? SN_NARROW_ROWS : 0;
+    std::vector<int> own;
     for (int k = 0; k < tb[i + 1] - tb[i]; ++k) {
-      const int producer = k < head ? fwd.top[i] : fwd.first[i] + (k - head) / 64;
-      std::vector<int> &d = deps[fwd.top[owner[rowb[tb[i] + k]]]];
+      const int row = rowb[tb[i] + k], o = owner[row];
+      const int producer = k < head ? fwd.top[i] : fwd.first[i] + 4 * ((k - head) / 64);
+      std::vector<int> &d = fwd.deps[fwd.group[o] < 0 ? fwd.top[o]
+                                                      : fwd.group[o] + 4 * ((row - h_sup[o]) / 64)];
       if (d.empty() || d.back() != producer) d.push_back(producer);
+      if (own.empty() || own.back() != bwd.top[o]) own.push_back(bwd.top[o]);
     }
+    for (int r = head, u = fwd.first[i]; u >= 0 && r < tb[i + 1] - tb[i]; r += 64, u += 4)
+      fwd.deps[u].push_back(fwd.top[i]);
+    if (bwd.group[i] < 0)
+      bwd.deps[bwd.top[i]] = own;
+    else
+      for (int g = 0; 64 * g < w; ++g) bwd.deps[bwd.group[i] + 4 * g] = own;
+    for (SnSchedule *s : {&fwd, &bwd})
+      if (s->group[i] >= 0) {
+        s->unit[s->top[i]].d0 = s->group[i];
+        s->unit[s->top[i]].dn = -1;
+      }
   }
-  for (size_t u = 0; u < fwd.unit.size(); ++u)
-    if (fwd.unit[u].y > 0) deps[u].push_back(fwd.top[fwd.unit[u].x]);
-  std::vector<int> dptr, dlist, tdptr, tdlist;
-  flatten_deps(deps, dptr, dlist);
-  // transposed: the units that read x at the rows below (a narrow supernode,
-  // the column groups of a wide one) wait for the tops of their owners; a
-  // wide top waits for its own groups by tag
-  deps.assign(bwd.unit.size(), {});
-  for (size_t u = 0; u < bwd.unit.size(); ++u) {
-    const int i = bwd.unit[u].x;
-    if (bwd.unit[u].y == 0 && bwd.first[i] >= 0) continue;
-    std::vector<int> &d = deps[u];
-    for (int k = tb[i]; k < tb[i + 1]; ++k) {
-      const int o = bwd.top[owner[rowb[k]]];
-      if (d.empty() || d.back() != o) d.push_back(o);
-    }
-  }
-  flatten_deps(deps, tdptr, tdlist);
+  flatten_deps(fwd);
+  flatten_deps(bwd);
   auto *q = new symamd_snplan_s();
   q->n = n;
   q->m = m;
   q->tcount = tcount;
   q->ntasks = old_tasks;
-  q->units = (int)fwd.unit.size();
-  q->tickets = (int)fwd.tick.size() - 1;
-  q->tunits = (int)bwd.unit.size();
-  q->ttickets = (int)bwd.tick.size() - 1;
-  const int64_t flags = std::max(1, std::max(q->units, q->tunits));
+  q->tickets = (int)(fwd.unit.size() / 4);
+  q->ttickets = (int)(bwd.unit.size() / 4);
+  const int64_t flags = 4 * (int64_t)std::max(1, std::max(q->tickets, q->ttickets));
   int rc = SYMAMD_OK;
   auto up = [&](int **dst, const int *src, size_t count) {
     if (rc != SYMAMD_OK) return;
@@ -1034,22 +1175,13 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
         (count && hipMemcpy(*dst, src, sizeof(int) * count, hipMemcpyHostToDevice) != hipSuccess))
       rc = fail(SYMAMD_ERR_ALLOC, "supernodal plan upload failed");
   };
-  up(&q->d_sup, h_sup, m + 1);
-  up(&q->d_nrows, h_nrows, m);
-  up(&q->d_Lp, h_Lp, m + 1);
-  up(&q->d_tb, tb.data(), m + 1);
-  up(&q->d_list, reinterpret_cast<const int *>(list.data()), 4 * (size_t)n);
   up(&q->d_tdst, tdst.data(), tb[m]);
   up(&q->d_rowb, rowb.data(), tb[m]);
-  up(&q->d_unit, reinterpret_cast<const int *>(fwd.unit.data()), 2 * fwd.unit.size());
-  up(&q->d_tick, fwd.tick.data(), fwd.tick.size());
-  up(&q->d_dptr, dptr.data(), dptr.size());
-  up(&q->d_dlist, dlist.data(), dlist.size());
-  up(&q->d_tunit, reinterpret_cast<const int *>(bwd.unit.data()), 2 * bwd.unit.size());
-  up(&q->d_ttick, bwd.tick.data(), bwd.tick.size());
-  up(&q->d_tdptr, tdptr.data(), tdptr.size());
-  up(&q->d_tdlist, tdlist.data(), tdlist.size());
-  up(&q->d_tbelow, bwd.first.data(), m);
+  up(&q->d_list, reinterpret_cast<const int *>(list.data()), 4 * (size_t)n);
+  up(&q->d_unit, reinterpret_cast<const int *>(fwd.unit.data()), 8 * fwd.unit.size());
+  up(&q->d_dlist, fwd.dlist.data(), fwd.dlist.size());
+  up(&q->d_tunit, reinterpret_cast<const int *>(bwd.unit.data()), 8 * bwd.unit.size());
+  up(&q->d_tdlist, bwd.dlist.data(), bwd.dlist.size());
   if (rc == SYMAMD_OK &&
       (hipMalloc(&q->d_T, sizeof(double) * (q->tcount > 0 ? q->tcount : 1)) != hipSuccess ||
        hipMalloc(&q->d_flags, sizeof(int) * flags) != hipSuccess ||
@@ -1077,8 +1209,8 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
   // columns per tile: a row's entries are loaded once for the columns of a
   // tile, but each step of a top's chain then divides for all of them.  On
   // the 13-level factor, forward + transposed with tiles of 1 / 2 / 4: k = 2
-  // 1.19 / 1.29 / - ms, k = 4 1.46 / 1.38 / 1.73 ms, k = 32 5.86 / 3.57 /
-  // 3.21 ms.
+  // 0.86 / 0.93 / - ms, k = 4 1.11 / 1.05 / 1.32 ms, k = 13 2.30 / 1.78 / 1.83
+  // ms, k = 32 4.94 / 3.17 / 2.64 ms.
   const int kt = k < 4 ? 1 : k < 16 ? 2 : 4;
   const int tiles = (k + kt - 1) / kt;
   // temporaries and tags for the tiles' columns
@@ -1087,7 +1219,7 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
     int *flags = nullptr;
     const int64_t cols = (int64_t)tiles * kt;
     const int64_t tc = q->tcount > 0 ? q->tcount : 1;
-    const int64_t nt = std::max(1, std::max(q->units, q->tunits));
+    const int64_t nt = 4 * (int64_t)std::max(1, std::max(q->tickets, q->ttickets));
     if (hipMalloc(&T, sizeof(double) * tc * cols) != hipSuccess ||
         hipMalloc(&flags, sizeof(int) * nt * cols) != hipSuccess) {
       if (T) (void)hipFree(T);
@@ -1103,23 +1235,15 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
     q->kcap = (int)cols;
   }
   SnArgs a;
-  a.sup = q->d_sup;
-  a.nrows = q->d_nrows;
-  a.Lp = q->d_Lp;
+  a.unit = reinterpret_cast<const SnUnit *>(transposed ? q->d_tunit : q->d_unit);
   a.Lx = d_Lx;
   a.x = d_x;
   a.T = q->d_T;
-  a.tb = q->d_tb;
   a.tdst = q->d_tdst;
   a.list = reinterpret_cast<const int4 *>(q->d_list);
-  a.unit = reinterpret_cast<const int2 *>(transposed ? q->d_tunit : q->d_unit);
-  a.tick = transposed ? q->d_ttick : q->d_tick;
-  a.dptr = transposed ? q->d_tdptr : q->d_dptr;
   a.dlist = transposed ? q->d_tdlist : q->d_dlist;
-  a.nunits = transposed ? q->tunits : q->units;
   a.ntick = transposed ? q->ttickets : q->tickets;
   a.rowb = q->d_rowb;
-  a.tbelow = q->d_tbelow;
   a.flags = q->d_flags;
   a.state = q->d_state;
   a.k = k;
@@ -1153,10 +1277,8 @@ int sn_check(symamd_handle h, symamd_snplan_s *q) {
 
 void sn_destroy(symamd_snplan_s *q) {
   if (!q) return;
-  void *ptrs[] = {q->d_sup,  q->d_nrows, q->d_Lp,    q->d_tb,     q->d_list,  q->d_tdst,
-                  q->d_rowb, q->d_unit,  q->d_tick,  q->d_dptr,   q->d_dlist, q->d_tunit,
-                  q->d_ttick, q->d_tdptr, q->d_tdlist, q->d_tbelow, q->d_T,   q->d_flags,
-                  q->d_state};
+  void *ptrs[] = {q->d_tdst,  q->d_rowb,   q->d_list, q->d_unit, q->d_dlist,
+                  q->d_tunit, q->d_tdlist, q->d_T,    q->d_flags, q->d_state};
   for (void *x : ptrs)
     if (x) (void)hipFree(x);
   delete q;

@@ -94,3 +94,26 @@ def test_quotients_outside_the_reciprocal_range(dev, kind):
             assert (same | (np.isnan(got[c]) & np.isnan(want[c]))).all(), (kind, solve, c)
         g1 = x1.cpu().numpy()
         assert ((g1 == want[0]) | (np.isnan(g1) & np.isnan(want[0]))).all()
+
+
+@pytest.mark.parametrize("k", [1, 2, 5, 17])
+def test_long_lists_gathered_ahead_of_wide_tops(dev, k):
+    """A tree whose wide tops subtract 15 to 113 temporaries per row: lists
+    gathered by the top's own waves, by workgroups in one round and in
+    several, at every column tile."""
+    sup, nrows, Lp, Li, Lx = W.bcsc_tree(11, 8, 150, 2.0, 4)
+    n, w = int(sup[-1]), np.diff(sup)
+    cnt = np.zeros(n, int)
+    for i in range(len(w)):
+        cnt[Li[Lp[i] + w[i]:Lp[i] + nrows[i]]] += 1
+    longest = np.maximum.reduceat(cnt, sup[:-1])[w > 64]
+    assert longest.min() <= 48 and longest.max() > 64 and ((longest > 48) & (longest <= 64)).any()
+    B = W.uniform(35, 0, k * n).reshape(k, n)
+    plan = sa.SupernodalPlan(sup, nrows, Lp, Li)
+    X = to_dev(B.copy())
+    print(f"[sn lists] k={k} n={n}", flush=True)
+    plan.solve(to_dev(Lx), X if k > 1 else X[0])
+    plan.check()
+    got = X.cpu().numpy()
+    for c in range(k):
+        assert bitwise_equal(got[c], oracle.sptrsv_csc_block(sup, nrows, Lp, Li, Lx, B[c])), c
