@@ -56,6 +56,11 @@ void free_plan_arrays(symamd_plan p) {
   }
   for (auto &kv : p->split)
     if (kv.second.d_rec) (void)hipFree(kv.second.d_rec);
+  for (void *q : p->ws_retired) (void)hipFree(q);
+  for (auto &kv : p->rows) {
+    (void)hipFree(kv.second.d_rec);
+    (void)hipFree(kv.second.d_item);
+  }
   for (auto &kv : p->rplans) free_region_plan(kv.second);
   for (auto &kv : p->rplans_t) free_region_plan(kv.second);
   free_ic0_pairs(p);
@@ -317,6 +322,11 @@ int prepare_solve(symamd_handle h, symamd_plan p, int k, int layout, const Choic
     SYMAMD_TRY(split_lists(h, p, split_threshold(h, tile_cols(k, c.tile)), &sl));
     return through_workspace(h, k, layout) ? prepare_workspace(h, p, k) : SYMAMD_OK;
   }
+  if (rows_path(h, p, k, c.exec == SYMAMD_EXEC_REGIONS ? SYMAMD_EXEC_SYNCFREE : c.exec, c.lanes,
+                c.tile)) {
+    const int rc = prepare_rows(h, p, k, through_workspace(h, k, layout));
+    if (rc != SYMAMD_ERR_ALLOC) return rc;  // without the memory: the unit executor
+  }
   UnitSet *us = nullptr;
   SYMAMD_TRY(plan_units(h, p, forward_rows_per_unit(k, c.lanes, c.tile), false, &us));
   const int kt = tile_cols(k, c.tile);
@@ -338,6 +348,8 @@ int run_solve(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld,
                                              : launch_regions(h, p, d_B, k, rs, cs);
     exec = SYMAMD_EXEC_SYNCFREE;
   }
+  if (rows_path(h, p, k, exec, lanes, tile))
+    return launch_rows(h, p, d_B, k, ld, rs, cs, through_workspace(h, k, layout));
   if (through_workspace(h, k, layout))
     return launch_forward_ws(h, p, d_B, k, ld, exec, lanes, tile);
   return launch_forward(h, p, d_B, k, rs, cs, exec, lanes, tile);
@@ -347,6 +359,7 @@ int capture_solve(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld,
                   int64_t rs, int64_t cs, int layout, const Choice &c, hipGraph_t *g,
                   hipGraphExec_t *ge) {
   SYMAMD_TRY(prepare_solve(h, p, k, layout, c));
+  p->ws_captured = true;
   hipStream_t cap = nullptr;
   SYMAMD_HIP(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
   hipStream_t saved = h->stream;

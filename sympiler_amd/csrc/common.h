@@ -316,6 +316,14 @@ struct SplitLists {
   std::vector<int> ptr;
 };
 
+// Schedule of the row executor (rows_exec.hip) for one number of column
+// lanes: rows in solving order and the items of every ticket.
+struct RowSchedule {
+  int4 *d_rec = nullptr;
+  int4 *d_item = nullptr;
+  int tickets = 0;
+};
+
 struct symamd_plan_s {
   int n = 0;
   int64_t nnz = 0;
@@ -342,6 +350,10 @@ struct symamd_plan_s {
   void *d_ws = nullptr;                // level-ordered row-major workspace
   // split level executor, per long-row threshold
   std::map<int, SplitLists> split;
+  std::map<int, RowSchedule> rows;  // row executor, per column lanes
+  bool rows_off = false;            // its workspace did not fit
+  bool ws_captured = false;         // a graph holds d_ws: replaced ones are kept
+  std::vector<void *> ws_retired;
   size_t ws_bytes = 0;
   int *d_orp = nullptr;                // caller CSR row pointers, n+1
   int *d_oci = nullptr;                // caller CSR column ids, nnz (built on first use)
@@ -464,6 +476,13 @@ int prepare_workspace(symamd_handle h, symamd_plan p, int k);
 // columns, and the long-row lists of a threshold (built once per plan and
 // threshold, outside graph capture).
 int split_threshold(symamd_handle h, int kt);
+// Row executor (rows_exec.hip): sync-free solves with several lanes per row.
+bool rows_path(symamd_handle h, symamd_plan p, int k, int exec, int lanes, int tile);
+// d_ws of at least `bytes`.
+int plan_workspace(symamd_plan p, size_t bytes);
+int prepare_rows(symamd_handle h, symamd_plan p, int k, bool turn);
+int launch_rows(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld, int64_t rs,
+                int64_t cs, bool turn);
 int split_lists(symamd_handle h, symamd_plan p, int thr, SplitLists **out);
 int launch_forward_ws(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld,
                       int exec, int lanes, int tile);

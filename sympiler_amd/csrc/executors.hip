@@ -995,15 +995,28 @@ int prepare_workspace(symamd_handle h, symamd_plan p, int k) {
       SYMAMD_HIP(hipGetLastError());
     }
   }
-  const size_t need = (size_t)p->n * k * (p->dtype == SYMAMD_F64 ? 8 : 4);
-  if (need > p->ws_bytes) {
-    if (p->d_ws) SYMAMD_HIP(hipFree(p->d_ws));
+  SYMAMD_TRY(plan_workspace(p, (size_t)p->n * k * (p->dtype == SYMAMD_F64 ? 8 : 4)));
+  SYMAMD_HIP(hipStreamSynchronize(h->stream));
+  return SYMAMD_OK;
+}
+
+// Grows the plan's workspace.  One that a captured graph holds stays until
+// the plan is destroyed.
+int plan_workspace(symamd_plan p, size_t bytes) {
+  if (bytes <= p->ws_bytes) return SYMAMD_OK;
+  void *ws = nullptr;
+  if (!p->ws_captured && p->d_ws) {
+    SYMAMD_HIP(hipFree(p->d_ws));
     p->d_ws = nullptr;
     p->ws_bytes = 0;
-    SYMAMD_HIP(hipMalloc(&p->d_ws, need));
-    p->ws_bytes = need;
   }
-  SYMAMD_HIP(hipStreamSynchronize(h->stream));
+  if (hipMalloc(&ws, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(SYMAMD_ERR_ALLOC, "plan workspace of %zu bytes", bytes);
+  }
+  if (p->d_ws) p->ws_retired.push_back(p->d_ws);
+  p->d_ws = ws;
+  p->ws_bytes = bytes;
   return SYMAMD_OK;
 }
 

@@ -1,0 +1,442 @@
+// rows_exec.hip -- forward solve of matrices with long, uneven rows for
+// gfx950: one persistent launch, rows shared by as many lanes as they have
+// entries, values passed from row to row by themselves.
+//
+// It runs sync-free solves with several lanes per row (the unit executor of
+// executors.hip cuts levels into units and waits for whole units; with rows
+// of 1 to 256 entries a unit waits for hundreds of others, about 7 us per
+// level).  Here every row is its own item:
+//   - before the solve the right-hand sides are copied aside and X is filled
+//     with the mark (a signalling NaN that no arithmetic produces), so a value
+//     read from X is either the mark or the solution: readers poll the values
+//     they need, and no tag or store acknowledgement lies on the chain;
+//   - a row's entries lie one or a few per lane, all their loads in flight at
+//     once; only the values not there yet are read again;
+//   - rows are scheduled level by level, in each level by the lanes they
+//     take, so that one wavefront solves 1 to 64 rows of similar length; with
+//     several right-hand sides a row too long for one wavefront is a
+//     workgroup's (its waves' sums meet in LDS).
+// What bounds it is the chain of levels for one right-hand side (a store on
+// one XCD reaching a poll on another, the lanes' reduction, the division:
+// 1.4 us per level) and, for several, the tickets a workgroup can take.
+// Zipf(1.8) matrix, n = 1e6, 449 levels, in ms with the unit executor and
+// here: one right-hand side 3.38 / 0.65, 4 columns 5.1 / 0.79, 13 columns
+// 10 / 1.06, 32 columns 18.0 / 1.35 (0.35 of it the turns of a column-major
+// block).
+// Workgroups take tickets in schedule order, so every value waited for is
+// held by a running workgroup; waits are bounded by the watchdog.
+//
+// Arithmetic: lanes sum their products, the sums are added across lanes (and
+// waves) in a fixed order, x = (b - sum) / L[i,i]; a row solved by one lane
+// per right-hand side subtracts its products in entry order, as the reference
+// does.  Results do not depend on timing.
+#include <algorithm>
+#include <vector>
+
+#include "device.h"
+
+namespace symamd {
+
+namespace {
+
+// Entries per lane in flight: one right-hand side, several, and the rows a
+// workgroup shares.  Lanes per row are chosen so that a row takes one round
+// where its wavefront is wide enough.
+constexpr int rows_epl(int c) { return c == 1 ? 4 : 8; }
+constexpr int ROWS_EPL_GROUP = 16;
+// Waves per workgroup.
+constexpr int rows_waves(int c) { return c == 1 ? 2 : 8; }
+// 32 column lanes: rows of at most ROWS_SHORT entries (two in three of the Zipf
+// matrix) are solved ROWS_PER_LANE to a lane, all their loads in flight, which
+// takes a quarter of their tickets (1.60 -> 1.35 ms; with 8 and 16 column
+// lanes, whose wavefronts hold more rows, it measured slower).
+constexpr int ROWS_SHORT = 2, ROWS_PER_LANE = 4;
+constexpr bool rows_short(int c) { return c == 32; }
+// Item kinds: log2 of the slices per row, or
+constexpr int ROWS_KIND_SHORT = 16, ROWS_KIND_GROUP = 17;
+
+template <typename T>
+struct RowArgs {
+  const int4 *rec;    // per scheduled row: first entry, diagonal entry, row
+  const int4 *item;   // per wave of a ticket: first record, rows, kind; a workgroup's row:
+                      // its record, kind
+  const int *ci;
+  const T *val;
+  const T *b;         // right-hand sides, row-major, k per row
+  T *x;               // marks, then the solution: row i, column c at i*rs + c*cs
+  int64_t rs, cs;
+  int k, tiles, ntick, total_waves;
+  int *state;
+  uint64_t timeout;
+};
+
+// Values of up to N entries of one lane: loads them all, then again those
+// that still read as the mark.
+template <typename T, int N>
+__device__ __forceinline__ void wait_values(T (&x)[N], const T *const (&p)[N],
+                                            const bool (&use)[N], int *state, uint64_t timeout) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) x[j] = ld_dev(p[j]);
+  bool pend = false;
+#pragma unroll
+  for (int j = 0; j < N; ++j) pend = pend || (use[j] && is_mark(x[j]));
+  if (!__any(pend)) return;
+  const uint64_t t0 = wall_ticks();
+  for (int rounds = 1; __any(pend); ++rounds) {
+    __builtin_amdgcn_s_sleep(1);
+    if (pend) {
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if (use[j] && is_mark(x[j])) x[j] = ld_dev(p[j]);
+      pend = false;
+#pragma unroll
+      for (int j = 0; j < N; ++j) pend = pend || (use[j] && is_mark(x[j]));
+    }
+    if ((rounds & 63) == 0 && wall_ticks() - t0 > timeout) {
+      if (pend) atomicOr(&state[ST_ERROR], 1);
+      break;
+    }
+  }
+}
+
+// Sum of entries e0 + first, + step, ... below e1 times x, in order, N at a
+// time; sub: subtracted from acc one by one instead.
+template <typename T, int N>
+__device__ __forceinline__ T row_sum(const RowArgs<T> &a, T acc, bool sub, int e0, int e1,
+                                     int first, int step, int64_t co, bool act) {
+  for (int base = first; __any(act && e0 + base < e1); base += N * step) {
+    T v[N], x[N];
+    const T *p[N];
+    bool use[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int e = e0 + base + j * step;
+      use[j] = act && e < e1;
+      const int q = min(e, e1);
+      v[j] = a.val[q];
+      p[j] = a.x + ((int64_t)a.ci[q] * a.rs + co);
+    }
+    wait_values<T, N>(x, p, use, a.state, a.timeout);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const T t = v[j] * x[j];
+      if (use[j]) acc = sub ? acc - t : acc + t;
+    }
+  }
+  return acc;
+}
+
+template <typename T, int C>
+__global__ __launch_bounds__(64 * rows_waves(C), 4) void k_rows(RowArgs<T> a) {
+  constexpr int W = rows_waves(C), SMAX = 64 / C;
+  __shared__ int slot;
+  __shared__ T part[W][C];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane % C, sub = lane / C;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) slot = atomicAdd(&a.state[ST_TICKET], 1);
+    __syncthreads();
+    const int tt = __builtin_amdgcn_readfirstlane(slot);
+    if (tt >= a.ntick * a.tiles) break;
+    const int tk = tt / a.tiles, tile = tt - tk * a.tiles;
+    const int col = tile * C + c;
+    const bool live = col < a.k;
+    const int cc = min(col, a.k - 1);
+    const int64_t co = cc * a.cs;
+    const int4 it = a.item[tk * W + wave];
+    if (it.w == ROWS_KIND_GROUP) {
+      // one row for the workgroup: wave and slice take every (W * SMAX)-th
+      // entry, slices are added by lane, waves in order
+      const int4 r = it;
+      const T b = a.b[(int64_t)r.z * a.k + cc], d = a.val[r.y];
+      T s = row_sum<T, ROWS_EPL_GROUP>(a, T(0), false, r.x, r.y, wave * SMAX + sub, W * SMAX, co,
+                                       true);
+#pragma unroll
+      for (int off = C; off < 64; off <<= 1) s += __shfl_xor(s, off);
+      if (sub == 0) part[wave][c] = s;
+      __syncthreads();
+      if (wave == 0 && sub == 0) {
+        T sum = part[0][c];
+#pragma unroll
+        for (int w = 1; w < W; ++w) sum += part[w][c];
+        if (live) st_dev(&a.x[r.z * a.rs + co], (b - sum) / d);
+      }
+      continue;
+    }
+    const int cnt = it.y;
+    if (cnt == 0) continue;
+    if (rows_short(C) && it.w == ROWS_KIND_SHORT) {
+      constexpr int M = ROWS_PER_LANE, N = ROWS_SHORT;
+      T v[M * N], x[M * N], b[M], d[M];
+      const T *p[M * N];
+      bool use[M * N];
+      int row[M];
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const int i = sub + SMAX * m;
+        const int4 r = a.rec[it.x + min(i, cnt - 1)];
+        row[m] = i < cnt ? r.z : -1;
+        b[m] = a.b[(int64_t)r.z * a.k + cc];
+        d[m] = a.val[r.y];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const int q = min(r.x + j, r.y);
+          use[m * N + j] = i < cnt && r.x + j < r.y;
+          v[m * N + j] = a.val[q];
+          p[m * N + j] = a.x + ((int64_t)a.ci[q] * a.rs + co);
+        }
+      }
+      wait_values<T, M * N>(x, p, use, a.state, a.timeout);
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        T s = b[m];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const T t = v[m * N + j] * x[m * N + j];
+          if (use[m * N + j]) s = s - t;
+        }
+        if (row[m] >= 0 && live) st_dev(&a.x[row[m] * a.rs + co], s / d[m]);
+      }
+      continue;
+    }
+    const int lg = it.w, slice = sub & ((1 << lg) - 1), i = sub >> lg;
+    const bool act = i < cnt;
+    const int4 r = a.rec[it.x + min(i, cnt - 1)];
+    const T b = a.b[(int64_t)r.z * a.k + cc], d = a.val[r.y];
+    T s = row_sum<T, rows_epl(C)>(a, lg ? T(0) : b, lg == 0, r.x, r.y, slice, 1 << lg, co, act);
+    for (int off = C; off < (C << lg); off <<= 1) s += __shfl_xor(s, off);
+    const T x = (lg ? b - s : s) / d;
+    if (act && slice == 0 && live) st_dev(&a.x[r.z * a.rs + co], x);
+  }
+  persistent_finish(a.state, a.total_waves);
+}
+
+// b[i*k + c] = X[i*rs + c*cs], X's place marked.
+template <typename T>
+__global__ __launch_bounds__(256) void k_rows_begin(int64_t count, int k, int64_t rs, int64_t cs,
+                                                    T *X, T *b) {
+  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < count;
+       t += (int64_t)gridDim.x * 256) {
+    const int64_t i = k == 1 ? t : t / k, c = t - i * k;
+    T *p = X + i * rs + c * cs;
+    b[t] = *p;
+    *p = mark_value<T>();
+  }
+}
+
+// Column-major block B (row i, column c at i + c*ld) through LDS tiles of 64
+// rows x 32 columns: begin copies it row-major to b and marks x; end copies x
+// back.
+template <typename T, bool BEGIN>
+__global__ __launch_bounds__(256) void k_rows_turn(int n, int k, int64_t ld, T *B, T *b, T *x) {
+  __shared__ T tile[64][33];
+  const int i0 = blockIdx.x * 64, c0 = blockIdx.y * 32;
+  const int tr = threadIdx.x % 64, tc = threadIdx.x / 64;
+  const int wc = threadIdx.x % 32, wr = threadIdx.x / 32;
+  if (BEGIN) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int c = tc + 4 * m, i = i0 + tr;
+      if (i < n && c0 + c < k) tile[tr][c] = B[i + (int64_t)(c0 + c) * ld];
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int r = wr + 8 * m, i = i0 + r;
+      if (i < n && c0 + wc < k) tile[r][wc] = x[(int64_t)i * k + c0 + wc];
+    }
+  }
+  __syncthreads();
+  if (BEGIN) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int r = wr + 8 * m, i = i0 + r;
+      if (i < n && c0 + wc < k) {
+        b[(int64_t)i * k + c0 + wc] = tile[r][wc];
+        x[(int64_t)i * k + c0 + wc] = mark_value<T>();
+      }
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int c = tc + 4 * m, i = i0 + tr;
+      if (i < n && c0 + c < k) B[i + (int64_t)(c0 + c) * ld] = tile[tr][c];
+    }
+  }
+}
+
+// Workgroups per CU: enough to have the rows of the next levels loaded ahead;
+// more only poll and slow the chain (n = 1e6, in ms: one right-hand side with
+// 512 / 1024 / 2048 waves 0.65 / 0.72 / 0.98; 4 columns with 1024 / 2048 /
+// 4096 1.11 / 0.79 / 0.91; 32 columns 2.69 / 1.55 / 1.35).
+constexpr int ROWS_PER_CU(int c) { return c == 1 ? 1 : c == 8 ? 1 : 2; }
+
+int rows_cols(int k) { return k == 1 ? 1 : k <= 8 ? 8 : k <= 16 ? 16 : 32; }
+
+// The schedule for C column lanes: per level the rows a workgroup shares,
+// then the others by descending slices, waves of a ticket filled from one
+// level.
+int rows_schedule(symamd_handle h, symamd_plan p, int C, RowSchedule **out) {
+  auto found = p->rows.find(C);
+  if (found != p->rows.end()) {
+    *out = &found->second;
+    return SYMAMD_OK;
+  }
+  const int n = p->n, W = rows_waves(C), smax = 64 / C, epl = rows_epl(C);
+  std::vector<int> rp(n + 1), perm(n);
+  SYMAMD_HIP(hipStreamSynchronize(h->stream));
+  SYMAMD_HIP(hipMemcpy(rp.data(), p->d_rp, sizeof(int) * (n + 1), hipMemcpyDeviceToHost));
+  SYMAMD_HIP(hipMemcpy(perm.data(), p->d_perm, sizeof(int) * n, hipMemcpyDeviceToHost));
+  int lgmax = 0;
+  while ((1 << lgmax) < smax) ++lgmax;
+  // class of a row, in solving order: the workgroup's (0), lgmax .. 0 slices
+  // as 1 .. lgmax + 1, short (lgmax + 2)
+  auto cls = [&](int q) {
+    const int len = rp[q + 1] - 1 - rp[q];
+    if (C > 1 && len > 2 * epl * smax) return 0;
+    if (rows_short(C) && len <= ROWS_SHORT) return lgmax + 2;
+    int lg = 0;
+    while (lg < lgmax && (epl << lg) < len) ++lg;
+    return lgmax + 1 - lg;
+  };
+  std::vector<int4> rec(n > 0 ? n : 1), item;
+  int at = 0;
+  std::vector<int> first(lgmax + 4);
+  for (int l = 0; l < p->levels; ++l) {
+    const int q0 = p->h_lvl_ptr[l], q1 = p->h_lvl_ptr[l + 1];
+    std::fill(first.begin(), first.end(), 0);
+    for (int q = q0; q < q1; ++q) ++first[cls(q) + 1];
+    for (size_t i = 1; i < first.size(); ++i) first[i] += first[i - 1];
+    std::vector<int> next(first.begin(), first.end() - 1);
+    for (int q = q0; q < q1; ++q)
+      rec[at + next[cls(q)]++] = make_int4(rp[q], rp[q + 1] - 1, perm[q], 0);
+    for (int i = 0; i < first[1]; ++i) {
+      int4 r = rec[at + i];
+      r.w = ROWS_KIND_GROUP;
+      item.insert(item.end(), W, r);
+    }
+    for (int c = 1; c < lgmax + 3; ++c) {
+      const int lg = c == lgmax + 2 ? ROWS_KIND_SHORT : lgmax + 1 - c;
+      const int rows = c == lgmax + 2 ? smax * ROWS_PER_LANE : smax >> lg;
+      for (int i = first[c]; i < first[c + 1]; i += rows)
+        item.push_back(make_int4(at + i, std::min(rows, first[c + 1] - i), 0, lg));
+    }
+    while (item.size() % W) item.push_back(make_int4(0, 0, 0, 0));
+    at += q1 - q0;
+  }
+  RowSchedule s;
+  s.tickets = (int)(item.size() / W);
+  if (hipMalloc(&s.d_rec, sizeof(int4) * rec.size()) != hipSuccess ||
+      hipMalloc(&s.d_item, sizeof(int4) * std::max<size_t>(item.size(), 1)) != hipSuccess) {
+    if (s.d_rec) (void)hipFree(s.d_rec);
+    return fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", n);
+  }
+  if (hipMemcpy(s.d_rec, rec.data(), sizeof(int4) * rec.size(), hipMemcpyHostToDevice) !=
+          hipSuccess ||
+      hipMemcpy(s.d_item, item.data(), sizeof(int4) * item.size(), hipMemcpyHostToDevice) !=
+          hipSuccess) {
+    (void)hipFree(s.d_rec);
+    (void)hipFree(s.d_item);
+    return fail(SYMAMD_ERR_HIP, "row schedule: copy failed");
+  }
+  *out = &(p->rows[C] = s);
+  return SYMAMD_OK;
+}
+
+template <typename T, int C>
+int launch_rows_c(symamd_handle h, RowArgs<T> a) {
+  constexpr int W = rows_waves(C);
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_rows<T, C>, 64 * W,
+                                                   0) != hipSuccess ||
+      per_cu < 1)
+    per_cu = 1;
+  int64_t grid = (int64_t)std::min(per_cu, ROWS_PER_CU(C)) * h->num_cus;
+  if (h->max_waves > 0) grid = std::min<int64_t>(grid, (h->max_waves + W - 1) / W);
+  grid = std::max<int64_t>(1, std::min<int64_t>(grid, (int64_t)a.ntick * a.tiles));
+  a.total_waves = (int)grid * W;
+  k_rows<T, C><<<(unsigned)grid, 64 * W, 0, h->stream>>>(a);
+  SYMAMD_HIP(hipGetLastError());
+  return SYMAMD_OK;
+}
+
+template <typename T>
+int launch_rows_t(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld, int64_t rs,
+                  int64_t cs, bool turn) {
+  RowSchedule *s = nullptr;
+  const int C = rows_cols(k);
+  SYMAMD_TRY(rows_schedule(h, p, C, &s));
+  const int64_t count = (int64_t)p->n * k;
+  RowArgs<T> a{};
+  a.rec = s->d_rec;
+  a.item = s->d_item;
+  a.ntick = s->tickets;
+  a.tiles = (k + C - 1) / C;
+  a.ci = p->d_ci;
+  a.val = (const T *)p->d_val;
+  T *const b = (T *)p->d_ws;
+  a.b = b;
+  a.k = k;
+  a.state = p->d_state;
+  a.timeout = h->timeout_ticks();
+  const dim3 tg((unsigned)((p->n + 63) / 64), (unsigned)((k + 31) / 32));
+  if (turn) {
+    a.x = b + count;
+    a.rs = k;
+    a.cs = 1;
+    k_rows_turn<T, true><<<tg, 256, 0, h->stream>>>(p->n, k, ld, (T *)d_B, b, a.x);
+  } else {
+    a.x = (T *)d_B;
+    a.rs = rs;
+    a.cs = cs;
+    const unsigned grid = (unsigned)std::min<int64_t>((count + 255) / 256, 8192);
+    k_rows_begin<T><<<grid, 256, 0, h->stream>>>(count, k, rs, cs, a.x, b);
+  }
+  SYMAMD_HIP(hipGetLastError());
+  switch (C) {
+    case 1: SYMAMD_TRY((launch_rows_c<T, 1>(h, a))); break;
+    case 8: SYMAMD_TRY((launch_rows_c<T, 8>(h, a))); break;
+    case 16: SYMAMD_TRY((launch_rows_c<T, 16>(h, a))); break;
+    default: SYMAMD_TRY((launch_rows_c<T, 32>(h, a)));
+  }
+  if (turn) {
+    k_rows_turn<T, false><<<tg, 256, 0, h->stream>>>(p->n, k, ld, (T *)d_B, b, a.x);
+    SYMAMD_HIP(hipGetLastError());
+  }
+  return SYMAMD_OK;
+}
+
+}  // namespace
+
+// Whether a sync-free solve of k right-hand sides runs here: several lanes
+// per row beside the column tile (one lane per row keeps the reference's
+// order in every row, which the unit executor does), the marked protocol on,
+// no unit trace, and memory for the workspace.
+bool rows_path(symamd_handle h, symamd_plan p, int k, int exec, int lanes, int tile) {
+  return exec == SYMAMD_EXEC_SYNCFREE && lanes > 1 && 2 * tile_cols(k, tile) <= 64 &&
+         !h->unmarked && !h->trace && !p->rows_off;
+}
+
+// The schedule and the workspace (the right-hand sides, and for turned blocks
+// the solution), before any launch or capture.
+int prepare_rows(symamd_handle h, symamd_plan p, int k, bool turn) {
+  RowSchedule *s = nullptr;
+  int rc = rows_schedule(h, p, rows_cols(k), &s);
+  if (rc == SYMAMD_OK)
+    rc = plan_workspace(p, (size_t)p->n * k * (turn ? 2 : 1) * (p->dtype == SYMAMD_F64 ? 8 : 4));
+  if (rc == SYMAMD_ERR_ALLOC) p->rows_off = true;
+  return rc;
+}
+
+// B in place; turn: a column-major block of leading dimension ld through the
+// row-major workspace.  prepare_rows must have run.
+int launch_rows(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld, int64_t rs,
+                int64_t cs, bool turn) {
+  if (p->n == 0 || k == 0) return SYMAMD_OK;
+  return p->dtype == SYMAMD_F64 ? launch_rows_t<double>(h, p, d_B, k, ld, rs, cs, turn)
+                                : launch_rows_t<float>(h, p, d_B, k, ld, rs, cs, turn);
+}
+
+}  // namespace symamd
