@@ -26,10 +26,11 @@
 // Workgroups take tickets in schedule order, so every value waited for is
 // held by a running workgroup; waits are bounded by the watchdog.
 //
-// Arithmetic: lanes sum their products, the sums are added across lanes (and
-// waves) in a fixed order, x = (b - sum) / L[i,i]; a row solved by one lane
-// per right-hand side subtracts its products in entry order, as the reference
-// does.  Results do not depend on timing.
+// Arithmetic: x = (b - sum) / L[i,i], the sum over a lane's entries pairwise,
+// then across lanes and waves in a fixed order; results do not depend on
+// timing.  (Subtracting the products of short rows from b one by one, in the
+// reference's order, leaves an error against 64 bits 1.6 times the unit
+// executor's, whose lanes sum first too.)
 #include <algorithm>
 #include <vector>
 
@@ -99,11 +100,12 @@ __device__ __forceinline__ void wait_values(T (&x)[N], const T *const (&p)[N],
   }
 }
 
-// Sum of entries e0 + first, + step, ... below e1 times x, in order, N at a
-// time; sub: subtracted from acc one by one instead.
+// Sum over entries e0 + first, + step, ... below e1 of value times x: rounds
+// of N entries, added pairwise, the rounds in order.
 template <typename T, int N>
-__device__ __forceinline__ T row_sum(const RowArgs<T> &a, T acc, bool sub, int e0, int e1,
-                                     int first, int step, int64_t co, bool act) {
+__device__ __forceinline__ T row_sum(const RowArgs<T> &a, int e0, int e1, int first, int step,
+                                     int64_t co, bool act) {
+  T acc = T(0);
   for (int base = first; __any(act && e0 + base < e1); base += N * step) {
     T v[N], x[N];
     const T *p[N];
@@ -118,10 +120,12 @@ __device__ __forceinline__ T row_sum(const RowArgs<T> &a, T acc, bool sub, int e
     }
     wait_values<T, N>(x, p, use, a.state, a.timeout);
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const T t = v[j] * x[j];
-      if (use[j]) acc = sub ? acc - t : acc + t;
-    }
+    for (int j = 0; j < N; ++j) v[j] = use[j] ? v[j] * x[j] : T(0);
+#pragma unroll
+    for (int h = N / 2; h >= 1; h >>= 1)
+#pragma unroll
+      for (int j = 0; j < h; ++j) v[j] = v[j] + v[j + h];
+    acc = acc + v[0];
   }
   return acc;
 }
@@ -151,8 +155,7 @@ __global__ __launch_bounds__(64 * rows_waves(C), 4) void k_rows(RowArgs<T> a) {
       // entry, slices are added by lane, waves in order
       const int4 r = it;
       const T b = a.b[(int64_t)r.z * a.k + cc], d = a.val[r.y];
-      T s = row_sum<T, ROWS_EPL_GROUP>(a, T(0), false, r.x, r.y, wave * SMAX + sub, W * SMAX, co,
-                                       true);
+      T s = row_sum<T, ROWS_EPL_GROUP>(a, r.x, r.y, wave * SMAX + sub, W * SMAX, co, true);
 #pragma unroll
       for (int off = C; off < 64; off <<= 1) s += __shfl_xor(s, off);
       if (sub == 0) part[wave][c] = s;
@@ -191,13 +194,11 @@ __global__ __launch_bounds__(64 * rows_waves(C), 4) void k_rows(RowArgs<T> a) {
       wait_values<T, M * N>(x, p, use, a.state, a.timeout);
 #pragma unroll
       for (int m = 0; m < M; ++m) {
-        T s = b[m];
+        T s = T(0);
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-          const T t = v[m * N + j] * x[m * N + j];
-          if (use[m * N + j]) s = s - t;
-        }
-        if (row[m] >= 0 && live) st_dev(&a.x[row[m] * a.rs + co], s / d[m]);
+        for (int j = 0; j < N; ++j)
+          if (use[m * N + j]) s = s + v[m * N + j] * x[m * N + j];
+        if (row[m] >= 0 && live) st_dev(&a.x[row[m] * a.rs + co], (b[m] - s) / d[m]);
       }
       continue;
     }
@@ -205,9 +206,9 @@ __global__ __launch_bounds__(64 * rows_waves(C), 4) void k_rows(RowArgs<T> a) {
     const bool act = i < cnt;
     const int4 r = a.rec[it.x + min(i, cnt - 1)];
     const T b = a.b[(int64_t)r.z * a.k + cc], d = a.val[r.y];
-    T s = row_sum<T, rows_epl(C)>(a, lg ? T(0) : b, lg == 0, r.x, r.y, slice, 1 << lg, co, act);
+    T s = row_sum<T, rows_epl(C)>(a, r.x, r.y, slice, 1 << lg, co, act);
     for (int off = C; off < (C << lg); off <<= 1) s += __shfl_xor(s, off);
-    const T x = (lg ? b - s : s) / d;
+    const T x = (b - s) / d;
     if (act && slice == 0 && live) st_dev(&a.x[r.z * a.rs + co], x);
   }
   persistent_finish(a.state, a.total_waves);
