@@ -499,7 +499,7 @@ int launch_lbc(symamd_handle h, int n, const int *d_Lp, const int *d_Li,
                const int *d_partition);
 // Regions (regions.cpp): clustering of the rows, the region-ordered level
 // permutation of a plan, and the owner schedule of a unit set for nw waves.
-int cluster_regions(int n, const int *Lp, const int *Li, int max_rows,
+int cluster_regions(int n, const int *Lp, const int *Li, int max_rows, bool banded,
                     std::vector<int> &region);
 int order_by_regions(symamd_handle h, symamd_plan p, const int *d_Lp, const int *d_Li);
 int plan_owners(symamd_handle h, symamd_plan p, UnitSet *us, int nw);

@@ -1102,13 +1102,15 @@ int region_waves(symamd_handle h, int k) {
 // memory-wave kernel, 256 for tasks of eight columns run by one wave and
 // 512 otherwise (measured on the IC(0) factors of the 128^3 and 64^3
 // Laplacians: k = 1 with the memory wave 0.309 / 0.137 ms at 1024 vs
-// 0.323 / 0.142 ms at 512 -- the 512-system batch of 2D grids prefers 512,
-// which the tuner finds; k = 32 with four waves per task is fastest at 512).
+// 0.323 / 0.142 ms at 512; k = 32 with four waves per task is fastest at
+// 512).  Past 16 tasks of 1024 rows per CU the tasks, not the chain, set the
+// time, and smaller ones run more to a CU: the batch of 512 grids (8.4 M rows)
+// takes 0.42 / 0.48 / 0.55 ms at 384 / 512 / 1024 rows (0.55 at 256).
 int region_cap(symamd_handle h, symamd_plan p, int k) {
   if (h->region_cap > 0) return h->region_cap;
   const int tuned = p ? tuned_region_cap(p, k) : 0;
   if (tuned > 0) return tuned;
-  if (k == 1 && h->region_mw) return 1024;
+  if (k == 1 && h->region_mw) return !p || p->n <= 16 * 1024 * h->num_cus ? 1024 : 384;
   return task_cols(k) == KG_MAX && region_waves(h, k) == 1 ? 256 : 512;
 }
 

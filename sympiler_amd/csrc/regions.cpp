@@ -62,13 +62,144 @@ WGraph initial_graph(int n, const int *Lp, const int *Li) {
   return g;
 }
 
+// Rounds of 64 rows that the levels of an a x b x c box take (its level s
+// holds the points with x + y + z = s).
+int64_t box_rounds(int64_t a, int64_t b, int64_t c) {
+  int64_t rounds = 0, width = 0;
+  auto plane = [&](int64_t s) {  // points of the a x b face with x + y = s
+    return s < 0 || s > a + b - 2 ? 0 : std::min({s + 1, a, b, a + b - 1 - s});
+  };
+  for (int64_t s = 0; s <= a + b + c - 3; ++s) {
+    width += plane(s) - plane(s - c);
+    rounds += (width + 63) / 64;
+  }
+  return rounds;
+}
+
+// How a grid of nx x ny x nz points (nz = 1: a plane) is cut into boxes: of
+// all cuts into px x py x pz equal boxes (sides differing by at most one) of
+// at most max_rows points, the one whose longest chain of boxes takes least,
+// at `hop` us per hand-off and `round` us per 64 rows of a level.  (4.4, 0.44)
+// are the region kernel's costs for a block of right-hand sides and (3.6,
+// 0.14) those for a single one, whose regions overlap band by band, on the
+// IC(0) factor of the 128^3 Laplacian; they give 8 x 8 x 8 boxes there, and
+// for a single right-hand side 8 x 8 x 16 where 1024 rows are allowed.
+// (10 x 10 x 10 boxes have a shorter chain, but levels of 75 rows: 0.331 ms
+// against 0.295.)  Boxes of uneven sides measured 8 % above this estimate in 3D
+// (8 x 10 x 10 there: 0.312 ms), not in a plane (300 x 500: 30 x 34 boxes 0.313
+// ms, 20 x 50 ones 0.377).
+void lattice_cut(int64_t nx, int64_t ny, int64_t nz, int max_rows, double hop, double round,
+                 int64_t (&pieces)[3]) {
+  const int64_t dim[3] = {nx, ny, nz};
+  double best = 0.0;
+  pieces[0] = 0;
+  auto side = [&](int a, int64_t p) { return (dim[a] + p - 1) / p; };
+  // candidate piece counts per axis: the fewest for every side up to max_rows
+  std::vector<int64_t> cand[3];
+  for (int a = 0; a < 3; ++a)
+    for (int64_t s = std::min<int64_t>(dim[a], max_rows); s >= 1; --s) {
+      const int64_t p = (dim[a] + s - 1) / s;
+      if (cand[a].empty() || cand[a].back() != p) cand[a].push_back(p);
+    }
+  for (int64_t px : cand[0])
+    for (int64_t py : cand[1]) {
+      const int64_t a = side(0, px), b = side(1, py);
+      if (a * b > max_rows) continue;
+      for (int64_t pz : cand[2]) {
+        const int64_t c = side(2, pz);
+        const double chain = (double)(px + py + pz - 2);
+        // even a box of one level costs a hand-off: more pieces cannot win
+        if (pieces[0] != 0 && chain * hop >= best) break;
+        if (a * b * c > max_rows) continue;
+        const bool uneven = nz > 1 && (nx % a || ny % b || nz % c);
+        const double cost =
+            chain * (hop + round * (double)box_rounds(a, b, c)) * (uneven ? 1.08 : 1.0);
+        if (pieces[0] == 0 || cost < best) {
+          best = cost;
+          pieces[0] = px;
+          pieces[1] = py;
+          pieces[2] = pz;
+        }
+      }
+    }
+}
+
+// Regions of grids in natural order: when the rows fall into runs without
+// entries between them (the systems of a batch), each of them the points of a
+// 2D or 3D grid whose rows read only their neighbours before them along the
+// axes (column offsets 1, nx and nx * ny), the regions are boxes of the grid.
+// The matching below gives such boxes where every side is a power of two
+// times a box's; on other grids the points left over at an edge grow into
+// plates that read and are read by the same neighbours, which end up merged
+// and cut by level: the 97 x 83 x 101 grid then has a chain of 134 regions
+// where boxes give 35.  False, and nothing set, for any other pattern.
+bool lattice_regions(int n, const int *Lp, const int *Li, int max_rows, bool banded,
+                     std::vector<int> &region, int &count) {
+  std::vector<int> low(n + 1, n);  // lowest column of rows >= i
+  for (int i = n - 1; i >= 0; --i) low[i] = std::min(low[i + 1], Lp[i] < Lp[i + 1] ? Li[Lp[i]] : i);
+  struct Run {
+    int first, rows;
+    int64_t d[3], pieces[3];  // offsets along the axes, boxes along the axes
+  };
+  std::vector<Run> runs;
+  int grids = 0;
+  for (int a = 0, b; a < n; a = b) {
+    b = a + 1;
+    while (b < n && low[b] < b) ++b;
+    Run r{a, b - a, {1, b - a, b - a}, {1, 1, 1}};
+    int64_t off[3] = {0, 0, 0};  // distinct offsets, ascending
+    int m = 0;
+    for (int i = a; i < b; ++i)
+      for (int j = Lp[i]; j < Lp[i + 1]; ++j) {
+        const int64_t d = (int64_t)i - Li[j];
+        if (d == 0 || (m > 0 && d == off[0]) || (m > 1 && d == off[1]) || (m > 2 && d == off[2]))
+          continue;
+        if (d < 0 || m == 3) return false;
+        off[m++] = d;
+        std::sort(off, off + m);
+      }
+    if (m > 0) {
+      if (m < 2 || off[0] != 1 || r.rows % off[1] || off[m - 1] % off[1] || r.rows % off[m - 1])
+        return false;
+      r.d[1] = off[1];
+      r.d[2] = m == 3 ? off[2] : r.rows;
+      // no neighbour across the end of a line or a plane
+      for (int i = a; i < b; ++i)
+        for (int j = Lp[i]; j < Lp[i + 1]; ++j) {
+          const int64_t d = (int64_t)i - Li[j], at = i - a;
+          if ((d == 1 && at % r.d[1] == 0) || (d == r.d[1] && at % r.d[2] < r.d[1])) return false;
+        }
+      lattice_cut(r.d[1], r.d[2] / r.d[1], r.rows / r.d[2], max_rows,
+                  banded ? 3.6 : 4.4, banded ? 0.14 : 0.44, r.pieces);
+      ++grids;
+    }
+    runs.push_back(r);
+  }
+  if (grids == 0) return false;
+  int64_t next = 0;
+  for (const Run &r : runs) {
+    const int64_t nx = r.d[1], ny = r.d[2] / r.d[1], nz = r.rows / r.d[2];
+    for (int i = 0; i < r.rows; ++i) {
+      const int64_t x = i % nx, y = i / nx % ny, z = i / (nx * ny);
+      region[r.first + i] = (int)(next + x * r.pieces[0] / nx +
+                                  r.pieces[0] * (y * r.pieces[1] / ny +
+                                                 r.pieces[1] * (z * r.pieces[2] / nz)));
+    }
+    next += r.pieces[0] * r.pieces[1] * r.pieces[2];
+  }
+  count = (int)next;
+  return true;
+}
+
 }  // namespace
 
-int cluster_regions(int n, const int *Lp, const int *Li, int max_rows,
+int cluster_regions(int n, const int *Lp, const int *Li, int max_rows, bool banded,
                     std::vector<int> &region) {
   region.resize(n);
   std::iota(region.begin(), region.end(), 0);
   if (n == 0 || max_rows < 2) return n;
+  int boxes = 0;
+  if (lattice_regions(n, Lp, Li, max_rows, banded, region, boxes)) return boxes;
   WGraph g = initial_graph(n, Lp, Li);
   std::vector<int> size(n, 1);
   int nc = n;
@@ -191,7 +322,7 @@ int order_by_regions(symamd_handle h, symamd_plan p, const int *d_Lp, const int 
   SYMAMD_HIP(hipMemcpy(Li.data(), d_Li, sizeof(int) * p->nnz, hipMemcpyDeviceToHost));
   SYMAMD_HIP(hipMemcpy(perm.data(), p->d_perm, sizeof(int) * n, hipMemcpyDeviceToHost));
   std::vector<int> reg;
-  const int R = cluster_regions(n, Lp.data(), Li.data(), h->region_rows, reg);
+  const int R = cluster_regions(n, Lp.data(), Li.data(), h->region_rows, false, reg);
   int64_t inside = 0, off = 0;
   for (int i = 0; i < n; ++i)
     for (int j = Lp[i]; j < Lp[i + 1]; ++j)
@@ -481,7 +612,7 @@ bool build_region_schedule(int n, int64_t nnz, int levels, const int *lvl_ptr,
   for (int i = 0; i < n; ++i)
     std::copy(cci.begin() + crp[ipos[i]], cci.begin() + crp[ipos[i] + 1], Li.begin() + Lp[i]);
   std::vector<int> reg;
-  int R = cluster_regions(n, Lp.data(), Li.data(), cap, reg);
+  int R = cluster_regions(n, Lp.data(), Li.data(), cap, band_slices < 255, reg);
   R = make_acyclic(n, Lp.data(), Li.data(), lev, cap, reg, R);
   int64_t inside = 0, offd = 0;
   for (int i = 0; i < n; ++i)
