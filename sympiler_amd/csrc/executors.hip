@@ -994,10 +994,10 @@ int prepare_workspace(symamd_handle h, symamd_plan p, int k) {
           p->nnz, p->d_ci, p->d_ipos, p->d_cpos);
       SYMAMD_HIP(hipGetLastError());
     }
+    // what was built serves solves on any stream from here on
+    SYMAMD_HIP(hipStreamSynchronize(h->stream));
   }
-  SYMAMD_TRY(plan_workspace(p, (size_t)p->n * k * (p->dtype == SYMAMD_F64 ? 8 : 4)));
-  SYMAMD_HIP(hipStreamSynchronize(h->stream));
-  return SYMAMD_OK;
+  return plan_workspace(p, (size_t)p->n * k * (p->dtype == SYMAMD_F64 ? 8 : 4));
 }
 
 // Grows the plan's workspace.  One that a captured graph holds stays until
