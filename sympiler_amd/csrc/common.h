@@ -127,6 +127,12 @@ struct UnitSet {
   int64_t xdeps = 0;
 };
 
+// Packed structure of a factorization's units (factor0.hip).
+struct FactorPack {
+  int64_t *d_off = nullptr;
+  int *d_wide = nullptr, *d_data = nullptr;
+};
+
 // IC(0) update pairs of one variant (factor0.hip): entry p of the caller's CSR
 // subtracts Lx[pa[t]] * Lx[pb[t]] for t in [pp[p], pp[p+1]), in order.
 struct Ic0Pairs {
@@ -135,6 +141,7 @@ struct Ic0Pairs {
   int *d_pa = nullptr;
   int *d_pb = nullptr;
   int *d_dpos = nullptr;    // position of L[c,c] for each entry (r, c)
+  FactorPack pack;
 };
 
 // Region schedule: each region (a compact cluster of rows, at most `cap`
@@ -394,6 +401,7 @@ struct symamd_ilu0_s {
   int64_t pairs = 0;
   int64_t *d_pp = nullptr;
   int *d_pa = nullptr, *d_pb = nullptr, *d_dpos = nullptr;
+  symamd::FactorPack pack;
 };
 
 // Supernodal (BCSC) solve plan (supernodal.hip): the rows' lists of
