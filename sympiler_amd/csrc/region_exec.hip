@@ -697,9 +697,14 @@ __device__ __forceinline__ void grad_bands(T *gL, const T *xs, const T *xfl, con
 // a task that reads them waits only for that, loads its halo values as soon
 // as it reaches their band and loads again any value still carrying the
 // mark.  Stores are never waited for, and no band is published: a value is
-// ready when it is no longer the mark.
+// ready when it is no longer the mark.  A second memory wave stores the rows
+// (and writes grad-L while there is nothing to store), so that a band's stores
+// never wait behind a round of halo loads, most of a microsecond on the chain
+// from region to region (one column of the IC(0) factors of the 128^3 / 64^3 /
+// 97 x 83 x 101 Laplacians: 0.295 / 0.129 / 0.205 ms with one memory wave, 0.268 /
+// 0.118 / 0.191 with two).
 template <typename T, int KT, int ES, int NC, bool MK>
-__global__ __launch_bounds__(64 * (NC + 1)) void k_regions_mw(RegionArgs<T> a) {
+__global__ __launch_bounds__(64 * (NC + 1 + MK)) void k_regions_mw(RegionArgs<T> a) {
   extern __shared__ __align__(16) uint8_t smem[];
   constexpr int KS = log2c<KT>();
   constexpr int VS = (int)sizeof(T);
@@ -716,7 +721,7 @@ __global__ __launch_bounds__(64 * (NC + 1)) void k_regions_mw(RegionArgs<T> a) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool memw = wid == NC;
+  const bool memw = wid == NC, storew = MK && wid == NC + 1;
   const int target = ld_dev(&a.state[ST_EPOCH]) + 1;
   const int64_t base = (int64_t)target << 8;
   const int ntasks = a.R * a.groups;
@@ -746,7 +751,7 @@ __global__ __launch_bounds__(64 * (NC + 1)) void k_regions_mw(RegionArgs<T> a) {
     const int *lwp = reinterpret_cast<const int *>(rb + L.wptr);
     if (wid == 0) trace_mark(a.trace, a.trace_cap, task, 0);
     // 1. the record, every wave a share of it
-    dma_bytes<NC + 1>(rb, a.rec + (size_t)ru * 16, rn * 16, wid);
+    dma_bytes<NC + 1 + MK>(rb, a.rec + (size_t)ru * 16, rn * 16, wid);
     vm_wait();
     if (tid <= NC) s_ctl[9 + tid] = 0;
     __syncthreads();
@@ -771,14 +776,66 @@ __global__ __launch_bounds__(64 * (NC + 1)) void k_regions_mw(RegionArgs<T> a) {
         vm_wait();
         if (lane == 0) st_dev(myflag, base + 1);
       }
-      // 3. rounds: issue the stores of every band all compute waves have
-      // finished and the halo loads of every band whose waits are met, wait
-      // once for all of them, then publish and signal
-      int loaded = 0, issued = 0, stored = 0;
-      bool halo_in = false;  // marked protocol: band `loaded`'s halo is in LDS
-      int graded = 0;        // marked protocol with grad-L: bands whose grad-L is written
       uint64_t t0 = wall_ticks();
       bool gave_up = false;
+      int loaded = 0;
+      if constexpr (MK) {
+        // 3. once every region read has marked its rows (a region stays marked
+        // for the rest of the launch), every halo value of the task is loaded
+        // at once; values still marked are loaded again band by band
+        bool halo_in = false;
+        while (loaded < nb) {
+          bool moved = false;
+          if (!halo_in) {
+            if (gave_up || all_marked(ldep, nd, a.tflags, base, a.groups, g, a.R)) {
+              if (nh > 0)
+                load_rows<T, KT, ES, true, 1>(xs + (size_t)a.smax * KT, a.X, lhalo, nh, kc, c0,
+                                              a.rs, a.cs, a.n, 0);
+              vm_wait();
+              wave_lds_sync();
+              halo_in = true;
+              moved = true;
+            }
+          }
+          if (halo_in) {
+            const int hb0 = lhb[loaded], hb1 = lhb[loaded + 1];
+            bool marked = false;
+            for (int t = hb0 + lane; t < hb1; t += 64) {
+              T *slot = &xs[(size_t)(a.smax + t) * KT];
+              if (is_mark(*slot)) {
+                const int id = lhalo[t];
+                const T v = (unsigned)id < (unsigned)a.n
+                                ? ld_dev(&a.X[(int64_t)id * a.rs + (int64_t)c0 * a.cs])
+                                : T(0);
+                *slot = v;
+                marked |= gave_up ? false : is_mark(v);
+              }
+            }
+            wave_lds_sync();
+            if (!__any(marked)) {
+              if (loaded == 0 && lane == 0) trace_mark(a.trace, a.trace_cap, task, 1);
+              ++loaded;
+              if (lane == 0)
+                __hip_atomic_store(&s_ctl[9], loaded, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+              moved = true;
+            }
+          }
+          if (moved) {
+            t0 = wall_ticks();
+          } else {
+            __builtin_amdgcn_s_sleep(1);
+            if (!gave_up && wall_ticks() - t0 > a.timeout) {
+              if (lane == 0) atomicOr(&a.state[ST_ERROR], 1);
+              gave_up = true;
+            }
+          }
+        }
+      }
+      // 3. (without marks) rounds: issue the stores of every band all compute
+      // waves have finished and the halo loads of every band whose waits are
+      // met, wait once for all of them, then publish and signal
+      int issued = 0, stored = MK ? nb : 0;
       while (stored < nb) {
         int done = nb;
 #pragma unroll
@@ -795,68 +852,6 @@ __global__ __launch_bounds__(64 * (NC + 1)) void k_regions_mw(RegionArgs<T> a) {
               st_dev(&a.X[(int64_t)id * a.rs + (int64_t)(c0 + c) * a.cs], xs[t]);
           }
           issued = done;
-        }
-        if constexpr (MK) {
-          // stores are not waited for: a reader re-loads what is still marked
-          stored = issued;
-          bool moved = stores;
-          if (loaded < nb) {
-            if (!halo_in) {
-              // once every region read has marked its rows (a region stays
-              // marked for the rest of the launch), every halo value of the
-              // task is loaded at once; values still marked are loaded again
-              // band by band below
-              if (gave_up || all_marked(ldep, nd, a.tflags, base, a.groups, g, a.R)) {
-                if (nh > 0)
-                  load_rows<T, KT, ES, true, 1>(xs + (size_t)a.smax * KT, a.X, lhalo, nh, kc, c0,
-                                                a.rs, a.cs, a.n, 0);
-                vm_wait();
-                wave_lds_sync();
-                halo_in = true;
-                moved = true;
-              }
-            }
-            if (halo_in) {
-              const int hb0 = lhb[loaded], hb1 = lhb[loaded + 1];
-              bool marked = false;
-              for (int t = hb0 + lane; t < hb1; t += 64) {
-                T *slot = &xs[(size_t)(a.smax + t) * KT];
-                if (is_mark(*slot)) {
-                  const int id = lhalo[t];
-                  const T v = (unsigned)id < (unsigned)a.n
-                                  ? ld_dev(&a.X[(int64_t)id * a.rs + (int64_t)c0 * a.cs])
-                                  : T(0);
-                  *slot = v;
-                  marked |= gave_up ? false : is_mark(v);
-                }
-              }
-              wave_lds_sync();
-              if (!__any(marked)) {
-                if (loaded == 0 && lane == 0) trace_mark(a.trace, a.trace_cap, task, 1);
-                ++loaded;
-                if (lane == 0)
-                  __hip_atomic_store(&s_ctl[9], loaded, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_WORKGROUP);
-                moved = true;
-              }
-            }
-          }
-          if (moved) {
-            t0 = wall_ticks();
-          } else if (a.gL && graded < stored) {
-            // grad-L only in rounds that would otherwise wait: a band a
-            // round, off the path of the halo values and the stores
-            grad_bands<T>(a.gL, xs, reinterpret_cast<const T *>(smem + a.xfb), rb, L, lsl, lband,
-                          graded, graded + 1, nr, ns, ne);
-            ++graded;
-          } else {
-            __builtin_amdgcn_s_sleep(1);
-            if (!gave_up && wall_ticks() - t0 > a.timeout) {
-              if (lane == 0) atomicOr(&a.state[ST_ERROR], 1);
-              gave_up = true;
-            }
-          }
-          continue;
         }
         int ready = loaded;
         if (loaded < nb) {
@@ -895,15 +890,42 @@ __global__ __launch_bounds__(64 * (NC + 1)) void k_regions_mw(RegionArgs<T> a) {
           }
         }
       }
-      if constexpr (MK)
-        if (a.gL && graded < nb)
-          grad_bands<T>(a.gL, xs, reinterpret_cast<const T *>(smem + a.xfb), rb, L, lsl, lband,
-                        graded, nb, nr, ns, ne);
       // the next task and its header
       const int nx = __builtin_amdgcn_readlane(ticket, 0);
       if (lane < 8) s_ctl[1 + lane] = nx < ntasks ? a.head[8 * (nx / a.groups) + lane] : 0;
       if (lane == 0) s_ctl[0] = nx;
       if (lane == 0) trace_mark(a.trace, a.trace_cap, task, 2);
+    } else if (storew) {
+      // the rows of every band the compute waves have finished (a value is
+      // stored after the mark of its row: the band's halo was loaded after the
+      // marks were), grad-L a band at a time between them; the compute waves'
+      // own waits end, so these do
+      int issued = 0, graded = 0;
+      while (issued < nb) {
+        int done = nb;
+#pragma unroll
+        for (int w = 0; w < NC; ++w) done = min(done, lds_get<int>(&s_ctl[10 + w]));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (done > issued) {
+          const int r0 = min(max(lsl[min(lband[issued], ns)], 0), nr);
+          const int r1 = min(max(lsl[min(lband[done], ns)], 0), nr);
+          for (int t = r0 + lane; t < r1; t += 64) {
+            const int id = lrow[t];
+            if ((unsigned)id < (unsigned)a.n)
+              st_dev(&a.X[(int64_t)id * a.rs + (int64_t)c0 * a.cs], xs[t]);
+          }
+          issued = done;
+        } else if (a.gL && graded < issued) {
+          grad_bands<T>(a.gL, xs, reinterpret_cast<const T *>(smem + a.xfb), rb, L, lsl, lband,
+                        graded, graded + 1, nr, ns, ne);
+          ++graded;
+        } else {
+          __builtin_amdgcn_s_sleep(1);
+        }
+      }
+      if (a.gL && graded < nb)
+        grad_bands<T>(a.gL, xs, reinterpret_cast<const T *>(smem + a.xfb), rb, L, lsl, lband,
+                      graded, nb, nr, ns, ne);
     } else {
       // compute wave `wid`: columns wid*CPL .. (column split) of every row
       for (int b = 0; b < nb; ++b) {
@@ -987,7 +1009,7 @@ int region_launch(symamd_handle h, symamd_plan p, const RegionPlan &rp, const vo
     kfn = (const void *)&k_regions_mw<T, KT, ES, NW, KT == 1>;
   else
     kfn = (const void *)&k_regions<T, KT, ES, NW>;
-  constexpr int WAVES = NW + (MW ? 1 : 0);
+  constexpr int WAVES = NW + (MW ? 1 : 0) + (MW && KT == 1 ? 1 : 0);  // see k_regions_mw
   // grad-L from the solve: marked single right-hand side kernel only
   const bool grad = MW && KT == 1 && d_gL && rp.gp;
   const size_t lds_base = region_image_bytes(rp, KT, (int)sizeof(T));
