@@ -41,9 +41,9 @@
 // Measured on the 13-level nested-dissection-shaped factor (8,191 supernodes
 // up to 512 wide, 36 M values), forward + transposed, in ms: one right-hand
 // side 1.36 + 3.06 with one wavefront per top, 0.45 + 0.65 with a workgroup,
-// 0.32 + 0.44 with the quotients from reciprocals, the whole diagonal block
+// 0.32 + 0.43 with the quotients from reciprocals, the whole diagonal block
 // in flight, gathered lists and turned tiles; 32 right-hand sides 4.6 + 6.9,
-// 1.71 + 1.50, 1.34 + 1.30.
+// 1.71 + 1.50, 1.34 + 1.27.
 #include <algorithm>
 #include <vector>
 
@@ -675,15 +675,24 @@ __device__ __forceinline__ void load_turn(double (&m)[16], const double *M, int 
   for (int j = 0; j < 16; ++j) m[j] = R[(int64_t)min(c0 + 4 * j + (lane >> 4), w - 1) * nr];
 }
 
-// The block turned: v[r] = row r of the lane's column.  tile: the wave's LDS.
-__device__ __forceinline__ void turn(double (&v)[16], const double (&m)[16], double *tile,
-                                     int lane) {
+// The block turned: v[r] = row r of the lane's column.  tile: the wave's LDS,
+// whose operations complete in the order a wave issues them.
+__device__ __forceinline__ void turn_in(const double (&m)[16], double *tile, int lane) {
+  asm volatile("" ::: "memory");
 #pragma unroll
   for (int j = 0; j < 16; ++j) tile[(4 * j + (lane >> 4)) * SN_PITCH_T + (lane & 15)] = m[j];
-  wave_lds_sync();
+  asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void turn_out(double (&v)[16], const double *tile, int lane) {
+  asm volatile("" ::: "memory");
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = tile[lane * SN_PITCH_T + r];
-  wave_lds_sync();
+  asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void turn(double (&v)[16], const double (&m)[16], double *tile,
+                                     int lane) {
+  turn_in(m, tile, lane);
+  turn_out(v, tile, lane);
 }
 
 // Eight rows c0 .. c0+7 of a wave's own columns (lanes lb .. lb+7).
@@ -710,46 +719,66 @@ __device__ __forceinline__ void top_group_t(double (&acc)[KT], double (&res)[KT]
   for (int c = 0; c < KT; ++c) res[c] = 0.0;
   hold<KT>(acc);
   const int last = (w - 1) >> 4;
-  for (int b0 = last; b0 >= 4 * g; b0 -= 2) {
+  auto eight = [&](const double (&v)[16], int b, int h) {
+    const int c0 = 16 * b + 8 * h;
+    double v8[8];
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int b = b0 - q;
-      if (b >= 4 * g) {
-        double v[16];
-        turn(v, m[q], tile, lane);
-        load_turn(m[q], M, max(16 * (b - 2), 0), 64 * g, w, nr, lane);
+    for (int j = 0; j < 8; ++j) v8[j] = v[8 * h + j];
+    if (b >= 4 * g + 4) {
+      if (c0 < w) {
+        lds_wait(prog, w - c0, seen);
+        double xv[8][KT];
 #pragma unroll
-        for (int h = 1; h >= 0; --h) {
-          const int c0 = 16 * b + 8 * h;
-          double v8[8];
+        for (int j = 0; j < 8; ++j)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v8[j] = v[8 * h + j];
-          if (b >= 4 * g + 4) {
-            if (c0 < w) {
-              lds_wait(prog, w - c0, seen);
-              double xv[8][KT];
+          for (int c = 0; c < KT; ++c) xv[j][c] = xs[min(c0 + j, w - 1) * KT + c];
 #pragma unroll
-              for (int j = 0; j < 8; ++j)
+        for (int j = 7; j >= 0; --j)
+          if (c0 + j < w) {
 #pragma unroll
-                for (int c = 0; c < KT; ++c) xv[j][c] = xs[min(c0 + j, w - 1) * KT + c];
-#pragma unroll
-              for (int j = 7; j >= 0; --j)
-                if (c0 + j < w) {
-#pragma unroll
-                  for (int c = 0; c < KT; ++c) acc[c] = acc[c] - v8[j] * xv[j][c];
-                }
-              hold<KT>(acc);
-            }
-          } else {
-            const int lb = c0 - 64 * g;
-            own_rows<KT>(acc, res, v8, dg, c0, lb, w, C, lane, [&] {
-              if (xs) {
-#pragma unroll
-                for (int c = 0; c < KT; ++c) xs[(64 * g + lane) * KT + c] = res[c];
-                lds_publish(prog, w - c0, lane);
-              }
-            });
+            for (int c = 0; c < KT; ++c) acc[c] = acc[c] - v8[j] * xv[j][c];
           }
+        hold<KT>(acc);
+      }
+    } else {
+      const int lb = c0 - 64 * g;
+      own_rows<KT>(acc, res, v8, dg, c0, lb, w, C, lane, [&] {
+        if (xs) {
+#pragma unroll
+          for (int c = 0; c < KT; ++c) xs[(64 * g + lane) * KT + c] = res[c];
+          lds_publish(prog, w - c0, lane);
+        }
+      });
+    }
+  };
+  if constexpr (KT < 4) {
+    // the next block is turned while this one is worked on (13-level factor:
+    // 442 -> 433 us; with four columns the registers run out, 1.30 -> 1.42 ms)
+    double va[16], vb[16];
+    turn(va, m[0], tile, lane);
+    load_turn(m[0], M, max(16 * (last - 2), 0), 64 * g, w, nr, lane);
+    auto block = [&](const double (&v)[16], double (&vn)[16], double (&mn)[16], int b) {
+      turn_in(mn, tile, lane);
+      load_turn(mn, M, max(16 * (b - 3), 0), 64 * g, w, nr, lane);
+      eight(v, b, 1);
+      turn_out(vn, tile, lane);
+      eight(v, b, 0);
+    };
+    for (int b = last; b >= 4 * g; b -= 2) {
+      block(va, vb, m[1], b);
+      if (b - 1 >= 4 * g) block(vb, va, m[0], b - 1);
+    }
+  } else {
+    for (int b0 = last; b0 >= 4 * g; b0 -= 2) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int b = b0 - q;
+        if (b >= 4 * g) {
+          double v[16];
+          turn(v, m[q], tile, lane);
+          load_turn(m[q], M, max(16 * (b - 2), 0), 64 * g, w, nr, lane);
+          eight(v, b, 1);
+          eight(v, b, 0);
         }
       }
     }
@@ -1209,8 +1238,8 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
   // columns per tile: a row's entries are loaded once for the columns of a
   // tile, but each step of a top's chain then divides for all of them.  On
   // the 13-level factor, forward + transposed with tiles of 1 / 2 / 4: k = 2
-  // 0.86 / 0.93 / - ms, k = 4 1.11 / 1.05 / 1.32 ms, k = 13 2.30 / 1.78 / 1.83
-  // ms, k = 32 4.94 / 3.17 / 2.64 ms.
+  // 0.86 / 0.93 / - ms, k = 4 1.11 / 1.02 / 1.32 ms, k = 13 2.30 / 1.76 / 1.83
+  // ms, k = 32 4.94 / 3.17 / 2.61 ms.
   const int kt = k < 4 ? 1 : k < 16 ? 2 : 4;
   const int tiles = (k + kt - 1) / kt;
   // temporaries and tags for the tiles' columns
