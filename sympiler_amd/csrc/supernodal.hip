@@ -1111,9 +1111,11 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
   // the rows' lists, in ascending supernode order, and the place in T of each
   // row below: entry j of the rows one wave gathers (64 consecutive ones of a
   // supernode) lies side by side, lists padded to the longest; rows of very
-  // uneven lists (padding past three entries in four) keep theirs contiguous
+  // uneven lists (padding past three entries in four), and all rows where that
+  // padding could pass 32-bit places, keep theirs contiguous
   std::vector<int> tdst(tb[m] > 0 ? tb[m] : 1), rowb(tb[m] > 0 ? tb[m] : 1);
   std::vector<int4> list(n > 0 ? n : 1, make_int4(0, 0, 0, 0));
+  const bool pad = 4 * (int64_t)cnt[n] <= INT_MAX;
   int64_t tcount = 0;
   for (int i = 0; i < m; ++i)
     for (int r0 = h_sup[i]; r0 < h_sup[i + 1]; r0 += 64) {
@@ -1121,14 +1123,12 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
       const int64_t total = cnt[r1] - cnt[r0];
       int64_t longest = 0;
       for (int r = r0; r < r1; ++r) longest = std::max<int64_t>(longest, cnt[r + 1] - cnt[r]);
-      const bool side = longest * (r1 - r0) <= 4 * total;
+      const bool side = pad && longest * (r1 - r0) <= 4 * total;
       for (int r = r0; r < r1; ++r)
         if (cnt[r + 1] > cnt[r])
           list[r] = make_int4((int)(tcount + (side ? r - r0 : cnt[r] - cnt[r0])), 0,
                               side ? r1 - r0 : 1, 0);
       tcount += side ? longest * (r1 - r0) : total;
-      if (tcount > INT_MAX)
-        return fail(SYMAMD_ERR_NOT_SUPPORTED, "supernodal analyze: over 2^31 temporaries");
     }
   std::vector<int> owner(n);
   for (int i = 0; i < m; ++i)
