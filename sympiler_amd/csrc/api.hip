@@ -75,8 +75,11 @@ void free_plan_arrays(symamd_plan p) {
 // average; then enough lanes that a typical row takes two steps and the
 // longest about eight (launches clip lanes x column tile to 64).  Measured on
 // the Zipf(1.8) n = 1e6 matrix (average 8.7 entries, longest 257) with the
-// sync-free executor: lanes 4 / 32 at k = 1: 11.5 / 4.3 ms; lanes 1 / 8 at
-// k = 8: 30.8 / 5.7 ms; lanes 1 / 2 at k = 32: 33.2 / 16.6 ms.
+// units of the sync-free executor: lanes 4 / 32 at k = 1: 11.5 / 4.3 ms; lanes
+// 1 / 8 at k = 8: 30.8 / 5.7 ms; lanes 1 / 2 at k = 32: 33.2 / 16.6 ms.  Where
+// the choice is more than one lane, sync-free solves run on the row executor
+// (rows_exec.hip), which takes 0.64 / 0.8 / 1.4 ms at k = 1 / 8 / 32 there and
+// picks the lanes row by row.
 Choice heuristic(symamd_plan p, int k) {
   (void)k;
   Choice c;

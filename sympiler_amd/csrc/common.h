@@ -486,8 +486,8 @@ int prepare_workspace(symamd_handle h, symamd_plan p, int k);
 int split_threshold(symamd_handle h, int kt);
 // Row executor (rows_exec.hip): sync-free solves with several lanes per row.
 bool rows_path(symamd_handle h, symamd_plan p, int k, int exec, int lanes, int tile);
-// d_ws of at least `bytes`.
-int plan_workspace(symamd_plan p, size_t bytes);
+// d_ws of at least `bytes`; a solve being captured keeps the one it uses.
+int plan_workspace(symamd_handle h, symamd_plan p, size_t bytes);
 int prepare_rows(symamd_handle h, symamd_plan p, int k, bool turn);
 int launch_rows(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld, int64_t rs,
                 int64_t cs, bool turn);

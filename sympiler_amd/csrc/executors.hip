@@ -33,11 +33,13 @@
 // Executors
 //   LEVELSET  one launch per level, one wave per unit; plain loads and
 //             stores (kernel boundaries order the levels).
-//   SYNCFREE  one persistent launch.  Units are dealt to waves round-robin
-//             from a cooperative launch (all waves co-resident), or taken
-//             from a ticket counter when the launch is captured in a graph;
-//             either way every unit a wave waits on is held by a running
-//             wave that reaches it first, so the grid cannot deadlock.
+//   SYNCFREE  one persistent launch (with one lane per row, or without the
+//             marked protocol; several lanes per row run in
+//             rows_exec.hip).  Units are dealt to waves round-robin from a
+//             cooperative launch (all waves co-resident), or taken from a
+//             ticket counter when the launch is captured in a graph; either
+//             way every unit a wave waits on is held by a running wave that
+//             reaches it first, so the grid cannot deadlock.
 //             Waits are bounded by a watchdog on the 100 MHz clock that
 //             records an error and lets the wave proceed, so every wave
 //             exits.
@@ -997,12 +999,13 @@ int prepare_workspace(symamd_handle h, symamd_plan p, int k) {
     // what was built serves solves on any stream from here on
     SYMAMD_HIP(hipStreamSynchronize(h->stream));
   }
-  return plan_workspace(p, (size_t)p->n * k * (p->dtype == SYMAMD_F64 ? 8 : 4));
+  return plan_workspace(h, p, (size_t)p->n * k * (p->dtype == SYMAMD_F64 ? 8 : 4));
 }
 
 // Grows the plan's workspace.  One that a captured graph holds stays until
 // the plan is destroyed.
-int plan_workspace(symamd_plan p, size_t bytes) {
+int plan_workspace(symamd_handle h, symamd_plan p, size_t bytes) {
+  if (capturing(h->stream)) p->ws_captured = true;
   if (bytes <= p->ws_bytes) return SYMAMD_OK;
   void *ws = nullptr;
   if (!p->ws_captured && p->d_ws) {

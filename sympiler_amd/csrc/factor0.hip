@@ -611,7 +611,7 @@ int launch_factor0(symamd_handle h, symamd_plan p, int64_t nnz, FactorArgs a, Fa
   if (!p->d_ic0_bad) SYMAMD_HIP(hipMalloc(&p->d_ic0_bad, sizeof(int)));
   double *copy = nullptr;
   if (a.Ax == a.Lx) {
-    SYMAMD_TRY(plan_workspace(p, sizeof(double) * (size_t)nnz));
+    SYMAMD_TRY(plan_workspace(h, p, sizeof(double) * (size_t)nnz));
     copy = (double *)p->d_ws;
   }
   k_factor0_begin<<<(unsigned)std::min<int64_t>(std::max<int64_t>((nnz + 255) / 256, 1), 8192),

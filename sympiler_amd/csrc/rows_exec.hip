@@ -426,7 +426,7 @@ int prepare_rows(symamd_handle h, symamd_plan p, int k, bool turn) {
   RowSchedule *s = nullptr;
   int rc = rows_schedule(h, p, rows_cols(k), &s);
   if (rc == SYMAMD_OK)
-    rc = plan_workspace(p, (size_t)p->n * k * (turn ? 2 : 1) * (p->dtype == SYMAMD_F64 ? 8 : 4));
+    rc = plan_workspace(h, p, (size_t)p->n * k * (turn ? 2 : 1) * (p->dtype == SYMAMD_F64 ? 8 : 4));
   if (rc == SYMAMD_ERR_ALLOC) p->rows_off = true;
   return rc;
 }

@@ -76,3 +76,31 @@ def test_captured_solve_keeps_its_workspace(dev):
         g.launch()
         plan.check()
         assert rel_err(x.cpu().numpy(), want[c]) <= 1e-12
+
+
+def test_solve_captured_by_the_caller_keeps_its_workspace(dev):
+    """The same with a capture the caller makes on the handle's stream."""
+    import torch
+    Lp, Li, Lx = matrix()
+    n = len(Lp) - 1
+    B = W.uniform(19, 0, n * 32).reshape(32, n)
+    want = oracle.sptrsm_csr(Lp, Li, Lx, B)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        plan = sa.Plan(*to_dev(Lp, Li, Lx), handle=sa.Handle(stream=stream))
+        plan.set_lanes(2)
+        x = to_dev(B[0].copy())
+        plan.solve(x, executor="syncfree")  # builds the schedule
+        plan.check()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            plan.solve(x, executor="syncfree")
+        for c in range(3):
+            X = to_dev(B.copy())
+            plan.solve(X, executor="syncfree")
+            plan.check()
+            assert rel_err(X.cpu().numpy(), want) <= 1e-12
+            x.copy_(to_dev(B[c].copy()))
+            g.replay()
+            plan.check()
+            assert rel_err(x.cpu().numpy(), want[c]) <= 1e-12
