@@ -609,6 +609,10 @@ int launch_factor0(symamd_handle h, symamd_plan p, int64_t nnz, FactorArgs a, Fa
   UnitSet *us = nullptr;
   SYMAMD_TRY(plan_units(h, p, 64, false, &us));
   if (!p->d_ic0_bad) SYMAMD_HIP(hipMalloc(&p->d_ic0_bad, sizeof(int)));
+  a.perm = p->d_perm;
+  a.ub = us->d_ub;
+  a.U = us->count;
+  SYMAMD_TRY(factor_pack<MODE>(h, a, pack));  // before A's place is marked: it can fail
   double *copy = nullptr;
   if (a.Ax == a.Lx) {
     SYMAMD_TRY(plan_workspace(h, p, sizeof(double) * (size_t)nnz));
@@ -618,12 +622,8 @@ int launch_factor0(symamd_handle h, symamd_plan p, int64_t nnz, FactorArgs a, Fa
                     256, 0, h->stream>>>(nnz, a.Ax, copy, a.Lx, p->d_ic0_bad);
   SYMAMD_HIP(hipGetLastError());
   if (copy) a.Ax = copy;
-  a.perm = p->d_perm;
-  a.ub = us->d_ub;
   a.state = p->d_state;
   a.bad = p->d_ic0_bad;
-  a.U = us->count;
-  SYMAMD_TRY(factor_pack<MODE>(h, a, pack));
   a.poff = pack.d_off;
   a.pwide = pack.d_wide;
   a.pdata = pack.d_data;
