@@ -331,6 +331,7 @@ int rows_schedule(symamd_handle h, symamd_plan p, int C, RowSchedule **out) {
   s.tickets = (int)(item.size() / W);
   if (hipMalloc(&s.d_rec, sizeof(int4) * rec.size()) != hipSuccess ||
       hipMalloc(&s.d_item, sizeof(int4) * std::max<size_t>(item.size(), 1)) != hipSuccess) {
+    (void)hipGetLastError();
     if (s.d_rec) (void)hipFree(s.d_rec);
     return fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", n);
   }
