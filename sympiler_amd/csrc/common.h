@@ -549,6 +549,10 @@ int launch_grad_l(symamd_handle h, symamd_plan p, const void *d_X, const void *d
 // the region's and its halo's values of one column group per row), unless
 // the handle sets one.
 int region_cap(symamd_handle h, symamd_plan p, int k);
+// Over 16 tasks of 1024 rows per CU: single right-hand sides take smaller ones.
+inline bool large_for_regions(symamd_handle h, symamd_plan p) {
+  return p->n > 16 * 1024 * h->num_cus;
+}
 // The region cap the tuner chose for k right-hand sides (either layout), or 0.
 int tuned_region_cap(symamd_plan p, int k);
 int region_band(symamd_handle h, int k);

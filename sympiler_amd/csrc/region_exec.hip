@@ -1132,7 +1132,7 @@ int region_cap(symamd_handle h, symamd_plan p, int k) {
   if (h->region_cap > 0) return h->region_cap;
   const int tuned = p ? tuned_region_cap(p, k) : 0;
   if (tuned > 0) return tuned;
-  if (k == 1 && h->region_mw) return !p || p->n <= 16 * 1024 * h->num_cus ? 1024 : 384;
+  if (k == 1 && h->region_mw) return p && large_for_regions(h, p) ? 384 : 1024;
   return task_cols(k) == KG_MAX && region_waves(h, k) == 1 ? 256 : 512;
 }
 
