@@ -421,6 +421,8 @@ struct symamd_snplan_s {
   int *d_unit = nullptr, *d_dlist = nullptr, *d_tunit = nullptr, *d_tdlist = nullptr;
   double *d_T = nullptr;
   int *d_flags = nullptr, *d_state = nullptr;
+  bool captured = false;       // a caller's graph reads d_T and d_flags: replaced ones are kept
+  std::vector<void *> retired;
 };
 
 struct symamd_graph_s {
@@ -430,6 +432,13 @@ struct symamd_graph_s {
 };
 
 namespace symamd {
+
+// Whether work issued on the stream is being recorded into a graph.
+inline bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) return false;
+  return st != hipStreamCaptureStatusNone;
+}
 
 // Ensures the unit partition with `rows` rows per unit exists with its
 // dependency lists, for the forward solve or (adjoint) the transposed one.

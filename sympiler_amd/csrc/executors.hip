@@ -650,12 +650,6 @@ int resident_grid(symamd_handle h, const void *kernel, int units) {
   return (int)(want < cap ? want : cap);
 }
 
-bool capturing(hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess) return false;
-  return st != hipStreamCaptureStatusNone;
-}
-
 // Launch a persistent kernel.  Plans with a region order use the owner
 // schedule on every co-resident wave (cooperative launch); otherwise units
 // are dealt round-robin (cooperative) or, inside graph capture or when

@@ -532,12 +532,6 @@ __global__ __launch_bounds__(256) void k_factor0_begin(int64_t nnz, const double
   }
 }
 
-bool stream_capturing(hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess) return false;
-  return st != hipStreamCaptureStatusNone;
-}
-
 // Device buffers released on every exit path.
 struct Scratch {
   std::vector<void *> ptrs;
@@ -638,7 +632,7 @@ int launch_factor0(symamd_handle h, symamd_plan p, int64_t nnz, FactorArgs a, Fa
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(a.U, cap));
   a.total_waves = grid;
   bool launched = false;
-  if (!stream_capturing(h->stream) && !h->force_tickets) {
+  if (!capturing(h->stream) && !h->force_tickets) {
     a.ticketed = 0;
     void *args[] = {&a};
     if (hipLaunchCooperativeKernel(kfn, dim3(grid), dim3(64), args, 0, h->stream) ==

@@ -1242,8 +1242,13 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
   // ms, k = 32 4.94 / 3.17 / 2.61 ms.
   const int kt = k < 4 ? 1 : k < 16 ? 2 : 4;
   const int tiles = (k + kt - 1) / kt;
-  // temporaries and tags for the tiles' columns
+  // temporaries and tags for the tiles' columns; those that a caller's graph
+  // reads stay until the plan is destroyed
+  const bool cap = capturing(h->stream);
   if (tiles * kt > q->kcap) {
+    if (cap)
+      return fail(SYMAMD_ERR_NOT_SUPPORTED,
+                  "supernodal temporaries for %d columns not prepared before capture", k);
     double *T = nullptr;
     int *flags = nullptr;
     const int64_t cols = (int64_t)tiles * kt;
@@ -1257,12 +1262,18 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
     // cleared tags read as "not ready" in every epoch
     SYMAMD_HIP(hipMemsetAsync(flags, 0, sizeof(int) * nt * cols, h->stream));
     SYMAMD_HIP(hipStreamSynchronize(h->stream));
-    if (q->d_T) (void)hipFree(q->d_T);
-    if (q->d_flags) (void)hipFree(q->d_flags);
+    for (void *old : {(void *)q->d_T, (void *)q->d_flags}) {
+      if (q->captured)
+        q->retired.push_back(old);
+      else
+        (void)hipFree(old);
+    }
+    q->captured = false;
     q->d_T = T;
     q->d_flags = flags;
     q->kcap = (int)cols;
   }
+  if (cap) q->captured = true;
   SnArgs a;
   a.unit = reinterpret_cast<const SnUnit *>(transposed ? q->d_tunit : q->d_unit);
   a.Lx = d_Lx;
@@ -1310,6 +1321,7 @@ void sn_destroy(symamd_snplan_s *q) {
                   q->d_tunit, q->d_tdlist, q->d_T,    q->d_flags, q->d_state};
   for (void *x : ptrs)
     if (x) (void)hipFree(x);
+  for (void *x : q->retired) (void)hipFree(x);
   delete q;
 }
 
