@@ -1256,6 +1256,7 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
     const int64_t nt = 4 * (int64_t)std::max(1, std::max(q->tickets, q->ttickets));
     if (hipMalloc(&T, sizeof(double) * tc * cols) != hipSuccess ||
         hipMalloc(&flags, sizeof(int) * nt * cols) != hipSuccess) {
+      (void)hipGetLastError();
       if (T) (void)hipFree(T);
       return fail(SYMAMD_ERR_ALLOC, "supernodal temporaries for %d columns", k);
     }

@@ -1,6 +1,7 @@
 """Supernodal solves recorded by the caller: the temporaries and tags that the
 graph reads outlive later, wider solves on the same plan; a wider solve is
-refused while recording and leaves the recording whole."""
+refused while recording and leaves the recording whole; and a block whose
+temporaries fit no GPU leaves nothing behind for the next solve."""
 import numpy as np
 import pytest
 
@@ -44,3 +45,24 @@ def test_solve_captured_by_the_caller_keeps_its_temporaries(dev, direction):
             for i in range(k):
                 assert bitwise_equal(X[i].cpu().numpy(), want[i])
             del filler
+
+
+def test_solve_after_a_block_that_did_not_fit(dev):
+    """A dense triangle of 2000 one-column supernodes has 2 M temporaries per
+    column: 20000 columns of them (320 GB) fit no GPU."""
+    import torch
+    n, k = 2000, 20000
+    sup, nrows = np.arange(n + 1, dtype=np.int32), np.arange(n, 0, -1, dtype=np.int32)
+    Lp = np.concatenate([[0], np.cumsum(nrows)]).astype(np.int32)
+    Li = np.concatenate([np.arange(i, n) for i in range(n)]).astype(np.int32)
+    Lx = W.uniform(42, 0, len(Li)) / n
+    Lx[Lp[:-1]] = 1.0 + Lx[Lp[:-1]]
+    b = W.uniform(43, 0, n)
+    plan = sa.SupernodalPlan(sup, nrows, Lp, Li)
+    dLx = to_dev(Lx)
+    with pytest.raises(sa.SymAmdError, match="temporaries"):
+        plan.solve(dLx, torch.zeros(k, n, dtype=torch.float64, device="cuda"))
+    x = to_dev(b.copy())
+    plan.solve(dLx, x)
+    plan.check()
+    assert bitwise_equal(x.cpu().numpy(), oracle.sptrsv_csc_block(sup, nrows, Lp, Li, Lx, b))
