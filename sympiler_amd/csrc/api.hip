@@ -325,9 +325,10 @@ int prepare_solve(symamd_handle h, symamd_plan p, int k, int layout, const Choic
     SYMAMD_TRY(split_lists(h, p, split_threshold(h, tile_cols(k, c.tile)), &sl));
     return through_workspace(h, k, layout) ? prepare_workspace(h, p, k) : SYMAMD_OK;
   }
-  if (rows_path(h, p, k, c.exec == SYMAMD_EXEC_REGIONS ? SYMAMD_EXEC_SYNCFREE : c.exec, c.lanes,
-                c.tile)) {
-    const int rc = prepare_rows(h, p, k, through_workspace(h, k, layout));
+  const bool turn = through_workspace(h, k, layout);
+  if (rows_path(h, p, k, turn, c.exec == SYMAMD_EXEC_REGIONS ? SYMAMD_EXEC_SYNCFREE : c.exec,
+                c.lanes, c.tile)) {
+    const int rc = prepare_rows(h, p, k, turn);
     if (rc != SYMAMD_ERR_ALLOC) return rc;  // without the memory: the unit executor
   }
   UnitSet *us = nullptr;
@@ -351,9 +352,10 @@ int run_solve(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld,
                                              : launch_regions(h, p, d_B, k, rs, cs);
     exec = SYMAMD_EXEC_SYNCFREE;
   }
-  if (rows_path(h, p, k, exec, lanes, tile))
-    return launch_rows(h, p, d_B, k, ld, rs, cs, through_workspace(h, k, layout));
-  if (through_workspace(h, k, layout))
+  const bool turn = through_workspace(h, k, layout);
+  if (rows_path(h, p, k, turn, exec, lanes, tile))
+    return launch_rows(h, p, d_B, k, ld, rs, cs, turn);
+  if (turn)
     return launch_forward_ws(h, p, d_B, k, ld, exec, lanes, tile);
   return launch_forward(h, p, d_B, k, rs, cs, exec, lanes, tile);
 }

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <cstddef>
 #include <cstdint>
 #include <cstdio>
 #include <map>
@@ -329,6 +330,7 @@ struct RowSchedule {
   int4 *d_rec = nullptr;
   int4 *d_item = nullptr;
   int tickets = 0;
+  bool failed = false;  // no memory for it: the unit executor
 };
 
 struct symamd_plan_s {
@@ -359,7 +361,7 @@ struct symamd_plan_s {
   std::map<int, SplitLists> split;
   std::map<int, RowSchedule> rows;  // row executor, per column lanes
   bool rows_off = false;            // its workspace did not fit
-  bool ws_captured = false;         // a graph holds d_ws: replaced ones are kept
+  bool ws_captured = false;         // a graph holds d_ws: it is kept when replaced
   std::vector<void *> ws_retired;
   size_t ws_bytes = 0;
   int *d_orp = nullptr;                // caller CSR row pointers, n+1
@@ -440,6 +442,15 @@ inline bool capturing(hipStream_t s) {
   return st != hipStreamCaptureStatusNone;
 }
 
+// Allows this thread allocations, and work on other streams, while a stream is
+// recorded in the global mode (which forbids them to every thread).
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  RelaxedCapture(const RelaxedCapture &) = delete;
+};
+
 // Ensures the unit partition with `rows` rows per unit exists with its
 // dependency lists, for the forward solve or (adjoint) the transposed one.
 int plan_units(symamd_handle h, symamd_plan p, int rows, bool adjoint,
@@ -493,9 +504,11 @@ int prepare_workspace(symamd_handle h, symamd_plan p, int k);
 // columns, and the long-row lists of a threshold (built once per plan and
 // threshold, outside graph capture).
 int split_threshold(symamd_handle h, int kt);
-// Row executor (rows_exec.hip): sync-free solves with several lanes per row.
-bool rows_path(symamd_handle h, symamd_plan p, int k, int exec, int lanes, int tile);
-// d_ws of at least `bytes`; a solve being captured keeps the one it uses.
+// Row executor (rows_exec.hip): sync-free solves with several lanes per row
+// (turn: of a column-major block, through the workspace).
+bool rows_path(symamd_handle h, symamd_plan p, int k, bool turn, int exec, int lanes, int tile);
+// d_ws of at least `bytes`; a solve being captured keeps the one it uses, and
+// may grow it.
 int plan_workspace(symamd_handle h, symamd_plan p, size_t bytes);
 int prepare_rows(symamd_handle h, symamd_plan p, int k, bool turn);
 int launch_rows(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld, int64_t rs,

@@ -979,6 +979,8 @@ int split_lists(symamd_handle h, symamd_plan p, int thr, SplitLists **out) {
 }
 
 int prepare_workspace(symamd_handle h, symamd_plan p, int k) {
+  if ((!p->d_ipos || !p->d_cpos) && capturing(h->stream))
+    return fail(SYMAMD_ERR_NOT_SUPPORTED, "column-major solves not prepared before capture");
   if (!p->d_ipos) {
     UnitSet *us = nullptr;  // building any unit set builds the inverse map
     SYMAMD_TRY(plan_units(h, p, 64, false, &us));
@@ -997,16 +999,20 @@ int prepare_workspace(symamd_handle h, symamd_plan p, int k) {
 }
 
 // Grows the plan's workspace.  One that a captured graph holds stays until
-// the plan is destroyed.
+// the plan is destroyed.  While a caller records the stream the old one stays
+// too (freeing it would wait for the device), and the new one is allocated as
+// outside: a block of another width may be recorded after a narrower solve.
 int plan_workspace(symamd_handle h, symamd_plan p, size_t bytes) {
-  if (capturing(h->stream)) p->ws_captured = true;
+  const bool cap = capturing(h->stream);
+  if (cap && bytes <= p->ws_bytes) p->ws_captured = true;
   if (bytes <= p->ws_bytes) return SYMAMD_OK;
   void *ws = nullptr;
-  if (!p->ws_captured && p->d_ws) {
+  if (!p->ws_captured && !cap && p->d_ws) {
     SYMAMD_HIP(hipFree(p->d_ws));
     p->d_ws = nullptr;
     p->ws_bytes = 0;
   }
+  RelaxedCapture relaxed;
   if (hipMalloc(&ws, bytes) != hipSuccess) {
     (void)hipGetLastError();
     return fail(SYMAMD_ERR_ALLOC, "plan workspace of %zu bytes", bytes);
@@ -1014,6 +1020,7 @@ int plan_workspace(symamd_handle h, symamd_plan p, size_t bytes) {
   if (p->d_ws) p->ws_retired.push_back(p->d_ws);
   p->d_ws = ws;
   p->ws_bytes = bytes;
+  p->ws_captured = cap;
   return SYMAMD_OK;
 }
 

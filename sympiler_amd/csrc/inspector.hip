@@ -762,6 +762,8 @@ int plan_units(symamd_handle h, symamd_plan p, int rows, bool adjoint,
     *out = &it->second;
     return SYMAMD_OK;
   }
+  if (capturing(h->stream))
+    return fail(SYMAMD_ERR_NOT_SUPPORTED, "work units of %d rows not prepared before capture", rows);
   if (adjoint) SYMAMD_TRY(plan_transpose(h, p));
   // units of the forward solve are cut by the entries of the forward copy,
   // those of the transposed solve by the entries of the transposed copy

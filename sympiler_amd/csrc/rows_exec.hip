@@ -32,6 +32,7 @@
 // reference's order, leaves an error against 64 bits 1.6 times the unit
 // executor's, whose lanes sum first too.)
 #include <algorithm>
+#include <new>
 #include <vector>
 
 #include "device.h"
@@ -279,17 +280,14 @@ int rows_cols(int k) { return k == 1 ? 1 : k <= 8 ? 8 : k <= 16 ? 16 : 32; }
 // The schedule for C column lanes: per level the rows a workgroup shares,
 // then the others by descending slices, waves of a ticket filled from one
 // level.
-int rows_schedule(symamd_handle h, symamd_plan p, int C, RowSchedule **out) {
-  auto found = p->rows.find(C);
-  if (found != p->rows.end()) {
-    *out = &found->second;
-    return SYMAMD_OK;
-  }
+int build_rows(symamd_plan p, int C, hipStream_t stream, RowSchedule &s) {
   const int n = p->n, W = rows_waves(C), smax = 64 / C, epl = rows_epl(C);
   std::vector<int> rp(n + 1), perm(n);
-  SYMAMD_HIP(hipStreamSynchronize(h->stream));
-  SYMAMD_HIP(hipMemcpy(rp.data(), p->d_rp, sizeof(int) * (n + 1), hipMemcpyDeviceToHost));
-  SYMAMD_HIP(hipMemcpy(perm.data(), p->d_perm, sizeof(int) * n, hipMemcpyDeviceToHost));
+  SYMAMD_HIP(hipMemcpyAsync(rp.data(), p->d_rp, sizeof(int) * (n + 1), hipMemcpyDeviceToHost,
+                            stream));
+  SYMAMD_HIP(hipMemcpyAsync(perm.data(), p->d_perm, sizeof(int) * n, hipMemcpyDeviceToHost,
+                            stream));
+  SYMAMD_HIP(hipStreamSynchronize(stream));
   int lgmax = 0;
   while ((1 << lgmax) < smax) ++lgmax;
   // class of a row, in solving order: the workgroup's (0), lgmax .. 0 slices
@@ -327,24 +325,51 @@ int rows_schedule(symamd_handle h, symamd_plan p, int C, RowSchedule **out) {
     while (item.size() % W) item.push_back(make_int4(0, 0, 0, 0));
     at += q1 - q0;
   }
-  RowSchedule s;
   s.tickets = (int)(item.size() / W);
   if (hipMalloc(&s.d_rec, sizeof(int4) * rec.size()) != hipSuccess ||
       hipMalloc(&s.d_item, sizeof(int4) * std::max<size_t>(item.size(), 1)) != hipSuccess) {
     (void)hipGetLastError();
-    if (s.d_rec) (void)hipFree(s.d_rec);
     return fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", n);
   }
-  if (hipMemcpy(s.d_rec, rec.data(), sizeof(int4) * rec.size(), hipMemcpyHostToDevice) !=
-          hipSuccess ||
-      hipMemcpy(s.d_item, item.data(), sizeof(int4) * item.size(), hipMemcpyHostToDevice) !=
-          hipSuccess) {
-    (void)hipFree(s.d_rec);
-    (void)hipFree(s.d_item);
-    return fail(SYMAMD_ERR_HIP, "row schedule: copy failed");
-  }
-  *out = &(p->rows[C] = s);
+  SYMAMD_HIP(hipMemcpyAsync(s.d_rec, rec.data(), sizeof(int4) * rec.size(),
+                            hipMemcpyHostToDevice, stream));
+  SYMAMD_HIP(hipMemcpyAsync(s.d_item, item.data(), sizeof(int4) * item.size(),
+                            hipMemcpyHostToDevice, stream));
+  SYMAMD_HIP(hipStreamSynchronize(stream));
   return SYMAMD_OK;
+}
+
+// The schedule, built on first use.  While a caller records the handle's
+// stream it is built on a stream of its own (rows_path has seen that one was
+// built before, so the plan's arrays are in place).  Without the memory the
+// plan remembers so, for this number of column lanes.
+int rows_schedule(symamd_handle h, symamd_plan p, int C, RowSchedule **out) {
+  auto found = p->rows.find(C);
+  if (found == p->rows.end()) {
+    const bool cap = capturing(h->stream);
+    RelaxedCapture relaxed;
+    hipStream_t own = nullptr;
+    if (cap) SYMAMD_HIP(hipStreamCreateWithFlags(&own, hipStreamNonBlocking));
+    RowSchedule s;
+    int rc;
+    try {
+      rc = build_rows(p, C, cap ? own : h->stream, s);
+    } catch (const std::bad_alloc &) {
+      rc = fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", p->n);
+    }
+    if (own) (void)hipStreamDestroy(own);
+    if (rc != SYMAMD_OK) {
+      if (s.d_rec) (void)hipFree(s.d_rec);
+      if (s.d_item) (void)hipFree(s.d_item);
+      if (rc != SYMAMD_ERR_ALLOC) return rc;
+      s = RowSchedule();
+      s.failed = true;
+    }
+    found = p->rows.emplace(C, s).first;
+  }
+  *out = &found->second;
+  return found->second.failed ? fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", p->n)
+                              : SYMAMD_OK;
 }
 
 template <typename T, int C>
@@ -412,22 +437,32 @@ int launch_rows_t(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld, 
 
 }  // namespace
 
+// Bytes of the workspace: the right-hand sides, and for turned blocks the
+// solution.
+static size_t rows_bytes(symamd_plan p, int k, bool turn) {
+  return (size_t)p->n * k * (turn ? 2 : 1) * (p->dtype == SYMAMD_F64 ? 8 : 4);
+}
+
 // Whether a sync-free solve of k right-hand sides runs here: several lanes
 // per row beside the column tile (one lane per row keeps the reference's
 // order in every row, which the unit executor does), the marked protocol on,
-// no unit trace, and memory for the workspace.
-bool rows_path(symamd_handle h, symamd_plan p, int k, int exec, int lanes, int tile) {
-  return exec == SYMAMD_EXEC_SYNCFREE && lanes > 1 && 2 * tile_cols(k, tile) <= 64 &&
-         !h->unmarked && !h->trace && !p->rows_off;
+// no unit trace, and memory for the schedule and the workspace.  A solve being
+// recorded by the caller needs an earlier one here, as the unit executor does.
+bool rows_path(symamd_handle h, symamd_plan p, int k, bool turn, int exec, int lanes, int tile) {
+  if (exec != SYMAMD_EXEC_SYNCFREE || lanes < 2 || 2 * tile_cols(k, tile) > 64 || h->unmarked ||
+      h->trace || p->rows_off)
+    return false;
+  const auto s = p->rows.find(rows_cols(k));
+  if (s != p->rows.end()) return !s->second.failed;
+  return !p->rows.empty() || !capturing(h->stream);
 }
 
-// The schedule and the workspace (the right-hand sides, and for turned blocks
-// the solution), before any launch or capture.
+// The schedule and the workspace, before any launch or capture.
 int prepare_rows(symamd_handle h, symamd_plan p, int k, bool turn) {
   RowSchedule *s = nullptr;
-  int rc = rows_schedule(h, p, rows_cols(k), &s);
-  if (rc == SYMAMD_OK)
-    rc = plan_workspace(h, p, (size_t)p->n * k * (turn ? 2 : 1) * (p->dtype == SYMAMD_F64 ? 8 : 4));
+  SYMAMD_TRY(rows_schedule(h, p, rows_cols(k), &s));
+  const size_t bytes = rows_bytes(p, k, turn);
+  const int rc = plan_workspace(h, p, bytes);
   if (rc == SYMAMD_ERR_ALLOC) p->rows_off = true;
   return rc;
 }
