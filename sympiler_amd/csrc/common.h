@@ -360,7 +360,7 @@ struct symamd_plan_s {
   // split level executor, per long-row threshold
   std::map<int, SplitLists> split;
   std::map<int, RowSchedule> rows;  // row executor, per column lanes
-  bool rows_off = false;            // its workspace did not fit
+  size_t rows_limit = SIZE_MAX;     // a workspace of this size did not fit: smaller ones only
   bool ws_captured = false;         // a graph holds d_ws: it is kept when replaced
   std::vector<void *> ws_retired;
   size_t ws_bytes = 0;

@@ -450,20 +450,21 @@ static size_t rows_bytes(symamd_plan p, int k, bool turn) {
 // recorded by the caller needs an earlier one here, as the unit executor does.
 bool rows_path(symamd_handle h, symamd_plan p, int k, bool turn, int exec, int lanes, int tile) {
   if (exec != SYMAMD_EXEC_SYNCFREE || lanes < 2 || 2 * tile_cols(k, tile) > 64 || h->unmarked ||
-      h->trace || p->rows_off)
+      h->trace || rows_bytes(p, k, turn) >= p->rows_limit)
     return false;
   const auto s = p->rows.find(rows_cols(k));
   if (s != p->rows.end()) return !s->second.failed;
   return !p->rows.empty() || !capturing(h->stream);
 }
 
-// The schedule and the workspace, before any launch or capture.
+// The schedule and the workspace, before any launch or capture.  A workspace
+// that did not fit is not asked for again, nor is a larger one.
 int prepare_rows(symamd_handle h, symamd_plan p, int k, bool turn) {
   RowSchedule *s = nullptr;
   SYMAMD_TRY(rows_schedule(h, p, rows_cols(k), &s));
   const size_t bytes = rows_bytes(p, k, turn);
   const int rc = plan_workspace(h, p, bytes);
-  if (rc == SYMAMD_ERR_ALLOC) p->rows_off = true;
+  if (rc == SYMAMD_ERR_ALLOC) p->rows_limit = bytes;
   return rc;
 }
 
