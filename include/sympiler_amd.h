@@ -491,10 +491,12 @@ int symamd_sn_destroy(symamd_snplan plan);
  * cache keyed by the matrix fingerprint); SYMAMD_EXEC_AUTO then uses it.
  * Candidates: the sync-free unit executor (lanes per row, and for k > 8
  * column tiles of 8 to 32 columns solved as separate work items), the
- * level-set executor replayed from a graph (lanes per row) and the region
- * executor (for one right-hand side at region caps 512 and 1024; the chosen
- * cap also serves the plan's adjoint).  Writes a human-readable summary
- * (may be NULL). */
+ * level-set executor replayed from a graph (lanes per row), the region
+ * executor (for one right-hand side at region caps 512 and 1024, and 384 where
+ * that is the untuned one; the chosen cap also serves the plan's adjoint), the
+ * split level executor and the row executor ("rows" in the summary; sync-free
+ * forward solves only: the plan's adjoint takes the fastest of the others).
+ * Writes a human-readable summary (may be NULL). */
 int symamd_tune(symamd_handle h, symamd_plan plan, int k,
                 symamd_layout layout, char *summary, int summary_len);
 

@@ -13,7 +13,7 @@ namespace symamd {
 
 namespace {
 thread_local std::string g_last_error;
-std::map<uint64_t, std::map<int64_t, Choice>> g_tune_cache;  // fingerprint ->
+std::map<uint64_t, std::map<int64_t, Tuned>> g_tune_cache;  // fingerprint ->
 
 uint64_t fnv1a(uint64_t h, const void *data, size_t len) {
   const unsigned char *b = (const unsigned char *)data;
@@ -106,13 +106,14 @@ __global__ __launch_bounds__(256) void k_max_row(int n, const int *__restrict__ 
     atomicMax(out, max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3])));
 }
 
-// forward: a forward solve (the region executor is a candidate)
+// forward: a forward solve (the region and row executors are candidates)
 Choice choose(symamd_handle h, symamd_plan p, int k, int layout, int exec, bool forward) {
   Choice c;
   auto it = p->tuned.find(tune_key(k, layout));
+  const bool tuned = it != p->tuned.end();
   if (exec == SYMAMD_EXEC_AUTO) {
-    if (it != p->tuned.end()) {
-      c = it->second;
+    if (tuned) {
+      c = forward ? it->second.best : it->second.units;
     } else {
       c = heuristic(p, k);
       if (forward && region_preferred(h, p, k, layout)) c.exec = SYMAMD_EXEC_REGIONS;
@@ -120,12 +121,18 @@ Choice choose(symamd_handle h, symamd_plan p, int k, int layout, int exec, bool 
   } else {
     c = heuristic(p, k);
     c.exec = exec;
-    if (it != p->tuned.end() && it->second.exec == exec) {
-      c.lanes = it->second.lanes;
-      c.tile = it->second.tile;
-    }
+    if (tuned)
+      for (const Choice &t : {it->second.units, it->second.best})
+        if (t.exec == exec && (forward || t.rows != 1)) {
+          c.lanes = t.lanes;
+          c.tile = t.tile;
+          c.rows = t.rows;
+        }
   }
-  if (p->lanes_override > 0) c.lanes = p->lanes_override;
+  if (p->lanes_override > 0) {
+    c.lanes = p->lanes_override;
+    c.rows = -1;
+  }
   return c;
 }
 
@@ -134,8 +141,9 @@ Choice choose(symamd_handle h, symamd_plan p, int k, int layout, int exec, bool 
 int tuned_region_cap(symamd_plan p, int k) {
   for (int layout : {SYMAMD_ROW_MAJOR, SYMAMD_COL_MAJOR}) {
     auto it = p->tuned.find(tune_key(k, layout));
-    if (it != p->tuned.end() && it->second.exec == SYMAMD_EXEC_REGIONS && it->second.cap > 0)
-      return it->second.cap;
+    if (it != p->tuned.end() && it->second.units.exec == SYMAMD_EXEC_REGIONS &&
+        it->second.units.cap > 0)
+      return it->second.units.cap;
   }
   return 0;
 }
@@ -327,7 +335,7 @@ int prepare_solve(symamd_handle h, symamd_plan p, int k, int layout, const Choic
   }
   const bool turn = through_workspace(h, k, layout);
   if (rows_path(h, p, k, turn, c.exec == SYMAMD_EXEC_REGIONS ? SYMAMD_EXEC_SYNCFREE : c.exec,
-                c.lanes, c.tile)) {
+                c)) {
     const int rc = prepare_rows(h, p, k, turn);
     if (rc != SYMAMD_ERR_ALLOC) return rc;  // without the memory: the unit executor
   }
@@ -340,7 +348,9 @@ int prepare_solve(symamd_handle h, symamd_plan p, int k, int layout, const Choic
 }
 
 int run_solve(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld,
-              int64_t rs, int64_t cs, int layout, int exec, int lanes, int tile) {
+              int64_t rs, int64_t cs, int layout, const Choice &c) {
+  int exec = c.exec, lanes = c.lanes;
+  const int tile = c.tile;
   if (exec == SYMAMD_EXEC_LEVELSET_GRAPH) exec = SYMAMD_EXEC_LEVELSET;
   if (exec == SYMAMD_EXEC_LEVELSET_SPLIT) lanes = 1;
   if (exec == SYMAMD_EXEC_REGIONS) {
@@ -353,7 +363,7 @@ int run_solve(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld,
     exec = SYMAMD_EXEC_SYNCFREE;
   }
   const bool turn = through_workspace(h, k, layout);
-  if (rows_path(h, p, k, turn, exec, lanes, tile))
+  if (rows_path(h, p, k, turn, exec, c))
     return launch_rows(h, p, d_B, k, ld, rs, cs, turn);
   if (turn)
     return launch_forward_ws(h, p, d_B, k, ld, exec, lanes, tile);
@@ -373,7 +383,7 @@ int capture_solve(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld,
   if (hipStreamBeginCapture(cap, hipStreamCaptureModeRelaxed) != hipSuccess) {
     rc = fail(SYMAMD_ERR_HIP, "hipStreamBeginCapture failed");
   } else {
-    rc = run_solve(h, p, d_B, k, ld, rs, cs, layout, c.exec, c.lanes, c.tile);
+    rc = run_solve(h, p, d_B, k, ld, rs, cs, layout, c);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(cap, &graph);
     if (rc == SYMAMD_OK && e != hipSuccess)
@@ -413,7 +423,7 @@ int solve_impl(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld,
     return SYMAMD_OK;
   }
   SYMAMD_TRY(prepare_solve(h, p, k, layout, c));
-  return run_solve(h, p, d_B, k, ld, rs, cs, layout, c.exec, c.lanes, c.tile);
+  return run_solve(h, p, d_B, k, ld, rs, cs, layout, c);
 }
 
 }  // namespace
@@ -673,7 +683,8 @@ int symamd_choice(symamd_handle h, symamd_plan plan, int k, symamd_layout layout
   if (k < 1) return fail(SYMAMD_ERR_INVALID_ARG, "k must be >= 1");
   Choice c = choose(h, plan, k, layout, SYMAMD_EXEC_AUTO, true);
   if (exec) *exec = c.exec;
-  if (lanes) *lanes = c.lanes;
+  // the row executor shares rows between lanes, whatever its units would do
+  if (lanes) *lanes = c.rows == 1 && c.lanes < 2 ? 2 : c.lanes;
   return SYMAMD_OK;
 }
 
@@ -886,13 +897,29 @@ int symamd_tune(symamd_handle h, symamd_plan plan, int k, symamd_layout layout,
   SYMAMD_HIP(hipEventCreate(&e1));
   const int gmax_rows = std::max(1, pow2_ceil((int)std::ceil(plan->avg_row_nnz)) * 2);
   std::string log;
-  Choice best;
-  float best_ms = 1e30f;
+  Tuned best;
+  Choice sync;  // the fastest units of the sync-free executor
+  float best_ms = 1e30f, units_ms = 1e30f, sync_ms = 1e30f;
   const int saved_override = plan->lanes_override;
   plan->lanes_override = 0;
   const int execs[] = {SYMAMD_EXEC_SYNCFREE, SYMAMD_EXEC_LEVELSET_GRAPH, SYMAMD_EXEC_REGIONS,
                        SYMAMD_EXEC_LEVELSET_SPLIT};
   int rc = SYMAMD_OK;
+  auto time_choice = [&](const Choice &c, float &ms) {
+    plan->tuned[tune_key(k, layout)] = {c, c};
+    ms = 1e30f;
+    rc = solve_impl(h, plan, d_B, k, ld, layout, SYMAMD_EXEC_AUTO, true);  // warm / capture
+    for (int rep = 0; rep < 3 && rc == SYMAMD_OK; ++rep) {
+      (void)hipEventRecord(e0, h->stream);
+      rc = solve_impl(h, plan, d_B, k, ld, layout, SYMAMD_EXEC_AUTO, true);
+      (void)hipEventRecord(e1, h->stream);
+      (void)hipEventSynchronize(e1);
+      float t = 0;
+      (void)hipEventElapsedTime(&t, e0, e1);
+      ms = std::min(ms, t);
+    }
+    return rc == SYMAMD_OK;
+  };
   // candidates: the executor; for the unit executors the column tile (all
   // of k up to 64 columns, or narrower tiles of 8 to 32 columns solved as
   // separate work items) and the lanes per row that share a row's entries
@@ -924,32 +951,44 @@ int symamd_tune(symamd_handle h, symamd_plan plan, int k, symamd_layout layout,
         c.lanes = g;
         c.tile = tile;
         c.cap = cap;
-        plan->tuned[tune_key(k, layout)] = c;
-        rc = solve_impl(h, plan, d_B, k, ld, layout, SYMAMD_EXEC_AUTO, true);  // warm / capture
-        if (rc != SYMAMD_OK) break;
-        float ms = 1e30f;
-        for (int rep = 0; rep < 3 && rc == SYMAMD_OK; ++rep) {
-          (void)hipEventRecord(e0, h->stream);
-          rc = solve_impl(h, plan, d_B, k, ld, layout, SYMAMD_EXEC_AUTO, true);
-          (void)hipEventRecord(e1, h->stream);
-          (void)hipEventSynchronize(e1);
-          float t = 0;
-          (void)hipEventElapsedTime(&t, e0, e1);
-          ms = std::min(ms, t);
-        }
-        if (rc != SYMAMD_OK) break;
+        c.rows = 0;
+        float ms;
+        if (!time_choice(c, ms)) break;
         char line[128];
         snprintf(line, sizeof line, "exec=%d lanes=%d tile=%d cap=%d ms=%.4f\n", ex, g, kt,
                  cap, ms);
         log += line;
-        if (ms < best_ms * 0.97f) {  // prefer earlier (fewer lanes, sync-free) on ties
-          best_ms = ms;
-          best = c;
+        // prefer earlier (fewer lanes, sync-free) on ties
+        if (ms < units_ms * 0.97f) {
+          units_ms = ms;
+          best.units = c;
+        }
+        if (ex == SYMAMD_EXEC_SYNCFREE && ms < sync_ms * 0.97f) {
+          sync_ms = ms;
+          sync = c;
         }
       }
       if (rc != SYMAMD_OK) break;
     }
     if (rc != SYMAMD_OK) break;
+  }
+  best.best = best.units;
+  best_ms = units_ms;
+  // the row executor, which has no choice of lanes or tile (it keeps those of
+  // the units it stands in for, where they have to run after all)
+  sync.rows = 1;
+  if (rc == SYMAMD_OK &&
+      rows_path(h, plan, k, through_workspace(h, k, layout), SYMAMD_EXEC_SYNCFREE, sync)) {
+    float ms;
+    if (time_choice(sync, ms)) {
+      char line[128];
+      snprintf(line, sizeof line, "exec=%d rows ms=%.4f\n", sync.exec, ms);
+      log += line;
+      if (ms < best_ms * 0.97f) {
+        best_ms = ms;
+        best.best = sync;
+      }
+    }
   }
   plan->lanes_override = saved_override;
   (void)hipEventDestroy(e0);
@@ -975,8 +1014,11 @@ int symamd_tune(symamd_handle h, symamd_plan plan, int k, symamd_layout layout,
   plan->tuned[tune_key(k, layout)] = best;
   g_tune_cache[plan->fingerprint][tune_key(k, layout)] = best;
   char line[128];
-  snprintf(line, sizeof line, "best exec=%d lanes=%d tile=%d cap=%d ms=%.4f\n", best.exec,
-           best.lanes, tile_cols(k, best.tile), best.cap, best_ms);
+  if (best.best.rows == 1)
+    snprintf(line, sizeof line, "best exec=%d rows ms=%.4f\n", best.best.exec, best_ms);
+  else
+    snprintf(line, sizeof line, "best exec=%d lanes=%d tile=%d cap=%d ms=%.4f\n", best.best.exec,
+             best.best.lanes, tile_cols(k, best.best.tile), best.best.cap, best_ms);
   log += line;
   if (summary && summary_len > 0) {
     strncpy(summary, log.c_str(), summary_len - 1);

@@ -289,6 +289,14 @@ struct Choice {
   int lanes = 1;  // lanes cooperating on one row's nonzeros
   int tile = 0;   // columns per tile of the unit executors (0: from k)
   int cap = 0;    // region cap of the region executor (0: the default)
+  int rows = -1;  // sync-free: the row executor (1), the units (0), as the plan says (-1)
+};
+
+// What the tuner chose: for forward solves, and among the executors other than
+// the row executor, whose lanes, tile and cap serve what that one does not run
+// (transposed solves, solves of a named executor).
+struct Tuned {
+  Choice best, units;
 };
 
 }  // namespace symamd
@@ -382,7 +390,7 @@ struct symamd_plan_s {
   int *d_ic0_bad = nullptr;
   // schedule choices
   int lanes_override = 0;
-  std::map<int64_t, symamd::Choice> tuned;  // key(k, layout) -> choice
+  std::map<int64_t, symamd::Tuned> tuned;  // key(k, layout) -> choice
   uint64_t fingerprint = 0;
   double avg_row_nnz = 1.0;
   int max_row_nnz = 1;
@@ -506,7 +514,7 @@ int prepare_workspace(symamd_handle h, symamd_plan p, int k);
 int split_threshold(symamd_handle h, int kt);
 // Row executor (rows_exec.hip): sync-free solves with several lanes per row
 // (turn: of a column-major block, through the workspace).
-bool rows_path(symamd_handle h, symamd_plan p, int k, bool turn, int exec, int lanes, int tile);
+bool rows_path(symamd_handle h, symamd_plan p, int k, bool turn, int exec, const Choice &c);
 // d_ws of at least `bytes`; a solve being captured keeps the one it uses, and
 // may grow it.
 int plan_workspace(symamd_handle h, symamd_plan p, size_t bytes);

@@ -443,15 +443,18 @@ static size_t rows_bytes(symamd_plan p, int k, bool turn) {
   return (size_t)p->n * k * (turn ? 2 : 1) * (p->dtype == SYMAMD_F64 ? 8 : 4);
 }
 
-// Whether a sync-free solve of k right-hand sides runs here: several lanes
-// per row beside the column tile (one lane per row keeps the reference's
-// order in every row, which the unit executor does), the marked protocol on,
-// no unit trace, and memory for the schedule and the workspace.  A solve being
-// recorded by the caller needs an earlier one here, as the unit executor does.
-bool rows_path(symamd_handle h, symamd_plan p, int k, bool turn, int exec, int lanes, int tile) {
-  if (exec != SYMAMD_EXEC_SYNCFREE || lanes < 2 || 2 * tile_cols(k, tile) > 64 || h->unmarked ||
-      h->trace || rows_bytes(p, k, turn) >= p->rows_limit)
+// Whether a solve of k right-hand sides runs here: sync-free, the marked
+// protocol on, no unit trace, memory for the schedule and the workspace, and
+// either the tuner timed it so or, untuned, several lanes per row fit beside
+// the unit executor's column tile (one lane per row keeps the reference's
+// order in every row, which that one does; so it also solves untuned blocks of
+// more than 32 columns).  A solve being recorded by the caller needs an
+// earlier one here, as the unit executor does.
+bool rows_path(symamd_handle h, symamd_plan p, int k, bool turn, int exec, const Choice &c) {
+  if (exec != SYMAMD_EXEC_SYNCFREE || c.rows == 0 || h->unmarked || h->trace ||
+      rows_bytes(p, k, turn) >= p->rows_limit)
     return false;
+  if (c.rows < 0 && (c.lanes < 2 || 2 * tile_cols(k, c.tile) > 64)) return false;
   const auto s = p->rows.find(rows_cols(k));
   if (s != p->rows.end()) return !s->second.failed;
   return !p->rows.empty() || !capturing(h->stream);
