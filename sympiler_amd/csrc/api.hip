@@ -901,6 +901,9 @@ int symamd_tune(symamd_handle h, symamd_plan plan, int k, symamd_layout layout,
   Choice sync;  // the fastest units of the sync-free executor
   float best_ms = 1e30f, units_ms = 1e30f, sync_ms = 1e30f;
   const int saved_override = plan->lanes_override;
+  void *const ws_before = plan->d_ws;
+  const bool ws_held = plan->ws_captured;
+  const size_t retired = plan->ws_retired.size();
   plan->lanes_override = 0;
   const int execs[] = {SYMAMD_EXEC_SYNCFREE, SYMAMD_EXEC_LEVELSET_GRAPH, SYMAMD_EXEC_REGIONS,
                        SYMAMD_EXEC_LEVELSET_SPLIT};
@@ -1007,6 +1010,14 @@ int symamd_tune(symamd_handle h, symamd_plan plan, int k, symamd_layout layout,
     }
   }
   (void)hipFree(d_B);
+  // nor do those hold a workspace any more: what they outgrew goes, and the
+  // present one may be replaced, unless an earlier graph has it
+  for (size_t i = plan->ws_retired.size(); i-- > retired;)
+    if (!(ws_held && plan->ws_retired[i] == ws_before)) {
+      (void)hipFree(plan->ws_retired[i]);
+      plan->ws_retired.erase(plan->ws_retired.begin() + i);
+    }
+  plan->ws_captured = ws_held && plan->d_ws == ws_before;
   if (rc != SYMAMD_OK) {
     plan->tuned.erase(tune_key(k, layout));
     return rc;

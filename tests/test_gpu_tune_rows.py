@@ -63,3 +63,21 @@ def test_adjoint_keeps_the_lanes_of_the_units(dev):
         if np.array_equal(got.cpu().numpy(), auto):
             same.append(lanes)
     assert set(same) & set(near), (same, near, log)
+
+
+def test_tuning_holds_no_outgrown_workspace(dev):
+    """The graphs of the tuner are gone when it returns, so a wider solve
+    replaces the workspace they held (58 MB for 12 columns) by its own (77 MB
+    for 16) instead of keeping both."""
+    import torch
+    Lp, Li, Lx = W.zipf_lower(300000, 1.8, 64, 5000, 66)
+    n = len(Lp) - 1
+    plan = sa.Plan(*to_dev(Lp, Li, Lx))
+    plan.set_lanes(2)
+    plan.tune(k=12)
+    X = to_dev(W.uniform(67, 0, n * 16).reshape(16, n))
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    plan.solve(X, executor="syncfree")
+    plan.check()
+    assert before - torch.cuda.mem_get_info()[0] < 40 << 20
