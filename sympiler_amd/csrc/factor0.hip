@@ -318,30 +318,32 @@ __device__ __forceinline__ void short_prep(const FactorArgs &a, int b0, int m, i
 }
 
 // A unit whose rows all are short, with at most SHORT_PB pairs each, has its
-// structure packed: word w of the unit's rows side by side, so that a wave
-// reads it in whole cache lines (from the caller's row-ordered arrays a level's
-// rows touch some 30 lines each, 4 GB in all for the 128^3 Laplacian).  Words:
+// structure packed: word w of the unit's rows side by side (word w of row l at
+// w * rows + l: a unit of one row, as in a chain, takes no more than its
+// words), so that a wave reads it in whole cache lines (from the caller's
+// row-ordered arrays a level's rows touch some 30 lines each, 4 GB in all for
+// the 128^3 Laplacian).  Words:
 // first entry, entries | diagonal << 8, pairs of each entry (4 bits each),
 // the divisors' positions, the pairs' other-row positions, and their offsets in
 // this row (first | second << 8, 255: another row's).
 constexpr int PACK_WORDS = 3;
 
 template <int MODE>
-__device__ __forceinline__ void packed_prep(const FactorArgs &a, const int *D, int E, int P,
-                                            int &b0, int &m, int &dr, ShortRow &w,
+__device__ __forceinline__ void packed_prep(const FactorArgs &a, const int *D, int rows, int E,
+                                            int P, int &b0, int &m, int &dr, ShortRow &w,
                                             PairSlots &ps) {
   b0 = D[0];
-  const int meta = D[64];
-  const unsigned counts = (unsigned)D[128];
+  const int meta = D[rows];
+  const unsigned counts = (unsigned)D[2 * rows];
   m = meta & 255;
   dr = meta >> 8;
 #pragma unroll
-  for (int j = 0; j < SHORT_RB; ++j) w.dp[j] = j < E ? D[64 * (PACK_WORDS + j)] : -1;
+  for (int j = 0; j < SHORT_RB; ++j) w.dp[j] = j < E ? D[rows * (PACK_WORDS + j)] : -1;
 #pragma unroll
   for (int k = 0; k < SHORT_PB; ++k) {
     if (k >= P) break;
-    const int o = D[64 * (PACK_WORDS + E + P + k)];
-    ps.yp[k] = D[64 * (PACK_WORDS + E + k)];
+    const int o = D[rows * (PACK_WORDS + E + P + k)];
+    ps.yp[k] = D[rows * (PACK_WORDS + E + k)];
     ps.ia[k] = (int16_t)(o & 255);
     ps.ib[k] = (int16_t)((o >> 8) == 255 ? -1 : o >> 8);
   }
@@ -364,13 +366,13 @@ __global__ __launch_bounds__(256) void k_factor0_pack(FactorArgs a, int64_t *siz
                                                       int *data) {
   const int u = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (u >= a.U) return;
-  const int q = a.ub[u] + lane;
-  const bool act = q < a.ub[u + 1];
+  const int q = a.ub[u] + lane, rows = a.ub[u + 1] - a.ub[u];
+  const bool act = lane < rows;
   const int r = act ? a.perm[q] : 0;
   const int b0 = act ? a.rp[r] : 0, m = act ? a.rp[r + 1] - b0 : 0;
   const int64_t t0 = act ? a.pp[b0] : 0, np = act ? a.pp[b0 + m] - t0 : 0;
   if (!FILL) {
-    const bool all = __all(m <= SHORT_RB && np <= SHORT_PB);
+    const bool all = rows > 0 && __all(m <= SHORT_RB && np <= SHORT_PB);
     int E = m, P = (int)np;
     for (int off = 32; off > 0; off >>= 1) {
       E = max(E, __shfl_xor(E, off));
@@ -378,28 +380,28 @@ __global__ __launch_bounds__(256) void k_factor0_pack(FactorArgs a, int64_t *siz
     }
     if (lane == 0) {
       wide[u] = all ? E | P << 8 : -1;
-      size[u] = all ? 64 * (PACK_WORDS + E + 2 * P) : 0;
+      size[u] = all ? rows * (PACK_WORDS + E + 2 * P) : 0;
     }
     return;
   }
   const int wd = wide[u];
-  if (wd < 0) return;
+  if (wd < 0 || !act) return;
   const int E = wd & 255, P = wd >> 8;
   int *D = data + size[u] + lane;  // the sizes, scanned
-  const int dr = MODE == MODE_IC0 ? m - 1 : act ? a.adiag[r] - b0 : 0;
+  const int dr = MODE == MODE_IC0 ? m - 1 : a.adiag[r] - b0;
   unsigned counts = 0;
   for (int j = 0; j < E; ++j) {
     const bool in = j < m;
     if (in) counts |= (unsigned)(a.pp[b0 + j + 1] - a.pp[b0 + j]) << (4 * j);
-    D[64 * (PACK_WORDS + j)] = in && (MODE == MODE_ILU0 || j != dr) ? a.dpos[b0 + j] : -1;
+    D[rows * (PACK_WORDS + j)] = in && (MODE == MODE_ILU0 || j != dr) ? a.dpos[b0 + j] : -1;
   }
   D[0] = b0;
-  D[64] = m | (act ? dr : 0) << 8;
-  D[128] = (int)counts;
+  D[rows] = m | dr << 8;
+  D[2 * rows] = (int)counts;
   for (int k = 0; k < P; ++k) {
     const int ia = k < np ? a.pa[t0 + k] : b0, ib = k < np ? a.pb[t0 + k] : b0;
-    D[64 * (PACK_WORDS + E + k)] = ib;
-    D[64 * (PACK_WORDS + E + P + k)] = (ia - b0) | (ib < b0 ? 255 : ib - b0) << 8;
+    D[rows * (PACK_WORDS + E + k)] = ib;
+    D[rows * (PACK_WORDS + E + P + k)] = (ia - b0) | (ib < b0 ? 255 : ib - b0) << 8;
   }
 }
 
@@ -494,15 +496,16 @@ __global__ __launch_bounds__(64) void k_factor0(FactorArgs a) {
   for (;;) {
     const int u = next_unit(a.state, a.ticketed, cursor, a.total_waves);
     if (u >= a.U) break;
-    const int q = a.ub[u] + lane;
-    const bool act = q < a.ub[u + 1];
+    const int q = a.ub[u] + lane, rows = a.ub[u + 1] - a.ub[u];
+    const bool act = lane < rows;
     int r = 0, b0 = 0, m = 0, dr = 0;
     ShortRow w;
     const int wide = a.pwide[u];
     if (wide >= 0) {
-      if (act) r = a.perm[q];
-      packed_prep<MODE>(a, a.pdata + a.poff[u] + lane, wide & 255, wide >> 8, b0, m, dr, w,
-                        slots[threadIdx.x]);
+      // lanes past the unit's rows read its last one, and use none of it
+      r = a.perm[min(q, a.ub[u + 1] - 1)];
+      packed_prep<MODE>(a, a.pdata + a.poff[u] + min(lane, rows - 1), rows, wide & 255, wide >> 8,
+                        b0, m, dr, w, slots[threadIdx.x]);
     } else if (act) {
       r = a.perm[q];
       b0 = a.rp[r];
