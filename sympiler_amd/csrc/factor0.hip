@@ -551,13 +551,21 @@ struct Scratch {
   }
 };
 
-// Persistent launch over the plan's forward units (co-resident grid,
-// cooperative unless capturing; else units from the ticket counter), then
-// wait for it and return the failed-pivot row (-1: none).
-// Wavefronts per CU: the next levels' units loaded ahead; more of them only
-// poll (IC(0) of the 128^3 Laplacian with 128 / 256 / 512 / 1024 waves 1.74 /
-// 1.37 / 1.64 / 1.88 ms, of the 64^3 one 0.66 / 0.70 / 0.74 / 0.78).
-constexpr int FACTOR_PER_CU = 1;
+// Wavefronts of the factorization: a small look-ahead over a level's units, at
+// least one per CU.  Those beyond it only poll and slow the chain of levels, on
+// which narrow levels spend their time; wide ones are solved by as many as
+// there are.  In ms, by units a level and waves: 86 (IC(0) of the 128^3
+// Laplacian) 128 / 256 / 512 / 1024 waves 1.74 / 1.37 / 1.64 / 1.88; 22 (64^3)
+// 0.66 / 0.70 / 0.74 / 0.78; 292 (the batch of 512 planes) 256 / 512 / 1024 /
+// 2048 2.88 / 2.07 / 2.05 / 2.54; 1000 (27-point grid of 64^3 in eight colours)
+// 256 / 1024 / 2048 / 3072 2.46 / 1.03 / 0.71 / 0.73; 16,384 (red-black 128^3)
+// 256 / 1024 / 3072 0.65 / 0.28 / 0.21.  The same number on every CU (258 waves
+// on 256 CUs: 1.43 ms for the first).
+constexpr int FACTOR_LEVELS_AHEAD = 3;
+int64_t factor_waves(symamd_handle h, symamd_plan p, int units, int per_cu) {
+  const int64_t ahead = FACTOR_LEVELS_AHEAD * (int64_t)units / std::max(p->levels, 1);
+  return h->num_cus * std::max<int64_t>(1, std::min<int64_t>(ahead / h->num_cus, per_cu));
+}
 
 int scan64(symamd_handle h, const int64_t *in, int64_t *out, int64_t count, Scratch &sc);
 
@@ -600,6 +608,9 @@ void free_pack(FactorPack &f) {
   f = FactorPack();
 }
 
+// Persistent launch over the plan's forward units (co-resident grid,
+// cooperative unless capturing; else units from the ticket counter), then
+// wait for it and return the failed-pivot row (-1: none).
 template <int MODE>
 int launch_factor0(symamd_handle h, symamd_plan p, int64_t nnz, FactorArgs a, FactorPack &pack,
                    int *bad_row) {
@@ -630,7 +641,7 @@ int launch_factor0(symamd_handle h, symamd_plan p, int64_t nnz, FactorArgs a, Fa
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, 64, 0) != hipSuccess ||
       per_cu < 1)
     per_cu = 1;
-  int64_t cap = (int64_t)std::min(per_cu, FACTOR_PER_CU) * h->num_cus;
+  int64_t cap = factor_waves(h, p, a.U, per_cu);
   if (h->max_waves > 0 && h->max_waves < cap) cap = h->max_waves;
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(a.U, cap));
   a.total_waves = grid;

@@ -1,5 +1,6 @@
 """Zero-fill factorizations over the shapes a level set can have: chains (one
-row a level, whose packed structure takes no more than the rows need)."""
+row a level, whose packed structure takes no more than the rows need), and
+levels of more units than the card has CUs, with packed and unpacked units."""
 import numpy as np
 import pytest
 
@@ -34,3 +35,70 @@ def test_chain_takes_the_memory_of_its_rows(dev):
     assert before - torch.cuda.mem_get_info()[0] < 24 << 20
     want = oracle_factor(Lp, Li, A, "left")
     assert bitwise_equal(got.cpu().numpy(), want[0] if isinstance(want, tuple) else want)
+
+
+def colours(g, stencil):
+    """Lower triangle of a grid's Laplacian, rows ordered by colour: two levels
+    (stencil 7, red and black) or eight (27)."""
+    i = np.arange(g ** 3)
+    x, y, z = i % g, i // g % g, i // (g * g)
+    r, c = [], []
+    for d in range(1, 14):
+        dz, rem = divmod(d + 4, 9)
+        dy, dx = rem // 3 - 1, rem % 3 - 1
+        if stencil == 7 and abs(dx) + abs(dy) + abs(dz) != 1:
+            continue
+        ok = (x + dx >= 0) & (x + dx < g) & (y + dy >= 0) & (y + dy < g) & (z + dz < g)
+        r.append(i[ok])
+        c.append((i + dx + g * (dy + g * dz))[ok])
+    r, c = np.concatenate(r), np.concatenate(c)
+    colour = (x + y + z) % 2 if stencil == 7 else x % 2 + 2 * (y % 2) + 4 * (z % 2)
+    new = np.empty(g ** 3, int)
+    new[np.argsort(colour, kind="stable")] = i
+    lo, hi = np.minimum(new[r], new[c]), np.maximum(new[r], new[c])
+    rows, cols = np.concatenate([hi, i]), np.concatenate([lo, i])
+    order = np.lexsort((cols, rows))
+    rows, cols = rows[order], cols[order]
+    Lp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=g ** 3))]).astype(np.int32)
+    v = np.full(len(cols), -1.0)
+    v[rows == cols] = stencil - 1 + 0.01
+    return Lp, cols.astype(np.int32), v
+
+
+@pytest.mark.parametrize("stencil,levels", [(7, 2), (27, 8)])
+def test_levels_wider_than_the_card(dev, stencil, levels):
+    Lp, Li, A = colours(48, stencil)
+    plan = sa.Plan(*to_dev(Lp, Li, A))
+    assert plan.levels == levels
+    want = oracle_factor(Lp, Li, A, "left")
+    want = want[0] if isinstance(want, tuple) else want
+    a = to_dev(A)
+    got, _ = plan.ic0(a, strict=False)
+    assert bitwise_equal(got.cpu().numpy(), want)
+    plan.ic0(a, out=a, strict=False)
+    assert bitwise_equal(a.cpu().numpy(), want)
+
+
+def test_wide_levels_use_the_whole_card(dev):
+    """Red-black 96^3: 6,912 units a level, which one wavefront per CU takes 27
+    rounds for; limiting the waves to that makes it slower."""
+    import torch
+    Lp, Li, A = colours(96, 7)
+    a = to_dev(A)
+    out = torch.empty_like(a)
+
+    def best(waves):
+        h = sa.Handle()
+        h.set_max_waves(waves)
+        plan = sa.Plan(*to_dev(Lp, Li, A), handle=h)
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        ms = []
+        for _ in range(8):
+            e[0].record()
+            plan.ic0(a, out=out, strict=False)
+            e[1].record()
+            e[1].synchronize()
+            ms.append(e[0].elapsed_time(e[1]))
+        return min(ms)
+
+    assert best(0) < 0.8 * best(256)
