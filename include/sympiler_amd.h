@@ -105,7 +105,12 @@ int symamd_set_timeout_ms(symamd_handle h, double ms);
  *     for its value stores; readers re-load any value still marked.  0 = the
  *     tag is published after the stores are acknowledged.  The solve
  *     overwrites B in place either way; intermediate contents of B are
- *     unspecified while a solve runs. */
+ *     unspecified while a solve runs.  IC(0) and ILU(0) mark the factor's
+ *     storage the same way (in place, A is copied to the plan's workspace
+ *     first, 8 bytes an entry); 0, or no memory for that copy, = units wait
+ *     for the tags of those they read.  The row executor (sync-free solves
+ *     of any number of right-hand sides with several lanes per row) needs the
+ *     marks: 0 = such solves run on the units. */
 /*   SYMAMD_OPT_REGIONS (read by symamd_analyze*): 1 = cluster the rows into
  *     compact regions of the dependency graph (heavy-edge matching, at most
  *     SYMAMD_OPT_REGION_ROWS rows each) when at least half of L's

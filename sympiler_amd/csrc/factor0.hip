@@ -47,7 +47,10 @@
 // row is either the mark or final: lanes poll the values they need, and no
 // unit tag or store acknowledgement lies on the chain of levels, which bounds
 // the factorization.  128^3 grid, 382 levels, in ms: IC(0) 2.01 with tagged units,
-// 1.37 here; ILU(0) 3.01, 1.96.
+// 1.37 here; ILU(0) 3.01, 1.96.  In place, A is copied aside first; without the
+// memory for that, and with the marked protocol off, units wait for the tags of
+// those they read and the factor's storage stays as it is until its rows are
+// written.
 #include <rocprim/device/device_scan.hpp>
 
 #include <algorithm>
@@ -199,6 +202,8 @@ struct FactorArgs {
   const int *adiag;          // ILU(0): position of each row's diagonal
   const int *perm;           // level position -> row
   const int *ub;             // units
+  const int *dptr, *dlist;   // tagged units: the units that unit u reads,
+  int *uflags;               //   and their tags
   const int64_t *poff;       // packed units: unit u's words start at pdata[poff[u]]
   const int *pwide, *pdata;  //   its entries and pairs per row (e | p << 8), or -1: not packed
   int *state;
@@ -487,11 +492,14 @@ __device__ __forceinline__ void long_row(const FactorArgs &a, int r, int b0, int
 
 // One wave per unit (a run of at most 64 rows of one level), one lane per
 // row.  Units are taken in level order, so every value waited for is a
-// running wave's.
-template <int MODE>
+// running wave's.  TAGGED: a unit's structure is read, then the tags of the
+// units it reads are waited for; all values are final from there on (and none
+// is the mark's), so nothing below waits.
+template <int MODE, bool TAGGED>
 __global__ __launch_bounds__(64) void k_factor0(FactorArgs a) {
   __shared__ PairSlots slots[64];
   const int lane = threadIdx.x;
+  const int target = TAGGED ? ld_dev(&a.state[ST_EPOCH]) + 1 : 0;
   int cursor = (int)blockIdx.x;
   for (;;) {
     const int u = next_unit(a.state, a.ticketed, cursor, a.total_waves);
@@ -500,7 +508,7 @@ __global__ __launch_bounds__(64) void k_factor0(FactorArgs a) {
     const bool act = lane < rows;
     int r = 0, b0 = 0, m = 0, dr = 0;
     ShortRow w;
-    const int wide = a.pwide[u];
+    const int wide = a.pwide ? a.pwide[u] : -1;
     if (wide >= 0) {
       // lanes past the unit's rows read its last one, and use none of it
       r = a.perm[min(q, a.ub[u + 1] - 1)];
@@ -513,18 +521,24 @@ __global__ __launch_bounds__(64) void k_factor0(FactorArgs a) {
       dr = MODE == MODE_IC0 ? m - 1 : a.adiag[r] - b0;
       if (m <= SHORT_RB) short_prep<MODE>(a, b0, m, dr, w, slots[threadIdx.x]);
     }
+    if (TAGGED) wait_units(a.dptr, a.dlist, u, a.uflags, target, a.state, a.timeout);
     if (act) {
       if (m <= SHORT_RB)
         short_fin<MODE>(a, r, b0, m, dr, w, slots[threadIdx.x]);
       else
         long_row<MODE>(a, r, b0, m, dr);
     }
+    if (TAGGED) {
+      publish_fence();
+      if (lane == 0) st_dev(&a.uflags[u], target);
+    }
   }
   persistent_finish(a.state, a.total_waves);
 }
 
-// The factor's storage marked, the failed-pivot word cleared; A's values
-// copied aside first where the factor takes their place.
+// The failed-pivot word cleared and, of nnz entries (none for tagged units),
+// the factor's storage marked; A's values copied aside first where the factor
+// takes their place.
 __global__ __launch_bounds__(256) void k_factor0_begin(int64_t nnz, const double *A, double *copy,
                                                        double *L, int *bad) {
   const int64_t t0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -569,16 +583,20 @@ int64_t factor_waves(symamd_handle h, symamd_plan p, int units, int per_cu) {
 
 int scan64(symamd_handle h, const int64_t *in, int64_t *out, int64_t count, Scratch &sc);
 
-// The packed units of a factorization, built on first use.
+// The packed units of a factorization, built on first use.  Without the memory
+// every unit is read from the caller's arrays.
 template <int MODE>
 int factor_pack(symamd_handle h, FactorArgs a, FactorPack &f) {
   if (f.d_off) return SYMAMD_OK;
   Scratch sc, keep;
   int64_t *size = nullptr, *off = nullptr;
   int *wide = nullptr, *data = nullptr;
-  SYMAMD_TRY(sc.alloc(&size, (size_t)a.U + 1));
-  SYMAMD_TRY(keep.alloc(&off, (size_t)a.U + 1));
-  SYMAMD_TRY(keep.alloc(&wide, (size_t)a.U));
+  if (sc.alloc(&size, (size_t)a.U + 1) != SYMAMD_OK ||
+      keep.alloc(&off, (size_t)a.U + 1) != SYMAMD_OK ||
+      keep.alloc(&wide, (size_t)a.U) != SYMAMD_OK) {
+    (void)hipGetLastError();
+    return SYMAMD_OK;
+  }
   SYMAMD_HIP(hipMemsetAsync(size, 0, sizeof(int64_t) * ((size_t)a.U + 1), h->stream));
   const unsigned blocks = (unsigned)std::max((a.U + 3) / 4, 1);
   k_factor0_pack<MODE, false><<<blocks, 256, 0, h->stream>>>(a, size, wide, nullptr);
@@ -590,7 +608,7 @@ int factor_pack(symamd_handle h, FactorArgs a, FactorPack &f) {
   if (keep.alloc(&data, (size_t)words) == SYMAMD_OK) {
     k_factor0_pack<MODE, true><<<blocks, 256, 0, h->stream>>>(a, off, wide, data);
     SYMAMD_HIP(hipGetLastError());
-  } else {  // no room: every unit from the caller's arrays
+  } else {
     (void)hipGetLastError();
     SYMAMD_HIP(hipMemsetAsync(wide, 0xff, sizeof(int) * std::max(a.U, 1), h->stream));
   }
@@ -622,10 +640,14 @@ int launch_factor0(symamd_handle h, symamd_plan p, int64_t nnz, FactorArgs a, Fa
   a.U = us->count;
   SYMAMD_TRY(factor_pack<MODE>(h, a, pack));  // before A's place is marked: it can fail
   double *copy = nullptr;
-  if (a.Ax == a.Lx) {
-    SYMAMD_TRY(plan_workspace(h, p, sizeof(double) * (size_t)nnz));
-    copy = (double *)p->d_ws;
+  bool tagged = h->unmarked;
+  if (a.Ax == a.Lx && !tagged) {
+    const int rc = plan_workspace(h, p, sizeof(double) * (size_t)nnz);
+    if (rc != SYMAMD_OK && rc != SYMAMD_ERR_ALLOC) return rc;
+    tagged = rc == SYMAMD_ERR_ALLOC;
+    if (!tagged) copy = (double *)p->d_ws;
   }
+  if (tagged) nnz = 0;
   k_factor0_begin<<<(unsigned)std::min<int64_t>(std::max<int64_t>((nnz + 255) / 256, 1), 8192),
                     256, 0, h->stream>>>(nnz, a.Ax, copy, a.Lx, p->d_ic0_bad);
   SYMAMD_HIP(hipGetLastError());
@@ -635,8 +657,12 @@ int launch_factor0(symamd_handle h, symamd_plan p, int64_t nnz, FactorArgs a, Fa
   a.poff = pack.d_off;
   a.pwide = pack.d_wide;
   a.pdata = pack.d_data;
+  a.dptr = us->d_dptr;
+  a.dlist = us->d_dlist;
+  a.uflags = us->d_uflags;
   a.timeout = h->timeout_ticks();
-  const void *kfn = (const void *)&k_factor0<MODE>;
+  const void *kfn = tagged ? (const void *)&k_factor0<MODE, true>
+                           : (const void *)&k_factor0<MODE, false>;
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, 64, 0) != hipSuccess ||
       per_cu < 1)

@@ -1,12 +1,16 @@
 """Zero-fill factorizations over the shapes a level set can have: chains (one
 row a level, whose packed structure takes no more than the rows need), and
-levels of more units than the card has CUs, with packed and unpacked units."""
+levels of more units than the card has CUs, with packed and unpacked units; and
+the units' tags, which in-place factorizations without room for a copy of A
+wait for (with the marked protocol off, as here, all do)."""
 import numpy as np
 import pytest
 
 import oracle
 import sympiler_amd as sa
+from sympiler_amd import workloads as W
 from tests.helpers import bitwise_equal, to_dev
+from tests.test_gpu_factor_units import banded
 from tests.test_gpu_ic0 import oracle_factor
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +106,60 @@ def test_wide_levels_use_the_whole_card(dev):
         return min(ms)
 
     assert best(0) < 0.8 * best(256)
+
+
+@pytest.mark.parametrize("tickets", [False, True])
+@pytest.mark.parametrize("name", ["red_black", "colours", "chain", "band"])
+def test_tagged_units_need_no_copy(dev, name, tickets):
+    import torch
+    Lp, Li, A = {"red_black": lambda: colours(40, 7), "colours": lambda: colours(24, 27),
+                 "chain": lambda: chain(3000), "band": lambda: banded(3000, 6, 7, 3)}[name]()
+    n = len(Lp) - 1
+    h = sa.Handle(timeout_ms=2000)
+    h.set_marks(False)
+    h.set_tickets(tickets)
+    print(f"[tagged] {name} n={n}", flush=True)
+    plan = sa.Plan(*to_dev(Lp, Li, A), handle=h)
+    for variant in ("left", "csr"):
+        want = oracle_factor(Lp, Li, A, variant)
+        want = want[0] if isinstance(want, tuple) else want
+        a = to_dev(A)
+        got, _ = plan.ic0(a, variant=variant, strict=False)
+        assert bitwise_equal(got.cpu().numpy(), want)
+        plan.ic0(a, variant=variant, out=a, strict=False)
+        assert bitwise_equal(a.cpu().numpy(), want)
+
+
+def test_tagged_factor_in_place_takes_no_workspace(dev):
+    """3.5 M entries: a copy of A takes 28 MB."""
+    import torch
+    Lp, Li, A = colours(96, 7)
+    h = sa.Handle()
+    h.set_marks(False)
+    plan = sa.Plan(*to_dev(Lp, Li, A), handle=h)
+    a = to_dev(A)
+    want, _ = plan.ic0(a, strict=False)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    plan.ic0(a, out=a, strict=False)
+    assert before - torch.cuda.mem_get_info()[0] < 8 << 20
+    assert torch.equal(a, want)
+
+
+def test_tagged_ilu0_with_the_marks_bits(dev):
+    """An entry of A that holds the mark's NaN, and one that no update touches:
+    no unit waits for it."""
+    Ap, Ai, Ax, diags = W.grid3d_general(6, 2)
+    p = int(diags[np.flatnonzero(np.diff(Ap) > 0)[0]]) + 1
+    for bad in (False, True):
+        A = Ax.copy()
+        if bad:
+            A.view(np.uint64)[p] = 0x7FF4D0D0CAFEF00D
+        h = sa.Handle(timeout_ms=500)
+        h.set_marks(False)
+        plan = sa.Ilu0Plan(*to_dev(Ap, Ai, diags), handle=h)
+        a = to_dev(A)
+        plan.factor(a, out=a, strict=False)
+        want, _ = oracle.spilu0_csr(Ap, Ai, A, diags)
+        g, ok = a.cpu().numpy(), ~np.isnan(want)
+        assert np.array_equal(np.isnan(g), ~ok) and bitwise_equal(g[ok], want[ok])
