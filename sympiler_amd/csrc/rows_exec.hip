@@ -277,64 +277,157 @@ constexpr int ROWS_PER_CU(int c) { return c == 1 ? 1 : c == 8 ? 1 : 2; }
 
 int rows_cols(int k) { return k == 1 ? 1 : k <= 8 ? 8 : k <= 16 ? 16 : 32; }
 
-// The schedule for C column lanes: per level the rows a workgroup shares,
-// then the others by descending slices, waves of a ticket filled from one
-// level.
-int build_rows(symamd_plan p, int C, hipStream_t stream, RowSchedule &s) {
-  const int n = p->n, W = rows_waves(C), smax = 64 / C, epl = rows_epl(C);
-  std::vector<int> rp(n + 1), perm(n);
-  SYMAMD_HIP(hipMemcpyAsync(rp.data(), p->d_rp, sizeof(int) * (n + 1), hipMemcpyDeviceToHost,
-                            stream));
-  SYMAMD_HIP(hipMemcpyAsync(perm.data(), p->d_perm, sizeof(int) * n, hipMemcpyDeviceToHost,
-                            stream));
-  SYMAMD_HIP(hipStreamSynchronize(stream));
-  int lgmax = 0;
-  while ((1 << lgmax) < smax) ++lgmax;
-  // class of a row, in solving order: the workgroup's (0), lgmax .. 0 slices
-  // as 1 .. lgmax + 1, short (lgmax + 2)
-  auto cls = [&](int q) {
-    const int len = rp[q + 1] - 1 - rp[q];
-    if (C > 1 && len > 2 * epl * smax) return 0;
-    if (rows_short(C) && len <= ROWS_SHORT) return lgmax + 2;
+// The schedule's shape for C column lanes.  Classes of rows, in solving order:
+// those a workgroup shares (0), those of lgmax .. 0 slices (1 .. lgmax + 1),
+// short ones (lgmax + 2); up to ROWS_CLASSES.
+constexpr int ROWS_CLASSES = 9;
+struct RowShape {
+  int waves, smax, epl, lgmax;
+  bool group, shorts;
+  explicit RowShape(int C)
+      : waves(rows_waves(C)), smax(64 / C), epl(rows_epl(C)), lgmax(0), group(C > 1),
+        shorts(rows_short(C)) {
+    while ((1 << lgmax) < smax) ++lgmax;
+  }
+  __host__ __device__ int classes() const { return lgmax + 3; }
+  __device__ int cls(int len) const {
+    if (group && len > 2 * epl * smax) return 0;
+    if (shorts && len <= ROWS_SHORT) return lgmax + 2;
     int lg = 0;
     while (lg < lgmax && (epl << lg) < len) ++lg;
     return lgmax + 1 - lg;
+  }
+  // rows of one wave's item, and the item's kind
+  __host__ __device__ int rows(int c) const {
+    return c == 0 ? 1 : c == lgmax + 2 ? smax * ROWS_PER_LANE : smax >> (lgmax + 1 - c);
+  }
+  __device__ int kind(int c) const { return c == lgmax + 2 ? ROWS_KIND_SHORT : lgmax + 1 - c; }
+};
+
+// Rows of each class, a workgroup per level.
+constexpr int ROWS_BUILD = 512;
+__global__ __launch_bounds__(ROWS_BUILD) void k_rows_count(RowShape sh,
+                                                           const int *__restrict__ lvl,
+                                                           const int *__restrict__ rp,
+                                                           int *count) {
+  __shared__ int cnt[ROWS_CLASSES];
+  const int l = blockIdx.x, t = threadIdx.x;
+  if (t < ROWS_CLASSES) cnt[t] = 0;
+  __syncthreads();
+  for (int q = lvl[l] + t; q < lvl[l + 1]; q += ROWS_BUILD)
+    atomicAdd(&cnt[sh.cls(rp[q + 1] - 1 - rp[q])], 1);
+  __syncthreads();
+  if (t < ROWS_CLASSES) count[l * ROWS_CLASSES + t] = cnt[t];
+}
+
+// Records and items of a level, a workgroup per level: per level the rows a
+// workgroup shares, then the others by descending slices, each class in level
+// order; waves of a ticket filled from one level, the last ones left empty.
+// first[l] .. first[l + 1]: the level's items.
+__global__ __launch_bounds__(ROWS_BUILD) void k_rows_fill(RowShape sh,
+                                                          const int *__restrict__ lvl,
+                                                          const int *__restrict__ rp,
+                                                          const int *__restrict__ perm,
+                                                          const int *__restrict__ count,
+                                                          const int64_t *__restrict__ first,
+                                                          int4 *rec, int4 *item) {
+  __shared__ int next[ROWS_CLASSES], base[ROWS_CLASSES + 1];
+  __shared__ int in_wave[ROWS_BUILD / 64][ROWS_CLASSES];
+  const int l = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int q0 = lvl[l], q1 = lvl[l + 1], nc = sh.classes();
+  if (t == 0) {
+    base[0] = 0;
+    for (int c = 0; c < ROWS_CLASSES; ++c) {
+      next[c] = base[c];
+      base[c + 1] = base[c] + count[l * ROWS_CLASSES + c];
+    }
+  }
+  __syncthreads();
+  int4 *const it = item + first[l];
+  for (int qb = q0; qb < q1; qb += ROWS_BUILD) {
+    const int q = qb + t;
+    const int c = q < q1 ? sh.cls(rp[q + 1] - 1 - rp[q]) : -1;
+    int rank = 0;
+    for (int k = 0; k < nc; ++k) {
+      const unsigned long long m = __ballot(c == k);
+      if (c == k) rank = __popcll(m & ((1ull << lane) - 1));
+      if (lane == 0) in_wave[wave][k] = __popcll(m);
+    }
+    __syncthreads();
+    if (c >= 0) {
+      int at = next[c] + rank;
+      for (int w = 0; w < wave; ++w) at += in_wave[w][c];
+      int4 r = make_int4(rp[q], rp[q + 1] - 1, perm[q], 0);
+      rec[q0 + at] = r;
+      if (c == 0) {
+        r.w = ROWS_KIND_GROUP;
+        for (int w = 0; w < sh.waves; ++w) it[(int64_t)at * sh.waves + w] = r;
+      }
+    }
+    __syncthreads();
+    if (t < nc)
+      for (int w = 0; w < ROWS_BUILD / 64; ++w) next[t] += in_wave[w][t];
+    __syncthreads();
+  }
+  int64_t at = (int64_t)base[1] * sh.waves;
+  for (int c = 1; c < nc; ++c) {
+    const int R = sh.rows(c), n = base[c + 1] - base[c], items = (n + R - 1) / R;
+    for (int i = t; i < items; i += ROWS_BUILD)
+      it[at + i] = make_int4(q0 + base[c] + i * R, min(R, n - i * R), 0, sh.kind(c));
+    at += items;
+  }
+  for (int64_t i = at + t; i < first[l + 1] - first[l]; i += ROWS_BUILD)
+    it[i] = make_int4(0, 0, 0, 0);
+}
+
+// The schedule for C column lanes, built on the device (a host pass over the
+// rows and the copies of their arrays took 6 ms of the first solve of the Zipf
+// matrix): the host only places the levels' items.
+int build_rows(symamd_plan p, int C, hipStream_t stream, RowSchedule &s) {
+  const RowShape sh(C);
+  const int L = p->levels;
+  struct Scratch {
+    hipStream_t stream;
+    int *count = nullptr;
+    int64_t *first = nullptr;
+    ~Scratch() {
+      if (count) (void)hipFreeAsync(count, stream);
+      if (first) (void)hipFreeAsync(first, stream);
+    }
+  } d{stream};
+  std::vector<int> count((size_t)L * ROWS_CLASSES);
+  std::vector<int64_t> first(L + 1, 0);
+  auto get = [](auto **q, size_t bytes, hipStream_t st) {
+    return hipMallocAsync((void **)q, bytes, st) == hipSuccess;
   };
-  std::vector<int4> rec(n > 0 ? n : 1), item;
-  int at = 0;
-  std::vector<int> first(lgmax + 4);
-  for (int l = 0; l < p->levels; ++l) {
-    const int q0 = p->h_lvl_ptr[l], q1 = p->h_lvl_ptr[l + 1];
-    std::fill(first.begin(), first.end(), 0);
-    for (int q = q0; q < q1; ++q) ++first[cls(q) + 1];
-    for (size_t i = 1; i < first.size(); ++i) first[i] += first[i - 1];
-    std::vector<int> next(first.begin(), first.end() - 1);
-    for (int q = q0; q < q1; ++q)
-      rec[at + next[cls(q)]++] = make_int4(rp[q], rp[q + 1] - 1, perm[q], 0);
-    for (int i = 0; i < first[1]; ++i) {
-      int4 r = rec[at + i];
-      r.w = ROWS_KIND_GROUP;
-      item.insert(item.end(), W, r);
-    }
-    for (int c = 1; c < lgmax + 3; ++c) {
-      const int lg = c == lgmax + 2 ? ROWS_KIND_SHORT : lgmax + 1 - c;
-      const int rows = c == lgmax + 2 ? smax * ROWS_PER_LANE : smax >> lg;
-      for (int i = first[c]; i < first[c + 1]; i += rows)
-        item.push_back(make_int4(at + i, std::min(rows, first[c + 1] - i), 0, lg));
-    }
-    while (item.size() % W) item.push_back(make_int4(0, 0, 0, 0));
-    at += q1 - q0;
-  }
-  s.tickets = (int)(item.size() / W);
-  if (hipMalloc(&s.d_rec, sizeof(int4) * rec.size()) != hipSuccess ||
-      hipMalloc(&s.d_item, sizeof(int4) * std::max<size_t>(item.size(), 1)) != hipSuccess) {
+  if (!get(&d.count, sizeof(int) * count.size(), stream) ||
+      !get(&d.first, sizeof(int64_t) * first.size(), stream)) {
     (void)hipGetLastError();
-    return fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", n);
+    return fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", p->n);
   }
-  SYMAMD_HIP(hipMemcpyAsync(s.d_rec, rec.data(), sizeof(int4) * rec.size(),
+  k_rows_count<<<L, ROWS_BUILD, 0, stream>>>(sh, p->d_lvl_ptr, p->d_rp, d.count);
+  SYMAMD_HIP(hipGetLastError());
+  SYMAMD_HIP(hipMemcpyAsync(count.data(), d.count, sizeof(int) * count.size(),
+                            hipMemcpyDeviceToHost, stream));
+  SYMAMD_HIP(hipStreamSynchronize(stream));
+  for (int l = 0; l < L; ++l) {
+    const int *n = &count[(size_t)l * ROWS_CLASSES];
+    int64_t items = (int64_t)n[0] * sh.waves;
+    for (int c = 1; c < sh.classes(); ++c) items += (n[c] + sh.rows(c) - 1) / sh.rows(c);
+    first[l + 1] = first[l] + (items + sh.waves - 1) / sh.waves * sh.waves;
+  }
+  s.tickets = (int)(first[L] / sh.waves);
+  if (hipMalloc(&s.d_rec, sizeof(int4) * std::max(p->n, 1)) != hipSuccess ||
+      hipMalloc(&s.d_item, sizeof(int4) * std::max<int64_t>(first[L], 1)) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", p->n);
+  }
+  SYMAMD_HIP(hipMemcpyAsync(d.first, first.data(), sizeof(int64_t) * first.size(),
                             hipMemcpyHostToDevice, stream));
-  SYMAMD_HIP(hipMemcpyAsync(s.d_item, item.data(), sizeof(int4) * item.size(),
-                            hipMemcpyHostToDevice, stream));
+  k_rows_fill<<<L, ROWS_BUILD, 0, stream>>>(sh, p->d_lvl_ptr, p->d_rp, p->d_perm, d.count, d.first,
+                                            s.d_rec, s.d_item);
+  SYMAMD_HIP(hipGetLastError());
+  // what was built serves solves on any stream from here on
   SYMAMD_HIP(hipStreamSynchronize(stream));
   return SYMAMD_OK;
 }
