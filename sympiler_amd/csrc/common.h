@@ -333,10 +333,13 @@ struct SplitLists {
 };
 
 // Schedule of the row executor (rows_exec.hip) for one number of column
-// lanes: rows in solving order and the items of every ticket.
+// lanes: rows in solving order and the items of every ticket.  Counted first
+// (tickets, and the rows of each class per level for the rest), built when a
+// solve takes it.
 struct RowSchedule {
   int4 *d_rec = nullptr;
   int4 *d_item = nullptr;
+  std::vector<int> count;
   int tickets = 0;
   bool failed = false;  // no memory for it: the unit executor
 };

@@ -301,6 +301,12 @@ struct RowShape {
   __host__ __device__ int rows(int c) const {
     return c == 0 ? 1 : c == lgmax + 2 ? smax * ROWS_PER_LANE : smax >> (lgmax + 1 - c);
   }
+  // tickets of a level with these counts
+  int64_t tickets(const int *count) const {
+    int64_t items = (int64_t)count[0] * waves;
+    for (int c = 1; c < classes(); ++c) items += (count[c] + rows(c) - 1) / rows(c);
+    return (items + waves - 1) / waves;
+  }
   __device__ int kind(int c) const { return c == lgmax + 2 ? ROWS_KIND_SHORT : lgmax + 1 - c; }
 };
 
@@ -380,73 +386,95 @@ __global__ __launch_bounds__(ROWS_BUILD) void k_rows_fill(RowShape sh,
     it[i] = make_int4(0, 0, 0, 0);
 }
 
-// The schedule for C column lanes, built on the device (a host pass over the
+// Device scratch given back to the stream.
+struct RowScratch {
+  hipStream_t stream;
+  std::vector<void *> ptrs;
+  explicit RowScratch(hipStream_t s) : stream(s) {}
+  ~RowScratch() {
+    for (void *q : ptrs) (void)hipFreeAsync(q, stream);
+  }
+  template <typename T>
+  bool get(T **q, size_t count) {
+    if (hipMallocAsync((void **)q, sizeof(T) * count, stream) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    ptrs.push_back(*q);
+    return true;
+  }
+};
+
+// The schedule for C column lanes is made on the device (a host pass over the
 // rows and the copies of their arrays took 6 ms of the first solve of the Zipf
-// matrix): the host only places the levels' items.
+// matrix); the host only adds up the levels' items.
+int count_rows(symamd_plan p, int C, hipStream_t stream, RowSchedule &s) {
+  const RowShape sh(C);
+  const int L = p->levels;
+  RowScratch scratch(stream);
+  int *d_count = nullptr;
+  s.count.resize((size_t)L * ROWS_CLASSES);
+  if (!scratch.get(&d_count, s.count.size()))
+    return fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", p->n);
+  k_rows_count<<<L, ROWS_BUILD, 0, stream>>>(sh, p->d_lvl_ptr, p->d_rp, d_count);
+  SYMAMD_HIP(hipGetLastError());
+  SYMAMD_HIP(hipMemcpyAsync(s.count.data(), d_count, sizeof(int) * s.count.size(),
+                            hipMemcpyDeviceToHost, stream));
+  SYMAMD_HIP(hipStreamSynchronize(stream));
+  int64_t tickets = 0;
+  for (int l = 0; l < L; ++l) tickets += sh.tickets(&s.count[(size_t)l * ROWS_CLASSES]);
+  s.tickets = (int)tickets;
+  return SYMAMD_OK;
+}
+
 int build_rows(symamd_plan p, int C, hipStream_t stream, RowSchedule &s) {
   const RowShape sh(C);
   const int L = p->levels;
-  struct Scratch {
-    hipStream_t stream;
-    int *count = nullptr;
-    int64_t *first = nullptr;
-    ~Scratch() {
-      if (count) (void)hipFreeAsync(count, stream);
-      if (first) (void)hipFreeAsync(first, stream);
-    }
-  } d{stream};
-  std::vector<int> count((size_t)L * ROWS_CLASSES);
+  RowScratch scratch(stream);
+  int *d_count = nullptr;
+  int64_t *d_first = nullptr;
   std::vector<int64_t> first(L + 1, 0);
-  auto get = [](auto **q, size_t bytes, hipStream_t st) {
-    return hipMallocAsync((void **)q, bytes, st) == hipSuccess;
-  };
-  if (!get(&d.count, sizeof(int) * count.size(), stream) ||
-      !get(&d.first, sizeof(int64_t) * first.size(), stream)) {
-    (void)hipGetLastError();
-    return fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", p->n);
-  }
-  k_rows_count<<<L, ROWS_BUILD, 0, stream>>>(sh, p->d_lvl_ptr, p->d_rp, d.count);
-  SYMAMD_HIP(hipGetLastError());
-  SYMAMD_HIP(hipMemcpyAsync(count.data(), d.count, sizeof(int) * count.size(),
-                            hipMemcpyDeviceToHost, stream));
-  SYMAMD_HIP(hipStreamSynchronize(stream));
-  for (int l = 0; l < L; ++l) {
-    const int *n = &count[(size_t)l * ROWS_CLASSES];
-    int64_t items = (int64_t)n[0] * sh.waves;
-    for (int c = 1; c < sh.classes(); ++c) items += (n[c] + sh.rows(c) - 1) / sh.rows(c);
-    first[l + 1] = first[l] + (items + sh.waves - 1) / sh.waves * sh.waves;
-  }
-  s.tickets = (int)(first[L] / sh.waves);
-  if (hipMalloc(&s.d_rec, sizeof(int4) * std::max(p->n, 1)) != hipSuccess ||
+  for (int l = 0; l < L; ++l)
+    first[l + 1] = first[l] + sh.waves * (int64_t)sh.tickets(&s.count[(size_t)l * ROWS_CLASSES]);
+  if (!scratch.get(&d_count, s.count.size()) || !scratch.get(&d_first, first.size()) ||
+      hipMalloc(&s.d_rec, sizeof(int4) * std::max(p->n, 1)) != hipSuccess ||
       hipMalloc(&s.d_item, sizeof(int4) * std::max<int64_t>(first[L], 1)) != hipSuccess) {
     (void)hipGetLastError();
     return fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", p->n);
   }
-  SYMAMD_HIP(hipMemcpyAsync(d.first, first.data(), sizeof(int64_t) * first.size(),
+  SYMAMD_HIP(hipMemcpyAsync(d_count, s.count.data(), sizeof(int) * s.count.size(),
                             hipMemcpyHostToDevice, stream));
-  k_rows_fill<<<L, ROWS_BUILD, 0, stream>>>(sh, p->d_lvl_ptr, p->d_rp, p->d_perm, d.count, d.first,
+  SYMAMD_HIP(hipMemcpyAsync(d_first, first.data(), sizeof(int64_t) * first.size(),
+                            hipMemcpyHostToDevice, stream));
+  k_rows_fill<<<L, ROWS_BUILD, 0, stream>>>(sh, p->d_lvl_ptr, p->d_rp, p->d_perm, d_count, d_first,
                                             s.d_rec, s.d_item);
   SYMAMD_HIP(hipGetLastError());
   // what was built serves solves on any stream from here on
   SYMAMD_HIP(hipStreamSynchronize(stream));
+  std::vector<int>().swap(s.count);
   return SYMAMD_OK;
 }
 
-// The schedule, built on first use.  While a caller records the handle's
-// stream it is built on a stream of its own (rows_path has seen that one was
-// built before, so the plan's arrays are in place).  Without the memory the
-// plan remembers so, for this number of column lanes.
-int rows_schedule(symamd_handle h, symamd_plan p, int C, RowSchedule **out) {
+// The schedule, counted or built on first use.  While a caller records the
+// handle's stream that is done on a stream of its own (rows_path has seen that
+// one was counted before, so the plan's arrays are in place).  Without the
+// memory the plan remembers so, for this number of column lanes.
+int rows_schedule(symamd_handle h, symamd_plan p, int C, bool build, RowSchedule **out) {
   auto found = p->rows.find(C);
-  if (found == p->rows.end()) {
+  if (found == p->rows.end() || (build && !found->second.d_rec && !found->second.failed)) {
     const bool cap = capturing(h->stream);
     RelaxedCapture relaxed;
     hipStream_t own = nullptr;
     if (cap) SYMAMD_HIP(hipStreamCreateWithFlags(&own, hipStreamNonBlocking));
+    const hipStream_t stream = cap ? own : h->stream;
     RowSchedule s;
-    int rc;
+    int rc = SYMAMD_OK;
     try {
-      rc = build_rows(p, C, cap ? own : h->stream, s);
+      if (found != p->rows.end())
+        s = found->second;
+      else
+        rc = count_rows(p, C, stream, s);
+      if (rc == SYMAMD_OK && build) rc = build_rows(p, C, stream, s);
     } catch (const std::bad_alloc &) {
       rc = fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", p->n);
     }
@@ -458,11 +486,32 @@ int rows_schedule(symamd_handle h, symamd_plan p, int C, RowSchedule **out) {
       s = RowSchedule();
       s.failed = true;
     }
-    found = p->rows.emplace(C, s).first;
+    found = p->rows.insert_or_assign(C, std::move(s)).first;
   }
   *out = &found->second;
   return found->second.failed ? fail(SYMAMD_ERR_ALLOC, "row schedule for %d rows", p->n)
                               : SYMAMD_OK;
+}
+
+// Whether the tickets take no longer than the units would.  The unit executor
+// spends its time on levels (about 9 us each, and 0.25 us for every entry that
+// a lane of the longest row adds) and, where those are wide, on entries (18 ps
+// each) and right-hand sides (17 ps a value, 10 up to eight columns); this one
+// on tickets, which workgroups take from one counter (13 ns each; 14 with 8 or
+// 16 column lanes).  So long chains of narrow levels run here and few wide
+// levels on the units.  In ms, units / here, the side taken first: 27-point grid
+// of 96^3 in natural order (666 levels) k = 1 2.90 / 1.03, k = 32 4.40 / 1.78
+// (here); in eight colours 0.16 / 0.40, 0.82 / 1.15 (units); 20 levels of
+// 20,000 rows of 12 entries k = 1 0.22 / 0.17 (here), k = 32 0.54 / 0.71
+// (units); 100 levels of 4,000 k = 32 1.14 / 0.76 (here); 40 of 8,000 rows of 40
+// entries k = 1 0.49 / 0.49, k = 32 0.91 / 3.78 (units); two levels, 300,000 rows
+// of 64 entries, 0.36 / 0.42, 0.62 / 3.29 (units); 64 levels of 1,500 rows of up
+// to 63 entries k = 32 0.64 / 0.70 (here, the largest miss).
+bool tickets_win(symamd_plan p, int k, int lanes, int tile, int tickets) {
+  const int C = rows_cols(k), eff = std::max(1, std::min(lanes, 64 / tile_cols(k, tile)));
+  const double units = p->levels * (9000.0 + 250.0 * p->max_row_nnz / eff) + 0.018 * p->nnz +
+                       (k <= 8 ? 0.010 : 0.017) * p->n * k;
+  return tickets * (C == 8 || C == 16 ? 14.0 : 13.0) <= units;
 }
 
 template <typename T, int C>
@@ -487,7 +536,7 @@ int launch_rows_t(symamd_handle h, symamd_plan p, void *d_B, int k, int64_t ld, 
                   int64_t cs, bool turn) {
   RowSchedule *s = nullptr;
   const int C = rows_cols(k);
-  SYMAMD_TRY(rows_schedule(h, p, C, &s));
+  SYMAMD_TRY(rows_schedule(h, p, C, true, &s));
   const int64_t count = (int64_t)p->n * k;
   RowArgs<T> a{};
   a.rec = s->d_rec;
@@ -541,23 +590,27 @@ static size_t rows_bytes(symamd_plan p, int k, bool turn) {
 // either the tuner timed it so or, untuned, several lanes per row fit beside
 // the unit executor's column tile (one lane per row keeps the reference's
 // order in every row, which that one does; so it also solves untuned blocks of
-// more than 32 columns).  A solve being recorded by the caller needs an
-// earlier one here, as the unit executor does.
+// more than 32 columns) and the tickets take no longer.  A solve being recorded
+// by the caller needs an earlier one, as the unit executor does; it runs here
+// where the units it would need were not built by that one.
 bool rows_path(symamd_handle h, symamd_plan p, int k, bool turn, int exec, const Choice &c) {
   if (exec != SYMAMD_EXEC_SYNCFREE || c.rows == 0 || h->unmarked || h->trace ||
-      rows_bytes(p, k, turn) >= p->rows_limit)
+      rows_bytes(p, k, turn) >= p->rows_limit || p->n == 0)
     return false;
   if (c.rows < 0 && (c.lanes < 2 || 2 * tile_cols(k, c.tile) > 64)) return false;
-  const auto s = p->rows.find(rows_cols(k));
-  if (s != p->rows.end()) return !s->second.failed;
-  return !p->rows.empty() || !capturing(h->stream);
+  const bool cap = capturing(h->stream);
+  if (cap && p->rows.empty()) return false;
+  RowSchedule *s = nullptr;
+  if (rows_schedule(h, p, rows_cols(k), false, &s) != SYMAMD_OK) return false;
+  if (c.rows > 0 || tickets_win(p, k, c.lanes, c.tile, s->tickets)) return true;
+  return cap && !p->units.count(2 * forward_rows_per_unit(k, c.lanes, c.tile));
 }
 
 // The schedule and the workspace, before any launch or capture.  A workspace
 // that did not fit is not asked for again, nor is a larger one.
 int prepare_rows(symamd_handle h, symamd_plan p, int k, bool turn) {
   RowSchedule *s = nullptr;
-  SYMAMD_TRY(rows_schedule(h, p, rows_cols(k), &s));
+  SYMAMD_TRY(rows_schedule(h, p, rows_cols(k), true, &s));
   const size_t bytes = rows_bytes(p, k, turn);
   const int rc = plan_workspace(h, p, bytes);
   if (rc == SYMAMD_ERR_ALLOC) p->rows_limit = bytes;
