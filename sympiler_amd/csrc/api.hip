@@ -936,8 +936,7 @@ int symamd_tune(symamd_handle h, symamd_plan plan, int k, symamd_layout layout,
       for (int t = 8; t < tile_cols(k, 0); t *= 2) tiles.push_back(t);
     // region caps: for single right-hand sides 512 and 1024 rows (whichever
     // schedule fits; the cap of the handle, when set, alone), and the untuned
-    // cap where it is another: 512 uneven systems of 8.2M rows take 0.42 ms
-    // a replay at 384 and 0.49 ms at 512
+    // cap where it is another
     std::vector<int> caps = {0};
     if (ex == SYMAMD_EXEC_REGIONS && k == 1 && h->region_cap == 0) {
       caps = {512, 1024};

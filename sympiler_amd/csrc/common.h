@@ -4,6 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstddef>
 #include <cstdint>
@@ -582,9 +583,12 @@ int launch_grad_l(symamd_handle h, symamd_plan p, const void *d_X, const void *d
 // the region's and its halo's values of one column group per row), unless
 // the handle sets one.
 int region_cap(symamd_handle h, symamd_plan p, int k);
-// Over 16 tasks of 1024 rows per CU: single right-hand sides take smaller ones.
+// Plans whose single right-hand sides take smaller regions: more than 16 tasks
+// of 1024 rows per CU, levels of more than 40 rows per CU and at most 2.5
+// entries below the diagonal a row (see region_cap).
 inline bool large_for_regions(symamd_handle h, symamd_plan p) {
-  return p->n > 16 * 1024 * h->num_cus;
+  return p->n > 16 * 1024 * h->num_cus && p->n / std::max(p->levels, 1) > 40 * h->num_cus &&
+         p->avg_row_nnz <= 3.5;
 }
 // The region cap the tuner chose for k right-hand sides (either layout), or 0.
 int tuned_region_cap(symamd_plan p, int k);

@@ -1125,9 +1125,15 @@ int region_waves(symamd_handle h, int k) {
 // 512 otherwise (measured on the IC(0) factors of the 128^3 and 64^3
 // Laplacians: k = 1 with the memory wave 0.309 / 0.137 ms at 1024 vs
 // 0.323 / 0.142 ms at 512; k = 32 with four waves per task is fastest at
-// 512).  Past 16 tasks of 1024 rows per CU the tasks, not the chain, set the
-// time, and smaller ones run more to a CU: the batch of 512 grids (8.4 M rows)
-// takes 0.42 / 0.48 / 0.55 ms at 384 / 512 / 1024 rows (0.55 at 256).
+// 512).  Many planes side by side take smaller regions: past 16 tasks of 1024
+// rows per CU whose levels are wide, the tasks, not the chain, set the time, and
+// smaller ones run more to a CU; in three dimensions their halos outweigh that,
+// and a chain gets longer.  In ms at 384 / 512 / 1024 rows: 512 planes of 32 to
+// 224 a side (8.2M rows, 18,700 a level) 0.46 / 0.52 / 0.56, 300 of them (10,900
+// a level) 0.36 / 0.38 / 0.38, 24 of 400 to 700 (5,500 a level) 0.82 / 0.75 /
+// 0.64; one plane of 3000^2 (1,500) 2.80 / 2.66 / 2.40; one grid of 200^3
+// (13,400) 0.74 / 0.64 / 0.66, of 256^3 1.02 / 0.92 / 0.96; 40 grids of 50^3
+// (33,800) 0.41 / 0.28 / 0.29.
 int region_cap(symamd_handle h, symamd_plan p, int k) {
   if (h->region_cap > 0) return h->region_cap;
   const int tuned = p ? tuned_region_cap(p, k) : 0;
