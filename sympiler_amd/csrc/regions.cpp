@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <climits>
 #include <cstdint>
 #include <cstring>
@@ -86,10 +87,15 @@ int64_t box_rounds(int64_t a, int64_t b, int64_t c) {
 // for a single right-hand side 8 x 8 x 16 where 1024 rows are allowed.
 // (10 x 10 x 10 boxes have a shorter chain, but levels of 75 rows: 0.331 ms
 // against 0.295.)  Boxes of uneven sides measured 8 % above this estimate in 3D
-// (8 x 10 x 10 there: 0.312 ms), not in a plane (300 x 500: 30 x 34 boxes 0.313
-// ms, 20 x 50 ones 0.377).
-void lattice_cut(int64_t nx, int64_t ny, int64_t nz, int max_rows, double hop, double round,
+// (8 x 10 x 10 there: 0.312 ms).  In a plane, for a single right-hand side,
+// oblong boxes lag behind it the more the longer the chain is: 40 x 25 ones by
+// 6 % on 500^2 (a chain of 32), 13 % on 1024^2 (66), 15 % on 2000^2 (129);
+// 42 x 24 ones by 20 % on 1500 x 500, 0.852 ms against 0.767 of 32 x 32 ones;
+// on 100^2 and 300^2 (6, 18) they do not.  Narrow strips are cut as before: 8
+// boxes across 30 x 30,000 take 8.6 ms, 3 take 9.6.
+void lattice_cut(int64_t nx, int64_t ny, int64_t nz, int max_rows, bool banded,
                  int64_t (&pieces)[3]) {
+  const double hop = banded ? 3.6 : 4.4, round = banded ? 0.14 : 0.44;
   const int64_t dim[3] = {nx, ny, nz};
   double best = 0.0;
   pieces[0] = 0;
@@ -112,8 +118,13 @@ void lattice_cut(int64_t nx, int64_t ny, int64_t nz, int max_rows, double hop, d
         if (pieces[0] != 0 && chain * hop >= best) break;
         if (a * b * c > max_rows) continue;
         const bool uneven = nz > 1 && (nx % a || ny % b || nz % c);
-        const double cost =
-            chain * (hop + round * (double)box_rounds(a, b, c)) * (uneven ? 1.08 : 1.0);
+        const double oblong =
+            nz == 1 && banded
+                ? std::min(0.25, 0.3 * std::log((double)std::max(a, b) / (double)std::min(a, b))) *
+                      std::min(1.0, std::max(0.0, (chain - 12.0) / 48.0))
+                : 0.0;
+        const double cost = chain * (hop + round * (double)box_rounds(a, b, c)) *
+                            (uneven ? 1.08 : 1.0 + oblong);
         if (pieces[0] == 0 || cost < best) {
           best = cost;
           pieces[0] = px;
@@ -169,8 +180,7 @@ bool lattice_regions(int n, const int *Lp, const int *Li, int max_rows, bool ban
           const int64_t d = (int64_t)i - Li[j], at = i - a;
           if ((d == 1 && at % r.d[1] == 0) || (d == r.d[1] && at % r.d[2] < r.d[1])) return false;
         }
-      lattice_cut(r.d[1], r.d[2] / r.d[1], r.rows / r.d[2], max_rows,
-                  banded ? 3.6 : 4.4, banded ? 0.14 : 0.44, r.pieces);
+      lattice_cut(r.d[1], r.d[2] / r.d[1], r.rows / r.d[2], max_rows, banded, r.pieces);
       ++grids;
     }
     runs.push_back(r);
