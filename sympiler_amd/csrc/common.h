@@ -541,8 +541,10 @@ int launch_lbc(symamd_handle h, int n, const int *d_Lp, const int *d_Li,
                const int *d_partition);
 // Regions (regions.cpp): clustering of the rows, the region-ordered level
 // permutation of a plan, and the owner schedule of a unit set for nw waves.
+// boxes, when given: grids in natural order are cut into boxes; says whether
+// they were.
 int cluster_regions(int n, const int *Lp, const int *Li, int max_rows, bool banded,
-                    std::vector<int> &region);
+                    std::vector<int> &region, bool *boxes);
 int order_by_regions(symamd_handle h, symamd_plan p, const int *d_Lp, const int *d_Li);
 int plan_owners(symamd_handle h, symamd_plan p, UnitSet *us, int nw);
 // Region schedule of the plan for region cap `cap` and the band of k

@@ -22,6 +22,7 @@
 #include <climits>
 #include <cstdint>
 #include <cstring>
+#include <map>
 #include <numeric>
 #include <thread>
 #include <vector>
@@ -77,6 +78,10 @@ int64_t box_rounds(int64_t a, int64_t b, int64_t c) {
   return rounds;
 }
 
+// Costs of the region kernel for a block of right-hand sides, in us: a hand-off
+// and 64 rows of a level.
+constexpr double BLOCK_HOP = 4.4, BLOCK_ROUND = 0.44;
+
 // How a grid of nx x ny x nz points (nz = 1: a plane) is cut into boxes: of
 // all cuts into px x py x pz equal boxes (sides differing by at most one) of
 // at most max_rows points, the one whose longest chain of boxes takes least,
@@ -95,7 +100,7 @@ int64_t box_rounds(int64_t a, int64_t b, int64_t c) {
 // boxes across 30 x 30,000 take 8.6 ms, 3 take 9.6.
 void lattice_cut(int64_t nx, int64_t ny, int64_t nz, int max_rows, bool banded,
                  int64_t (&pieces)[3]) {
-  const double hop = banded ? 3.6 : 4.4, round = banded ? 0.14 : 0.44;
+  const double hop = banded ? 3.6 : BLOCK_HOP, round = banded ? 0.14 : BLOCK_ROUND;
   const int64_t dim[3] = {nx, ny, nz};
   double best = 0.0;
   pieces[0] = 0;
@@ -204,12 +209,13 @@ bool lattice_regions(int n, const int *Lp, const int *Li, int max_rows, bool ban
 }  // namespace
 
 int cluster_regions(int n, const int *Lp, const int *Li, int max_rows, bool banded,
-                    std::vector<int> &region) {
+                    std::vector<int> &region, bool *boxes) {
   region.resize(n);
   std::iota(region.begin(), region.end(), 0);
   if (n == 0 || max_rows < 2) return n;
-  int boxes = 0;
-  if (lattice_regions(n, Lp, Li, max_rows, banded, region, boxes)) return boxes;
+  int count = 0;
+  if (boxes && (*boxes = lattice_regions(n, Lp, Li, max_rows, banded, region, count)))
+    return count;
   WGraph g = initial_graph(n, Lp, Li);
   std::vector<int> size(n, 1);
   int nc = n;
@@ -332,7 +338,8 @@ int order_by_regions(symamd_handle h, symamd_plan p, const int *d_Lp, const int 
   SYMAMD_HIP(hipMemcpy(Li.data(), d_Li, sizeof(int) * p->nnz, hipMemcpyDeviceToHost));
   SYMAMD_HIP(hipMemcpy(perm.data(), p->d_perm, sizeof(int) * n, hipMemcpyDeviceToHost));
   std::vector<int> reg;
-  const int R = cluster_regions(n, Lp.data(), Li.data(), h->region_rows, false, reg);
+  bool boxes = false;
+  const int R = cluster_regions(n, Lp.data(), Li.data(), h->region_rows, false, reg, &boxes);
   int64_t inside = 0, off = 0;
   for (int i = 0; i < n; ++i)
     for (int j = Lp[i]; j < Lp[i + 1]; ++j)
@@ -603,6 +610,50 @@ int make_acyclic(int n, const int *Lp, const int *Li, const std::vector<int> &le
   return m;
 }
 
+// The longest chain of regions for a block of right-hand sides, at lattice_cut's
+// costs; the region graph has no cycle.
+double chain_cost(int n, const int *Lp, const int *Li, const std::vector<int> &lev,
+                  const std::vector<int> &reg, int R) {
+  std::vector<std::map<int, int>> rows(R);  // per region: rows of each level
+  std::vector<std::vector<int>> succ(R);
+  std::vector<int> indeg(R, 0), ready;
+  for (int i = 0; i < n; ++i) {
+    ++rows[reg[i]][lev[i]];
+    for (int j = Lp[i]; j < Lp[i + 1] - 1; ++j)
+      if (reg[Li[j]] != reg[i]) {
+        succ[reg[Li[j]]].push_back(reg[i]);
+        ++indeg[reg[i]];
+      }
+  }
+  for (int r = 0; r < R; ++r)
+    if (indeg[r] == 0) ready.push_back(r);
+  std::vector<double> before(R, 0.0);
+  double longest = 0.0;
+  for (size_t q = 0; q < ready.size(); ++q) {
+    const int r = ready[q];
+    int rounds = 0;
+    for (const auto &l : rows[r]) rounds += (l.second + 63) / 64;
+    const double end = before[r] + BLOCK_HOP + BLOCK_ROUND * rounds;
+    longest = std::max(longest, end);
+    for (int s : succ[r]) {
+      before[s] = std::max(before[s], end);
+      if (--indeg[s] == 0) ready.push_back(s);
+    }
+  }
+  return longest;
+}
+
+// Grids of at most this many rows have few boxes, and the matching's uneven
+// regions can have the shorter chain: for a block of right-hand sides it is
+// taken where its estimate is BOXES_LEAD below the boxes' (which it reaches only
+// so far: its regions have larger halos).  13 columns, in us, estimates and
+// times of the matching / the boxes: 24^2 29.5 / 39.6, 40.2 / 47.1; 37^2 45.3 /
+// 60.7, 55.5 / 61.5; 20 x 100 70 / 91, 75.6 / 82.3; 10^3 23.8 / 29.0, 40.1 /
+// 42.8; and the other way 42^2 80.5 / 67.3, 81.8 / 66.8; 9 x 13 x 17 44.9 /
+// 48.4, 62.1 / 54.3.
+constexpr int FEW_BOXES_ROWS = 4096;
+constexpr double BOXES_LEAD = 0.85;
+
 }  // namespace
 
 // Host part, from the level-ordered copy (perm, crp, cci: position -> row,
@@ -622,8 +673,19 @@ bool build_region_schedule(int n, int64_t nnz, int levels, const int *lvl_ptr,
   for (int i = 0; i < n; ++i)
     std::copy(cci.begin() + crp[ipos[i]], cci.begin() + crp[ipos[i] + 1], Li.begin() + Lp[i]);
   std::vector<int> reg;
-  int R = cluster_regions(n, Lp.data(), Li.data(), cap, band_slices < 255, reg);
+  bool boxes = false;
+  int R = cluster_regions(n, Lp.data(), Li.data(), cap, band_slices < 255, reg, &boxes);
   R = make_acyclic(n, Lp.data(), Li.data(), lev, cap, reg, R);
+  if (boxes && band_slices >= 255 && n <= FEW_BOXES_ROWS) {
+    std::vector<int> other;
+    int S = cluster_regions(n, Lp.data(), Li.data(), cap, false, other, nullptr);
+    S = make_acyclic(n, Lp.data(), Li.data(), lev, cap, other, S);
+    if (chain_cost(n, Lp.data(), Li.data(), lev, other, S) <
+        BOXES_LEAD * chain_cost(n, Lp.data(), Li.data(), lev, reg, R)) {
+      reg.swap(other);
+      R = S;
+    }
+  }
   int64_t inside = 0, offd = 0;
   for (int i = 0; i < n; ++i)
     for (int j = Lp[i]; j < Lp[i + 1] - 1; ++j) {

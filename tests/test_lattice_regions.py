@@ -99,3 +99,18 @@ def test_boxes_of_planes_for_one_column(nx, ny, boxes, chain):
     36 x 21 of 42 x 24 points, 0.87 ms against 0.77), short ones the fewest."""
     sch = schedule_host(*W.lap2d_tril(nx, ny), 1024, 4)
     assert sch["R"] == boxes[0] * boxes[1] and depth(sch) == chain
+
+
+@pytest.mark.parametrize("grid,regions", [((37, 37), 3), ((24, 24), 2), ((10, 10, 10), 2),
+                                          ((42, 42), 4), ((9, 13, 17), 8)])
+def test_few_boxes_against_the_matching(grid, regions):
+    """Small grids and blocks of right-hand sides: the matching's regions where
+    their chain is clearly shorter (37 x 37 in 3 regions instead of 4 boxes, 24 x
+    24 and 10^3 in uneven ones), boxes elsewhere."""
+    M = W.lap2d_tril(*grid) if len(grid) == 2 else W.lap3d_tril(*grid, 6.01, -1.0)
+    sch, _ = check(*M, 512, 255)
+    rows = sorted(len(r["rows"]) for r in _records(sch))
+    assert sch["R"] == regions
+    if regions == 2:
+        levels = sum(len(r["slices"]) - 1 for r in _records(sch))
+        assert rows[0] < rows[1] or levels < 2 * 22, (rows, levels)  # boxes: 22 each
