@@ -894,7 +894,7 @@ __global__ __launch_bounds__(64 * (NC + 1 + MK)) void k_regions_mw(RegionArgs<T>
       const int nx = __builtin_amdgcn_readlane(ticket, 0);
       if (lane < 8) s_ctl[1 + lane] = nx < ntasks ? a.head[8 * (nx / a.groups) + lane] : 0;
       if (lane == 0) s_ctl[0] = nx;
-      if (lane == 0) trace_mark(a.trace, a.trace_cap, task, 2);
+      if (!MK && lane == 0) trace_mark(a.trace, a.trace_cap, task, 2);
     } else if (storew) {
       // the rows of every band the compute waves have finished (a value is
       // stored after the mark of its row: the band's halo was loaded after the
@@ -923,6 +923,7 @@ __global__ __launch_bounds__(64 * (NC + 1 + MK)) void k_regions_mw(RegionArgs<T>
           __builtin_amdgcn_s_sleep(1);
         }
       }
+      trace_mark(a.trace, a.trace_cap, task, 2);
       if (a.gL && graded < nb)
         grad_bands<T>(a.gL, xs, reinterpret_cast<const T *>(smem + a.xfb), rb, L, lsl, lband,
                       graded, nb, nr, ns, ne);
