@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <map>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/sympiler_amd.h"
@@ -430,6 +431,8 @@ struct symamd_snplan_s {
   int n = 0, m = 0, kcap = 1;  // kcap: columns d_T and d_flags hold
   int ntasks = 0;              // tops and 128-row chunks below (bounds the columns accepted)
   int tickets = 0, ttickets = 0;
+  // forward, transposed: numbers of tickets a level has, and of such levels
+  std::vector<std::pair<int, int>> widths[2];
   int64_t tcount = 0;
   int *d_tdst = nullptr, *d_rowb = nullptr, *d_list = nullptr;
   int *d_unit = nullptr, *d_dlist = nullptr, *d_tunit = nullptr, *d_tdlist = nullptr;

@@ -45,6 +45,7 @@
 // in flight, gathered lists and turned tiles; 32 right-hand sides 4.6 + 6.9,
 // 1.71 + 1.50, 1.34 + 1.27.
 #include <algorithm>
+#include <map>
 #include <vector>
 
 #include "device.h"
@@ -1010,6 +1011,7 @@ struct SnSchedule {
   std::vector<int> top;               // per supernode: the slot that solves its top
   std::vector<int> group;             // per supernode: the slot of its first group, or -1
   std::vector<int> first;             // per supernode: the slot of its first chunk, or -1
+  std::map<int, int> widths;          // tickets of a level -> levels
   std::vector<int> dlist;
 };
 
@@ -1035,6 +1037,7 @@ void sn_schedule(int m, const int *h_sup, const int *h_nrows, const int *h_Lp,
     while (s.unit.size() % 4) s.unit.push_back({0, 0, 0, SN_NARROW_UNIT, 0, 0, 0, 0});
   };
   for (int a = 0, b = 0; a < m; a = b) {
+    const size_t before = s.unit.size();
     while (b < m && lev[order[b]] == lev[order[a]]) ++b;
     for (int j = a; j < b; ++j)
       if (!narrow(order[j]) &&
@@ -1061,6 +1064,7 @@ void sn_schedule(int m, const int *h_sup, const int *h_nrows, const int *h_Lp,
           close();
         }
       }
+    ++s.widths[(int)((s.unit.size() - before) / 4)];
   }
   s.deps.assign(s.unit.size(), {});
 }
@@ -1196,6 +1200,8 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
   q->ntasks = old_tasks;
   q->tickets = (int)(fwd.unit.size() / 4);
   q->ttickets = (int)(bwd.unit.size() / 4);
+  q->widths[0].assign(fwd.widths.begin(), fwd.widths.end());
+  q->widths[1].assign(bwd.widths.begin(), bwd.widths.end());
   const int64_t flags = 4 * (int64_t)std::max(1, std::max(q->tickets, q->ttickets));
   int rc = SYMAMD_OK;
   auto up = [&](int **dst, const int *src, size_t count) {
@@ -1227,6 +1233,38 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
   return SYMAMD_OK;
 }
 
+// Columns per tile: a row's entries are loaded once for the columns of a tile,
+// but each step of a top's chain then divides for all of them.  On the 13-level
+// factor, forward + transposed with tiles of 1 / 2 / 4: k = 2 0.86 / 0.93 / - ms,
+// k = 4 1.11 / 1.02 / 1.32 ms, k = 13 2.30 / 1.76 / 1.83 ms, k = 32 4.94 / 3.17 /
+// 2.61 ms.  Where the levels hold few tickets the chain is all there is, and
+// narrower tiles run side by side: a level takes 1 / 1.27 / 1.9 times as long
+// with tiles of 1 / 2 / 4 columns (about 5 us with one), once per SN_BUSY
+// tickets, and each ticket 12.5 ns of the counter.  Forward, k = 32, in ms with
+// tiles of 1 / 2 / 4: 600 supernodes of 64 columns in 364 levels 3.23 / 4.01 /
+// 5.98, 20,000 of 4 columns in 635 levels 3.27 / 3.08 / 4.01, of 1 column in 157
+// 2.78 / 1.68 / 1.25, the 13-level factor 2.47 / 1.60 / 1.37.
+static int sn_widest_tile(int k) { return k < 4 ? 1 : k < 16 ? 2 : 4; }
+static int sn_tile(const std::vector<std::pair<int, int>> &widths, int64_t tickets, int k) {
+  constexpr double SN_BUSY = 128.0, CHAIN[3] = {1.0, 1.27, 1.9};
+  const int widest = sn_widest_tile(k);
+  int best = widest;
+  double least = 0.0;
+  for (int kt = widest, i = widest / 2; kt >= 1; kt /= 2, i = kt / 2) {
+    const double tiles = (k + kt - 1) / kt;
+    if (kt < widest && tickets * tiles >= INT_MAX) break;
+    double us = 0.0;
+    for (const auto &w : widths)
+      us += w.second * (5.0 * CHAIN[i] * std::max(1.0, w.first * tiles / SN_BUSY) +
+                        0.0125 * w.first * tiles);
+    if (kt == widest || us < 0.92 * least) {
+      least = us;
+      best = kt;
+    }
+  }
+  return best;
+}
+
 int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_x, int k,
              int64_t ldx, bool transposed) {
   if (q->m == 0 || k == 0) return SYMAMD_OK;
@@ -1235,23 +1273,19 @@ int sn_solve(symamd_handle h, symamd_snplan_s *q, const double *d_Lx, double *d_
     return fail(SYMAMD_ERR_NOT_SUPPORTED,
                 "supernodal solve: %d tasks x %d columns exceed the 32-bit ticket range; "
                 "solve the columns in smaller batches", q->ntasks, k);
-  // columns per tile: a row's entries are loaded once for the columns of a
-  // tile, but each step of a top's chain then divides for all of them.  On
-  // the 13-level factor, forward + transposed with tiles of 1 / 2 / 4: k = 2
-  // 0.86 / 0.93 / - ms, k = 4 1.11 / 1.02 / 1.32 ms, k = 13 2.30 / 1.76 / 1.83
-  // ms, k = 32 4.94 / 3.17 / 2.61 ms.
-  const int kt = k < 4 ? 1 : k < 16 ? 2 : 4;
+  const int kt = sn_tile(q->widths[transposed], transposed ? q->ttickets : q->tickets, k);
   const int tiles = (k + kt - 1) / kt;
-  // temporaries and tags for the tiles' columns; those that a caller's graph
-  // reads stay until the plan is destroyed
+  // temporaries and tags for the columns of whole tiles; those that a caller's
+  // graph reads stay until the plan is destroyed
   const bool cap = capturing(h->stream);
-  if (tiles * kt > q->kcap) {
+  const int widest = sn_widest_tile(k);
+  const int64_t cols = ((int64_t)k + widest - 1) / widest * widest;
+  if (cols > q->kcap) {
     if (cap)
       return fail(SYMAMD_ERR_NOT_SUPPORTED,
                   "supernodal temporaries for %d columns not prepared before capture", k);
     double *T = nullptr;
     int *flags = nullptr;
-    const int64_t cols = (int64_t)tiles * kt;
     const int64_t tc = q->tcount > 0 ? q->tcount : 1;
     const int64_t nt = 4 * (int64_t)std::max(1, std::max(q->tickets, q->ttickets));
     if (hipMalloc(&T, sizeof(double) * tc * cols) != hipSuccess ||

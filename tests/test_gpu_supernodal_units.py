@@ -117,3 +117,46 @@ def test_long_lists_gathered_ahead_of_wide_tops(dev, k):
     got = X.cpu().numpy()
     for c in range(k):
         assert bitwise_equal(got[c], oracle.sptrsv_csc_block(sup, nrows, Lp, Li, Lx, B[c])), c
+
+
+@pytest.mark.parametrize("k", [16, 33])
+def test_chains_of_narrow_supernodes(dev, k):
+    """One supernode after another: tiles of one column run side by side, and a
+    block takes no longer than its columns' chain (in tiles of four, 1.9 times
+    as long as one column)."""
+    import torch
+    m, w = 300, 40
+    sup = (np.arange(m + 1) * w).astype(np.int32)
+    n = m * w
+    nrows = np.full(m, 2 * w, np.int32)
+    nrows[-1] = w
+    Lp = np.concatenate([[0], np.cumsum(nrows * w)]).astype(np.int32)
+    Li = np.concatenate([np.tile(np.arange(i * w, i * w + nrows[i]), w) for i in range(m)])
+    rng = np.random.default_rng(5)
+    Lx = rng.uniform(-1, 1, len(Li)) / (2 * w)
+    for i in range(m):
+        Lx[Lp[i] + np.arange(w) * (nrows[i] + 1)] = 1.5
+    plan = sa.SupernodalPlan(sup, nrows, Lp, Li.astype(np.int32))
+    dLx = to_dev(Lx)
+    B = W.uniform(36, 0, k * n).reshape(k, n)
+
+    def best(X):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        ms = []
+        for _ in range(6):
+            X.zero_()
+            X.add_(1.0)
+            e[0].record()
+            plan.solve(dLx, X)
+            e[1].record()
+            e[1].synchronize()
+            ms.append(e[0].elapsed_time(e[1]))
+        return min(ms)
+
+    X = to_dev(B.copy())
+    plan.solve(dLx, X)
+    plan.check()
+    got = X.cpu().numpy()
+    for c in range(k):
+        assert bitwise_equal(got[c], oracle.sptrsv_csc_block(sup, nrows, Lp, Li, Lx, B[c])), c
+    assert best(X) < 1.5 * best(X[0])
