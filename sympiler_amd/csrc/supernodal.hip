@@ -231,12 +231,13 @@ struct Diag {
 // is broadcast, and every later row subtracts its product; TRANS takes the
 // columns from the last one.  res keeps a lane's quotient.  Lanes already
 // solved, and lanes past the last column, go on computing values that nothing
-// reads.  entry(j) loads m[j] again, for the block whose quotients need the
-// division.
-template <int KT, bool TRANS, typename Entry>
+// reads.  A block whose quotients need the division (zeros of the right-hand
+// side do) is done again step by step, with entries picked from m: loading them
+// once more put a memory round trip on each step.
+template <int KT, bool TRANS>
 __device__ __forceinline__ void solve_block(double (&acc)[KT], double (&res)[KT],
                                             const double (&m)[8], const Diag &dg, int lb, int B,
-                                            int lane, Entry entry) {
+                                            int lane) {
   double start[KT];
 #pragma unroll
   for (int c = 0; c < KT; ++c) start[c] = acc[c];
@@ -262,7 +263,13 @@ __device__ __forceinline__ void solve_block(double (&acc)[KT], double (&res)[KT]
 #pragma unroll 1
     for (int t = 0; t < min(B, 8); ++t) {
       const int j = TRANS ? min(B, 8) - 1 - t : t;
-      const double mj = entry(j);
+      double mj = 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        double e = m[u];
+        asm volatile("" : "+v"(e));  // a value, not a place to be loaded from
+        mj = j == u ? e : mj;
+      }
 #pragma unroll
       for (int c = 0; c < KT; ++c) {
         const double q = acc[c] / dg.d;
@@ -289,20 +296,16 @@ __device__ __forceinline__ void last_columns(double &t, const double *x, const d
     if (j >= (B & 4) && j < B) t = t + x[j * KT] * m[j];
 }
 
-// A wave's own n <= 64 columns from column c0, in buf; done(lb, B) after each
-// block.
+// A wave's own n <= 64 columns, in buf; done(lb, B) after each block.
 template <int KT, typename Done>
 __device__ __forceinline__ void own_columns(double (&acc)[KT], double (&res)[KT],
                                             const double (&buf)[SN_AHEAD][8], const Diag &dg,
-                                            int c0, int n, const double *M, int row, int nr,
-                                            int lane, Done done) {
+                                            int n, int lane, Done done) {
 #pragma unroll
   for (int b = 0; b < 8; ++b) {
     const int B = min(8, n - 8 * b);
     if (B > 0) {
-      solve_block<KT, false>(acc, res, buf[b], dg, 8 * b, B, lane, [&](int j) {
-        return at(M + (int64_t)(c0 + 8 * b + j) * nr, row);
-      });
+      solve_block<KT, false>(acc, res, buf[b], dg, 8 * b, B, lane);
       done(8 * b, B);
     }
   }
@@ -351,7 +354,7 @@ __device__ __forceinline__ void top_group(const SnArgs &a, const Cols<KT> &col, 
     }
   }
   // the group's own columns
-  own_columns<KT>(acc, res, buf, dg, 64 * g, min(64, w - 64 * g), M, row, nr, lane,
+  own_columns<KT>(acc, res, buf, dg, min(64, w - 64 * g), lane,
                   [&](int lb, int B) {
                     // every lane stores: solved rows their x again, the
                     // others what no wave reads before their own block's count
@@ -403,7 +406,7 @@ __device__ __forceinline__ void narrow_unit(const SnArgs &a, const Cols<KT> &col
   wait_list(a.dlist + n.d0, n.dn, flags, target, a.state, a.timeout);
   gather_list<KT, 8 / KT>(acc, T, a.tcount, list);
   hold<KT>(acc);
-  own_columns<KT>(acc, res, buf, dg, 0, w, M, row, nr, lane, [](int, int) {});
+  own_columns<KT>(acc, res, buf, dg, w, lane, [](int, int) {});
   if (lane < w) {
 #pragma unroll
     for (int c = 0; c < KT; ++c) {
@@ -700,9 +703,9 @@ __device__ __forceinline__ void turn(double (&v)[16], const double (&m)[16], dou
 template <int KT, typename Done>
 __device__ __forceinline__ void own_rows(double (&acc)[KT], double (&res)[KT],
                                          const double (&m)[8], const Diag &dg, int c0, int lb,
-                                         int w, const double *C, int lane, Done done) {
+                                         int w, int lane, Done done) {
   if (c0 < w) {
-    solve_block<KT, true>(acc, res, m, dg, lb, w - c0, lane, [&](int j) { return C[c0 + j]; });
+    solve_block<KT, true>(acc, res, m, dg, lb, w - c0, lane);
     done();
   }
 }
@@ -715,7 +718,6 @@ __device__ __forceinline__ void top_group_t(double (&acc)[KT], double (&res)[KT]
                                             double (&m)[2][16], const Diag &dg, int g, int w,
                                             int nr, const double *M, double *tile, double *xs,
                                             int *prog, int &seen, int lane) {
-  const double *C = M + (int64_t)min(64 * g + lane, w - 1) * nr;
 #pragma unroll
   for (int c = 0; c < KT; ++c) res[c] = 0.0;
   hold<KT>(acc);
@@ -743,7 +745,7 @@ __device__ __forceinline__ void top_group_t(double (&acc)[KT], double (&res)[KT]
       }
     } else {
       const int lb = c0 - 64 * g;
-      own_rows<KT>(acc, res, v8, dg, c0, lb, w, C, lane, [&] {
+      own_rows<KT>(acc, res, v8, dg, c0, lb, w, lane, [&] {
         if (xs) {
 #pragma unroll
           for (int c = 0; c < KT; ++c) xs[(64 * g + lane) * KT + c] = res[c];
