@@ -1009,7 +1009,6 @@ namespace {
 // per unit).
 struct SnSchedule {
   std::vector<SnUnit> unit;           // four slots per ticket
-  std::vector<std::vector<int>> deps; // per slot
   std::vector<int> top;               // per supernode: the slot that solves its top
   std::vector<int> group;             // per supernode: the slot of its first group, or -1
   std::vector<int> first;             // per supernode: the slot of its first chunk, or -1
@@ -1067,19 +1066,6 @@ void sn_schedule(int m, const int *h_sup, const int *h_nrows, const int *h_Lp,
         }
       }
     ++s.widths[(int)((s.unit.size() - before) / 4)];
-  }
-  s.deps.assign(s.unit.size(), {});
-}
-
-void flatten_deps(SnSchedule &s) {
-  for (size_t u = 0; u < s.unit.size(); ++u) {
-    std::vector<int> &d = s.deps[u];
-    if (d.empty()) continue;
-    std::sort(d.begin(), d.end());
-    d.erase(std::unique(d.begin(), d.end()), d.end());
-    s.unit[u].d0 = (int)s.dlist.size();
-    s.unit[u].dn = (int)d.size();
-    s.dlist.insert(s.dlist.end(), d.begin(), d.end());
   }
 }
 
@@ -1145,19 +1131,27 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
   // before any supernode that waits, and every unit waits only for units
   // dealt before it
   std::vector<int> lev(m, 0), tlev(m, 0);
+  std::vector<int> own, optr(m + 1, 0);  // owners of a supernode's rows below, in row order
   int old_tasks = 0;
   for (int i = 0; i < m; ++i) {
     const int w = h_sup[i + 1] - h_sup[i];
+    int last = -1;
     for (int k = 0; k < h_nrows[i] - w; ++k) {
-      const int row = h_Li[h_Lp[i] + w + k];
+      const int row = h_Li[h_Lp[i] + w + k], o = owner[row];
+      int4 &l = list[row];
       rowb[tb[i] + k] = row;
-      tdst[tb[i] + k] = list[row].x + list[row].y++ * list[row].z;
-      lev[owner[row]] = std::max(lev[owner[row]], lev[i] + 1);
+      tdst[tb[i] + k] = l.x + l.y++ * l.z;
+      if (o != last) {
+        own.push_back(o);
+        lev[o] = std::max(lev[o], lev[i] + 1);
+        last = o;
+      }
     }
+    optr[i + 1] = (int)own.size();
     old_tasks += std::max(1, (h_nrows[i] - w + 127) / 128);
   }
   for (int i = m - 1; i >= 0; --i)
-    for (int k = tb[i]; k < tb[i + 1]; ++k) tlev[i] = std::max(tlev[i], tlev[owner[rowb[k]]] + 1);
+    for (int k = optr[i]; k < optr[i + 1]; ++k) tlev[i] = std::max(tlev[i], tlev[own[k]] + 1);
   std::vector<int> longest(m, 0);  // longest list of a supernode's rows
   for (int i = 0; i < m; ++i)
     for (int r = h_sup[i]; r < h_sup[i + 1]; ++r) longest[i] = std::max(longest[i], cnt[r + 1] - cnt[r]);
@@ -1167,34 +1161,51 @@ int sn_analyze(symamd_handle h, int n, int m, const int *h_sup, const int *h_nro
   // forward: a top, or the row groups of one that has them, waits for the
   // units that write its rows' temporaries, a chunk of the rows below for its
   // top.  transposed: the units that read x at the rows below (a narrow
-  // supernode, the column groups of a wide one) wait for the tops of their
-  // owners.  A top with groups waits for those
+  // supernode, the column groups of a wide one, which share a list) wait for the
+  // tops of their owners.  A top with groups waits for those.  A unit's rows
+  // meet another's in ascending order, so a pair met again follows itself.
+  std::vector<std::pair<int, int>> pairs;  // (waiting slot, slot waited for)
+  std::vector<int> last(fwd.unit.size(), -1);
   for (int i = 0; i < m; ++i) {
-    const int w = h_sup[i + 1] - h_sup[i];
-    const int head = w <= SN_NARROW ? SN_NARROW_ROWS : 0;
-    std::vector<int> own;
-    for (int k = 0; k < tb[i + 1] - tb[i]; ++k) {
+    const int w = h_sup[i + 1] - h_sup[i], below = tb[i + 1] - tb[i];
+    const int head = w <= SN_NARROW ? SN_NARROW_ROWS : 0, d0 = (int)bwd.dlist.size();
+    for (int k = 0; k < below; ++k) {
       const int row = rowb[tb[i] + k], o = owner[row];
       const int producer = k < head ? fwd.top[i] : fwd.first[i] + 4 * ((k - head) / 64);
-      std::vector<int> &d = fwd.deps[fwd.group[o] < 0 ? fwd.top[o]
-                                                      : fwd.group[o] + 4 * ((row - h_sup[o]) / 64)];
-      if (d.empty() || d.back() != producer) d.push_back(producer);
-      if (own.empty() || own.back() != bwd.top[o]) own.push_back(bwd.top[o]);
+      const int u = fwd.group[o] < 0 ? fwd.top[o] : fwd.group[o] + 4 * ((row - h_sup[o]) / 64);
+      if (last[u] != producer) pairs.emplace_back(u, producer);
+      last[u] = producer;
     }
-    for (int r = head, u = fwd.first[i]; u >= 0 && r < tb[i + 1] - tb[i]; r += 64, u += 4)
-      fwd.deps[u].push_back(fwd.top[i]);
-    if (bwd.group[i] < 0)
-      bwd.deps[bwd.top[i]] = own;
-    else
-      for (int g = 0; 64 * g < w; ++g) bwd.deps[bwd.group[i] + 4 * g] = own;
-    for (SnSchedule *s : {&fwd, &bwd})
+    for (int r = head, u = fwd.first[i]; u >= 0 && r < below; r += 64, u += 4)
+      pairs.emplace_back(u, fwd.top[i]);
+    for (int k = optr[i]; k < optr[i + 1]; ++k) bwd.dlist.push_back(bwd.top[own[k]]);
+    std::sort(bwd.dlist.begin() + d0, bwd.dlist.end());
+    bwd.dlist.erase(std::unique(bwd.dlist.begin() + d0, bwd.dlist.end()), bwd.dlist.end());
+    const int dn = (int)bwd.dlist.size() - d0;
+    for (int g = 0; dn > 0 && (bwd.group[i] < 0 ? g == 0 : 64 * g < w); ++g) {
+      SnUnit &u = bwd.unit[bwd.group[i] < 0 ? bwd.top[i] : bwd.group[i] + 4 * g];
+      u.d0 = d0;
+      u.dn = dn;
+    }
+  }
+  std::vector<int> dptr(fwd.unit.size() + 1, 0);
+  for (const auto &d : pairs) ++dptr[d.first + 1];
+  for (size_t u = 0; u + 1 < dptr.size(); ++u) dptr[u + 1] += dptr[u];
+  fwd.dlist.resize(pairs.size());
+  std::vector<int> at(dptr.begin(), dptr.end() - 1);
+  for (const auto &d : pairs) fwd.dlist[at[d.first]++] = d.second;
+  for (size_t u = 0; u < fwd.unit.size(); ++u)
+    if (dptr[u + 1] > dptr[u]) {
+      std::sort(fwd.dlist.begin() + dptr[u], fwd.dlist.begin() + dptr[u + 1]);
+      fwd.unit[u].d0 = dptr[u];
+      fwd.unit[u].dn = dptr[u + 1] - dptr[u];
+    }
+  for (SnSchedule *s : {&fwd, &bwd})
+    for (int i = 0; i < m; ++i)
       if (s->group[i] >= 0) {
         s->unit[s->top[i]].d0 = s->group[i];
         s->unit[s->top[i]].dn = -1;
       }
-  }
-  flatten_deps(fwd);
-  flatten_deps(bwd);
   auto *q = new symamd_snplan_s();
   q->n = n;
   q->m = m;
