@@ -91,7 +91,9 @@ int symamd_set_timeout_ms(symamd_handle h, double ms);
  *     integer; 0 disables) and capacity in uint64 entries of a trace
  *     buffer.  Sync-free launches then record, per work unit u, three
  *     100 MHz clock stamps: [3u] unit taken, [3u+1] dependencies ready,
- *     [3u+2] unit published (units beyond the capacity are not traced). */
+ *     [3u+2] unit published (units beyond the capacity are not traced).
+ *     Region launches record the same per task: taken, first halo values
+ *     loaded, rows stored.  A sync-free solve is traced on the units. */
 /*   SYMAMD_OPT_MAX_WAVES: cap on the wavefronts of a persistent launch
  *     (0 = as many as fit the GPU, the default).
  *   SYMAMD_OPT_COLMAJOR_DIRECT: 1 = solve column-major blocks of k > 1
@@ -128,7 +130,9 @@ int symamd_set_timeout_ms(symamd_handle h, double ms);
  *   SYMAMD_OPT_REGION_CAP (read at solve time): region size cap of the
  *     SYMAMD_EXEC_REGIONS schedule (0, the default: the cap symamd_tune
  *     chose for the plan, else 1024 rows for single right-hand sides on the
- *     memory-wavefront kernel, 256 for tasks of eight columns run by one
+ *     memory-wavefront kernel (384 for many planes side by side: more than 16
+ *     tasks of 1024 rows and levels of more than 40 rows per CU, at most 2.5
+ *     entries below the diagonal a row), 256 for tasks of eight columns run by one
  *     wavefront and 512 otherwise; halved -- down to 32 -- until a task's
  *     rows, halo and record fit a workgroup's LDS; a cap set here is used
  *     alone); each cap's schedule is built once per plan.
@@ -309,7 +313,9 @@ int symamd_region_schedule(symamd_handle h, symamd_plan plan, int k, int transpo
  * ran, else SYMAMD_EXEC_REGIONS when the plan has a usable region schedule
  * with at least 60 % of L's off-diagonal entries inside regions (column-major
  * blocks only through the workspace, see SYMAMD_OPT_COLMAJOR_DIRECT), else
- * SYMAMD_EXEC_SYNCFREE.  May build the region schedule. */
+ * SYMAMD_EXEC_SYNCFREE.  May build the region schedule.  At least two lanes
+ * are reported for a tuned choice of the row executor, which shares rows
+ * between lanes as it finds them. */
 int symamd_choice(symamd_handle h, symamd_plan plan, int k, symamd_layout layout,
                   int *exec, int *lanes);
 int symamd_plan_destroy(symamd_plan plan);

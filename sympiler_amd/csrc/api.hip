@@ -77,9 +77,10 @@ void free_plan_arrays(symamd_plan p) {
 // the Zipf(1.8) n = 1e6 matrix (average 8.7 entries, longest 257) with the
 // units of the sync-free executor: lanes 4 / 32 at k = 1: 11.5 / 4.3 ms; lanes
 // 1 / 8 at k = 8: 30.8 / 5.7 ms; lanes 1 / 2 at k = 32: 33.2 / 16.6 ms.  Where
-// the choice is more than one lane, sync-free solves run on the row executor
-// (rows_exec.hip), which takes 0.64 / 0.8 / 1.4 ms at k = 1 / 8 / 32 there and
-// picks the lanes row by row.
+// the choice is more than one lane, forward solves of up to 32 columns over
+// narrow levels run on the row executor (rows_path in rows_exec.hip), which
+// takes 0.64 / 0.8 / 1.4 ms at k = 1 / 8 / 32 there and picks the lanes row by
+// row; untuned blocks of more columns run on the units.
 Choice heuristic(symamd_plan p, int k) {
   (void)k;
   Choice c;

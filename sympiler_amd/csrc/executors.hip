@@ -33,8 +33,9 @@
 // Executors
 //   LEVELSET  one launch per level, one wave per unit; plain loads and
 //             stores (kernel boundaries order the levels).
-//   SYNCFREE  one persistent launch (with one lane per row, or without the
-//             marked protocol; several lanes per row run in
+//   SYNCFREE  one persistent launch (with one lane per row, more than 32
+//             columns untuned, few wide levels, or without the marked
+//             protocol; other solves with several lanes per row run in
 //             rows_exec.hip).  Units are dealt to waves round-robin from a
 //             cooperative launch (all waves co-resident), or taken from a
 //             ticket counter when the launch is captured in a graph; either

@@ -18,11 +18,12 @@
 //     workgroup's (its waves' sums meet in LDS).
 // What bounds it is the chain of levels for one right-hand side (a store on
 // one XCD reaching a poll on another, the lanes' reduction, the division:
-// 1.4 us per level) and, for several, the tickets a workgroup can take.
-// Zipf(1.8) matrix, n = 1e6, 449 levels, in ms with the unit executor and
-// here: one right-hand side 3.38 / 0.65, 4 columns 5.1 / 0.79, 13 columns
-// 10 / 1.06, 32 columns 18.0 / 1.35 (0.35 of it the turns of a column-major
-// block).
+// 1.4 us per level) and, for several and where levels are wide, the tickets
+// (one counter, 13 ns each; few wide levels stay on the units, see
+// tickets_win).  Zipf(1.8) matrix, n = 1e6, 459 levels, in ms with the unit
+// executor and here: one right-hand side 3.38 / 0.65, 4 columns 5.1 / 0.79, 13
+// columns 10 / 1.06, 32 columns 18.0 / 1.38 (0.22 of it the turns of a
+// column-major block).
 // Workgroups take tickets in schedule order, so every value waited for is
 // held by a running workgroup; waits are bounded by the watchdog.
 //
@@ -272,7 +273,10 @@ __global__ __launch_bounds__(256) void k_rows_turn(int n, int k, int64_t ld, T *
 // Workgroups per CU: enough to have the rows of the next levels loaded ahead;
 // more only poll and slow the chain (n = 1e6, in ms: one right-hand side with
 // 512 / 1024 / 2048 waves 0.65 / 0.72 / 0.98; 4 columns with 1024 / 2048 /
-// 4096 1.11 / 0.79 / 0.91; 32 columns 2.69 / 1.55 / 1.35).
+// 4096 1.11 / 0.79 / 0.91; 32 columns 2.69 / 1.55 / 1.35).  Where levels are
+// wide more do not help either, as the ticket counter is the limit: 27-point
+// grid of 96^3 in eight colours, one right-hand side, 512 / 1024 / 2048 / 4096
+// waves 0.40 / 0.42 / 0.43 / 0.47.
 constexpr int ROWS_PER_CU(int c) { return c == 1 ? 1 : c == 8 ? 1 : 2; }
 
 int rows_cols(int k) { return k == 1 ? 1 : k <= 8 ? 8 : k <= 16 ? 16 : 32; }

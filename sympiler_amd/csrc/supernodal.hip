@@ -29,10 +29,12 @@
 // loop): entry j of the 64 rows of a wave lies side by side, so a load of T
 // is one contiguous run.
 //
-// What bounds it: the chain of tree levels -- for each, the widest top's
-// columns (about 70 clocks each: two Newton steps for the quotient, a
-// broadcast, a multiply and a subtract) and the hand-offs -- for one
-// right-hand side and the last levels of a block.  A top's rows lie one per
+// What bounds it: the chain of tree levels, for one right-hand side and the
+// last levels of a block: for each, the hand-offs between its units (gather,
+// top, rows below) and the widest top's columns (about 70 clocks, 29 ns, each:
+// two Newton steps for the quotient, a broadcast, a multiply and a subtract;
+// the 2,734 columns on the 13-level factor's longest path are a quarter of its
+// forward solve).  A top's rows lie one per
 // lane, 64 to a wave, and each wave streams its rows' entries with SN_AHEAD
 // column blocks in flight; the wave whose rows are next solves its 64 columns
 // with lane broadcasts and hands x on through LDS, block of 8 by block of 8,
@@ -55,7 +57,7 @@ namespace symamd {
 namespace {
 
 // Column blocks of 8 whose entries are in flight: a wave's own 64 columns,
-// whose chain (about 20 ns a column) runs ahead of any load issued during it.
+// whose chain (about 29 ns a column) runs ahead of any load issued during it.
 constexpr int SN_AHEAD = 8;
 
 // One unit, read in one scalar load: the supernode's first column, width and

@@ -114,3 +114,21 @@ def test_few_boxes_against_the_matching(grid, regions):
     if regions == 2:
         levels = sum(len(r["slices"]) - 1 for r in _records(sch))
         assert rows[0] < rows[1] or levels < 2 * 22, (rows, levels)  # boxes: 22 each
+
+
+@pytest.mark.parametrize("grid,cap", [((13, 11, 17), 512), ((19, 9, 7), 64), ((3, 29, 5), 128),
+                                      ((2, 2, 41), 32), ((37, 23, 1), 128), ((101, 7, 1), 512),
+                                      ((2, 90, 1), 64)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_every_region_is_a_box(grid, cap, transposed):
+    nx, ny, nz = grid
+    M = W.lap3d_tril(*grid, 6.01, -1.0) if nz > 1 else W.lap2d_tril(nx, ny)
+    sch = schedule_host(*M, cap, 4, transposed=transposed)
+    seen = 0
+    for r in _records(sch):
+        i = np.asarray(r["rows"], np.int64)
+        sides = [len(np.unique(c)) for c in (i % nx, i // nx % ny, i // (nx * ny))]
+        spans = [np.ptp(c) + 1 for c in (i % nx, i // nx % ny, i // (nx * ny))]
+        assert sides == spans and np.prod(sides) == len(i) <= cap
+        seen += len(i)
+    assert seen == nx * ny * nz
