@@ -498,24 +498,29 @@ int rows_schedule(symamd_handle h, symamd_plan p, int C, bool build, RowSchedule
 }
 
 // Whether the tickets take no longer than the units would.  The unit executor
-// spends its time on levels (about 9 us each, and 0.25 us for every entry that
-// a lane of the longest row adds) and, where those are wide, on entries (18 ps
-// each) and right-hand sides (17 ps a value, 10 up to eight columns); this one
-// on tickets, which workgroups take from one counter (13 ns each; 14 with 8 or
-// 16 column lanes).  So long chains of narrow levels run here and few wide
-// levels on the units.  In ms, units / here, the side taken first: 27-point grid
-// of 96^3 in natural order (666 levels) k = 1 2.90 / 1.03, k = 32 4.40 / 1.78
-// (here); in eight colours 0.16 / 0.40, 0.82 / 1.15 (units); 20 levels of
-// 20,000 rows of 12 entries k = 1 0.22 / 0.17 (here), k = 32 0.54 / 0.71
-// (units); 100 levels of 4,000 k = 32 1.14 / 0.76 (here); 40 of 8,000 rows of 40
-// entries k = 1 0.49 / 0.49, k = 32 0.91 / 3.78 (units); two levels, 300,000 rows
-// of 64 entries, 0.36 / 0.42, 0.62 / 3.29 (units); 64 levels of 1,500 rows of up
-// to 63 entries k = 32 0.64 / 0.70 (here, the largest miss).
+// spends its time on levels (6.6 us each, and 0.25 us for every entry that a
+// lane of the longest row adds) and, where those are wide, on entries (15.5 ps
+// each) and on the values of wide blocks (2.2 ps each); this one on tickets,
+// which workgroups take from one counter (13 ns each for one right-hand side,
+// 12.2 with 8 column lanes, or 24 ps an entry where rows take several rounds;
+// 9.6 and 10 with 16 and 32, against which the units start 15 and 20 us ahead).  So long chains of narrow levels run here and
+// few wide levels on the units.  The constants are fitted to which of the two
+// was faster on 46 patterns in FP64 and FP32; near the line the side taken is up
+// to a fifth slower than the other.  In ms, units / here, the side taken after it: 27-point
+// grid of 96^3 in natural order (666 levels) k = 1 2.90 / 1.03, k = 32 4.40 /
+// 1.78, here; in eight colours 0.16 / 0.40, 0.82 / 1.15, units, of 64^3 0.11 /
+// 0.14, 0.26 / 0.38, units; 20 levels of 20,000 rows of 12 entries k = 1 0.22 /
+// 0.17, here, k = 32 0.54 / 0.71, units; 100 levels of 4,000 k = 32 1.14 / 0.76,
+// here; 40 of 8,000 rows of 40 entries k = 1 0.49 / 0.49, k = 32 0.91 / 3.78,
+// units; two levels, 300,000 rows of 64 entries, 0.36 / 0.42, 0.62 / 3.29, units;
+// 64 levels of 1,500 rows of up to 63 entries k = 32 0.64 / 0.70, here.
 bool tickets_win(symamd_plan p, int k, int lanes, int tile, int tickets) {
   const int C = rows_cols(k), eff = std::max(1, std::min(lanes, 64 / tile_cols(k, tile)));
-  const double units = p->levels * (9000.0 + 250.0 * p->max_row_nnz / eff) + 0.018 * p->nnz +
-                       (k <= 8 ? 0.010 : 0.017) * p->n * k;
-  return tickets * (C == 8 || C == 16 ? 14.0 : 13.0) <= units;
+  const double units = p->levels * (6600.0 + 250.0 * p->max_row_nnz / eff) + 0.0155 * p->nnz +
+                       (k <= 8 ? 0.0 : 0.0022) * p->n * k;
+  const double rows = C == 1 ? 13.0 * tickets : C == 8 ? std::max(12.2 * tickets, 0.024 * p->nnz)
+                      : C == 16 ? 15000.0 + 9.6 * tickets : 20000.0 + 10.0 * tickets;
+  return rows <= units;
 }
 
 template <typename T, int C>
