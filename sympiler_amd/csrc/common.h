@@ -130,8 +130,10 @@ struct UnitSet {
   int64_t xdeps = 0;
 };
 
-// Packed structure of a factorization's units (factor0.hip).
+// Packed structure of a factorization's units (factor0.hip), built for the
+// second factorization of a plan.
 struct FactorPack {
+  bool wanted = false;
   int64_t *d_off = nullptr;
   int *d_wide = nullptr, *d_data = nullptr;
 };

@@ -583,11 +583,18 @@ int64_t factor_waves(symamd_handle h, symamd_plan p, int units, int per_cu) {
 
 int scan64(symamd_handle h, const int64_t *in, int64_t *out, int64_t count, Scratch &sc);
 
-// The packed units of a factorization, built on first use.  Without the memory
+// The packed units of a factorization, built for the second one of a plan:
+// allocating them takes longer (0.6 ms for the 64^3 Laplacian) than one
+// factorization gains, and many plans factor once (first call there 3.1 ms with
+// tagged units, 4.0 with the packing in it, 3.0 without).  Without the memory
 // every unit is read from the caller's arrays.
 template <int MODE>
 int factor_pack(symamd_handle h, FactorArgs a, FactorPack &f) {
   if (f.d_off) return SYMAMD_OK;
+  if (!f.wanted) {
+    f.wanted = true;
+    return SYMAMD_OK;
+  }
   Scratch sc, keep;
   int64_t *size = nullptr, *off = nullptr;
   int *wide = nullptr, *data = nullptr;

@@ -22,7 +22,6 @@
 #include <climits>
 #include <cstdint>
 #include <cstring>
-#include <map>
 #include <numeric>
 #include <thread>
 #include <vector>
@@ -612,32 +611,45 @@ int make_acyclic(int n, const int *Lp, const int *Li, const std::vector<int> &le
 
 // The longest chain of regions for a block of right-hand sides, at lattice_cut's
 // costs; the region graph has no cycle.
-double chain_cost(int n, const int *Lp, const int *Li, const std::vector<int> &lev,
-                  const std::vector<int> &reg, int R) {
-  std::vector<std::map<int, int>> rows(R);  // per region: rows of each level
-  std::vector<std::vector<int>> succ(R);
-  std::vector<int> indeg(R, 0), ready;
-  for (int i = 0; i < n; ++i) {
-    ++rows[reg[i]][lev[i]];
-    for (int j = Lp[i]; j < Lp[i + 1] - 1; ++j)
-      if (reg[Li[j]] != reg[i]) {
-        succ[reg[Li[j]]].push_back(reg[i]);
-        ++indeg[reg[i]];
+double chain_cost(int n, const int *Lp, const int *Li, const std::vector<int> &by_lev,
+                  const std::vector<int> &lev, const std::vector<int> &reg, int R) {
+  // rounds of 64 rows, level by level (by_lev: the rows in level order)
+  std::vector<int> rounds(R, 0), rows(R, 0), touched;
+  for (int t = 0; t < n; ++t) {
+    const int r = reg[by_lev[t]];
+    if (rows[r]++ == 0) touched.push_back(r);
+    if (t + 1 == n || lev[by_lev[t + 1]] != lev[by_lev[t]]) {
+      for (int q : touched) {
+        rounds[q] += (rows[q] + 63) / 64;
+        rows[q] = 0;
       }
+      touched.clear();
+    }
   }
+  std::vector<int> ptr(R + 1, 0), indeg(R, 0), ready;
+  auto each_edge = [&](auto f) {
+    for (int i = 0; i < n; ++i)
+      for (int j = Lp[i]; j < Lp[i + 1] - 1; ++j)
+        if (reg[Li[j]] != reg[i]) f(reg[Li[j]], reg[i]);
+  };
+  each_edge([&](int from, int to) {
+    ++ptr[from + 1];
+    ++indeg[to];
+  });
+  for (int r = 0; r < R; ++r) ptr[r + 1] += ptr[r];
+  std::vector<int> succ(ptr[R]), at(ptr.begin(), ptr.end() - 1);
+  each_edge([&](int from, int to) { succ[at[from]++] = to; });
   for (int r = 0; r < R; ++r)
     if (indeg[r] == 0) ready.push_back(r);
   std::vector<double> before(R, 0.0);
   double longest = 0.0;
   for (size_t q = 0; q < ready.size(); ++q) {
     const int r = ready[q];
-    int rounds = 0;
-    for (const auto &l : rows[r]) rounds += (l.second + 63) / 64;
-    const double end = before[r] + BLOCK_HOP + BLOCK_ROUND * rounds;
+    const double end = before[r] + BLOCK_HOP + BLOCK_ROUND * rounds[r];
     longest = std::max(longest, end);
-    for (int s : succ[r]) {
-      before[s] = std::max(before[s], end);
-      if (--indeg[s] == 0) ready.push_back(s);
+    for (int e = ptr[r]; e < ptr[r + 1]; ++e) {
+      before[succ[e]] = std::max(before[succ[e]], end);
+      if (--indeg[succ[e]] == 0) ready.push_back(succ[e]);
     }
   }
   return longest;
@@ -680,8 +692,9 @@ bool build_region_schedule(int n, int64_t nnz, int levels, const int *lvl_ptr,
     std::vector<int> other;
     int S = cluster_regions(n, Lp.data(), Li.data(), cap, false, other, nullptr);
     S = make_acyclic(n, Lp.data(), Li.data(), lev, cap, other, S);
-    if (chain_cost(n, Lp.data(), Li.data(), lev, other, S) <
-        BOXES_LEAD * chain_cost(n, Lp.data(), Li.data(), lev, reg, R)) {
+    const std::vector<int> by_lev(perm, perm + n);
+    if (chain_cost(n, Lp.data(), Li.data(), by_lev, lev, other, S) <
+        BOXES_LEAD * chain_cost(n, Lp.data(), Li.data(), by_lev, lev, reg, R)) {
       reg.swap(other);
       R = S;
     }
